@@ -409,10 +409,10 @@ def bench_config5(args, dev, quick=False):
         "ms_per_step": wall * 1e3 / steps, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "bf16", "data": "synthetic",
         "config": {"workload": f"config5: fused lm_head + logprob/entropy, hidden [{T}, {H}], W [{V}, {H}], fwd + bwd to "
-                               "hidden and W, no [T, V] tensor kept (logits recomputed per 8192-column slab in the "
+                               "hidden and W, no [T, V] tensor kept (logits recomputed per group of columns in the "
                                "backward)", "tokens": T, "hidden": H, "vocab": V, "seed": SEED},
         "kernels": {"forward (gemm_nt_kernel<SoftmaxPartialsEpi> + merge)": {"ms": fwd_ms, "TFLOP/s": gemm / fwd_ms / 1e9},
-                    "backward (recompute + dlogits per slab, d hidden and d weight per 65536 columns)":
+                    "backward (recompute + dlogits, d hidden and d weight per 65536 columns)":
                         {"ms": bwd_ms, "TFLOP/s executed": 3 * gemm / bwd_ms / 1e9}},
         "library_gemm_yardstick": {"what": f"torch.mm in bf16 through the vendor library, no epilogue: W [{V}, {H}] . "
                                            f"hidden^T (the forward's and the recompute's GEMM), dlogits [{T}, {Vg}] . "

@@ -670,10 +670,10 @@ int siirl_fused_linear_logprob_entropy_fwd(const void* hidden, const void* weigh
 /*
  * Backward: for upstream gradients g_logprob[T] / g_entropy[T] (either may be NULL) writes
  * d_hidden[T, H] and / or d_weight[V, H] in the operands' dtype (either may be NULL).  The vocabulary is walked in
- * slabs of 8192 columns: the slab's logits are recomputed -- or, when saved_logits holds what the forward call with
+ * groups of columns: the group's logits are recomputed -- or, when saved_logits holds what the forward call with
  * the same hidden, weight and inv_temperature parked there, read back --, dlogits = inv_T * (g_lp (onehot - p)
  * - g_H p (z - ex)) is written to scratch as bf16 (token-major, one layout for both consumers), then
- * d_hidden += dlogits . W_slab (fp32 accumulation across slabs, rounded once) and d_weight_slab = dlogits^T . hidden.
+ * d_hidden += dlogits . W_group (fp32 accumulation across groups, rounded once) and d_weight_group = dlogits^T . hidden.
  * Both routes give the same bits.  For SIIRL_F16 and SIIRL_F32 operands the logits are recomputed as in the forward;
  * the two gradient GEMMs multiply the bf16 dlogits (bf16 for its range: a softmax gradient underflows fp16) with
  * hidden and W rounded to bf16, so the gradients carry one more 2^-9 rounding than with bf16 operands; the reference
@@ -695,7 +695,8 @@ int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const void* weigh
  * contribute nothing to either result and are left out of all three GEMMs here.  Rows not listed get zeros in
  * d_hidden; d_weight sums over the listed rows only.  The results are those of
  * siirl_fused_linear_logprob_entropy_bwd on the gathered operands, bit for bit (against the full call d_weight
- * differs by the rounding order of its sum over tokens).  n_rows == 0 writes zeros.  The logits are always
+ * differs by the rounding order of its sum over tokens, and d_hidden by that of its sum over the vocabulary where the
+ * two token counts, above 1024, have it cut into different runs).  n_rows == 0 writes zeros.  The logits are always
  * recomputed on this route.  workspace: siirl_fused_linear_bwd_rows_workspace_bytes(n_rows, ...) bytes, 256-byte
  * aligned.
  * Replaces: FusedLinearForPPO.backward siirl/utils/experimental/torch_functional.py:35-67,135-188 as reached from

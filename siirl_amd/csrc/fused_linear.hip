@@ -20,9 +20,9 @@
 //   * all loads of the main loop are inline asm with hand-placed s_waitcnt vmcnt: the compiler's own tracking
 //     would wait for every outstanding DMA before each LDS read.
 // Four epilogues: softmax partials (forward), dlogits in both layouts (backward), fp32 accumulate (d hidden),
-// bf16 store (d weight).  The backward walks the vocabulary in slabs: recompute the slab's logits, write
-// dlogits[T, slab] and its transpose, then dH += dlogits . W_slab and dW_slab = dlogits^T . hidden as two more
-// runs of the same core against packed transposed copies of W and hidden.
+// bf16 store (d weight).  The backward walks the vocabulary in groups of columns: recompute the group's logits into
+// dlogits[T, group], then dH += dlogits . W_group and dW_group = dlogits^T . hidden as two more runs of the same core
+// against packed transposed copies of W and hidden.
 // Optionally the forward also parks the fp32 accumulator tiles in memory (4 bytes per logit, in the accumulator's
 // own lane order, so stores and loads are whole 1 KB wave accesses); the backward then replays the tiles through
 // the same dlogits epilogue instead of recomputing the GEMM: a third of the backward's matrix work is traded for
@@ -52,19 +52,12 @@ constexpr int kStageBytes = kTileBytes;       // A tile only: B goes global -> r
 constexpr int kStages = 4;
 constexpr int kSmemBytes = kStages * kStageBytes;  // 131072
 constexpr int kDmaPerWave = kTileBytes / 1024 / (kThreads / 64);  // 1 KB per wave instruction
-#ifndef SIIRL_SLAB
-#define SIIRL_SLAB 8192
-#endif
-constexpr int kSlab = SIIRL_SLAB;                   // vocabulary columns per backward slab
-static_assert(kSlab % 256 == 0, "a slab is a whole number of workgroup tiles");
-#ifndef SIIRL_DH_GROUP
-#define SIIRL_DH_GROUP 8
-#endif
-constexpr int kDhGroup = SIIRL_DH_GROUP;      // slabs of dlogits kept before d hidden and d weight are updated: fewer
-                                              // fp32 read-modify-write passes over [T, H] (about 6 % of a d-hidden
-                                              // launch at 4 slabs), and 8 x 448 d-weight tiles fill 14 rounds of
-                                              // the 256 CUs exactly; measured 4 / 8 / all 19 slabs of V = 152064:
-                                              // 34.4 / 33.7 / 33.2 ms per backward
+// The backward walks the vocabulary in groups: the group's logits are recomputed into dlogits, then d hidden and
+// d weight are updated from them.  A group is 65536 columns at 16384 tokens and above (256 x 64 tiles of dlogits and
+// 256 x 14 of d weight at H = 3584 fill whole rounds of the 256 CUs; 4 / 8 / 19 times 8192 columns measured 34.4 / 33.7
+// / 33.2 ms per backward at T=16384, V=152064), and as many times more with fewer tokens as keep the same bytes of
+// dlogits: at T=200, V=152064 one group instead of three.
+constexpr int64_t kGroupCols = 65536, kGroupTokens = 16384;
 constexpr int kLdPad = 64;                    // extra elements per row of D: keeps a tile's rows off a
                                               // power-of-two stride, which would put them all in one memory channel
 
@@ -85,7 +78,7 @@ struct TileCoord {
 };
 // XCD-aware rasterisation.  Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2, so
 // workgroup id runs on XCD id % 8 as that XCD's (id / 8)-th workgroup.  The tile grid is cut into blocks of
-// blk_m x blk_n tiles (32 tiles: one XCD's resident set; blk_m is the launch's choice among 2, 4, 8, 16); block b
+// blk_m x blk_n tiles (32 tiles: one XCD's resident set; blk_m is the launch's choice among the powers of two); block b
 // goes to XCD b % 8 and its tiles to 32 consecutive workgroups of that XCD, so the workgroups sharing an L2 at any
 // time share blk_m A-tiles and blk_n B-tiles instead of streaming 32 different A-tiles.  Blocks sweep M fastest
 // inside a strip of blk_n N-tiles, which keeps a strip's B-tiles hot across the 8 XCDs.  (Sweeping N fastest instead, which would stream the big
@@ -428,14 +421,14 @@ struct SoftmaxPartialsEpi {
 // ------------------------------------------------------------------------------ epilogue: dlogits
 
 // d raw_logit = inv_T * ( g_lp * (1[v == y] - p) - g_h * p * (z - ex) ),  p = exp(z - lse), z = acc * inv_T,
-// written as bf16 to D[token][v] (ld = ldd); v is slab-relative and is the M dimension of this GEMM.  Rows v in
+// written as bf16 to D[token][v] (ld = ldd); v is group-relative and is the M dimension of this GEMM.  Rows v in
 // [Vs, Vpad) are written as zeros: they are K-padding of the d-hidden GEMM that consumes D.  A lane owns one token,
 // so the per-token coefficients are loaded once per lane and D gets 8-byte stores.  This one token-major layout
 // serves both consumers: d hidden reads it as its A[M = token][K = vocabulary], d weight as A given by K-rows.
 struct DlogitsEpi {
   float inv_T;
   int T, Vs, Vpad;
-  int64_t v0;  // first vocabulary column of the slab
+  int64_t v0;  // first vocabulary column of the group
   const float* lse;
   const float* ex;
   const float* g_lp;  // may be null
@@ -447,7 +440,7 @@ struct DlogitsEpi {
   //   d = p * (c0 + c1 * a) + [v == y] * cy,   p = exp2(a * ek + nl),
   // ek = inv_T * log2(e), nl = -lse * log2(e), c1 = -g_h * inv_T^2, c0 = inv_T * (g_h * ex - g_lp), cy = g_lp * inv_T:
   // two fused multiply-adds, one exp2 and one multiply per logit.  FULL: every vocabulary row of the tile is inside
-  // the slab.
+  // the group.
   template <bool FULL>
   __device__ __forceinline__ void tile(floatx4 (&acc)[MI][NJ], int m0, int n0, int wm, int wn, int lane) const {
     const float ek = inv_T * kLog2e;
@@ -468,7 +461,7 @@ struct DlogitsEpi {
       uint16_t* drow = D + (int64_t)tok * ldd;
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        const int v = m0 + acc_row(wm, i, 0, lane);  // 4 consecutive vocabulary rows of the slab
+        const int v = m0 + acc_row(wm, i, 0, lane);  // 4 consecutive vocabulary rows of the group
         float d[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -683,17 +676,19 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(const float* __rest
   if (logprob) logprob[row] = label_logit[row] - lse;
 }
 
-// out = in (+ in2), rounded to out_dtype (SIIRL_BF16, SIIRL_F16 or SIIRL_F32)
-__global__ __launch_bounds__(256) void sum_convert_kernel(const float* __restrict__ in, const float* __restrict__ in2,
-                                                          void* __restrict__ out, int64_t n, int out_dtype) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const float v = in2 ? in[i] + in2[i] : in[i];
+// out = the sum of `splits` buffers, `stride` four-element vectors apart, rounded to out_dtype (SIIRL_BF16, SIIRL_F16 or
+// SIIRL_F32).  A pure stream: 16-byte loads, the buffers added in their order.
+__global__ __launch_bounds__(256) void sum_convert_kernel(const f32x4* __restrict__ in, int64_t stride, int splits,
+                                                          void* __restrict__ out, int64_t n4, int out_dtype) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
+    f32x4 v = in[i];
+    for (int s = 1; s < splits; ++s) v += in[s * stride + i];
     if (out_dtype == SIIRL_BF16)
-      reinterpret_cast<uint16_t*>(out)[i] = (uint16_t)(pack_bf16(v, 0.f) & 0xffffu);
+      reinterpret_cast<uint2*>(out)[i] = make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
     else if (out_dtype == SIIRL_F16)
-      reinterpret_cast<uint16_t*>(out)[i] = (uint16_t)(pack_f16(v, 0.f) & 0xffffu);
+      reinterpret_cast<uint2*>(out)[i] = make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
     else
-      reinterpret_cast<float*>(out)[i] = v;
+      reinterpret_cast<f32x4*>(out)[i] = v;
   }
 }
 
@@ -724,11 +719,21 @@ __global__ __launch_bounds__(256) void split3_kernel(const float* __restrict__ i
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // AT: A is given by its K-rows (A[K][M], M contiguous, row pitch lda >= tiles_m * BM, K readable rows)
+// Shape of an XCD's block: `blk_m` tiles along M where the grid has room for it.  A grid narrower than the block in one
+// direction would leave most of the block's workgroup ids without a tile (a token count of one tile in blocks of 4 x 8:
+// 7 of 8 ids start and leave, each holding the CU's LDS meanwhile), so the block is made longer in the other one.
+inline int fit_blk_m(int blk_m, int64_t tiles_m, int64_t tiles_n) {
+  while (blk_m > 1 && blk_m / 2 >= tiles_m) blk_m /= 2;
+  while (blk_m < kBlkTiles && kBlkTiles / blk_m / 2 >= tiles_n) blk_m *= 2;
+  return blk_m;
+}
+
 template <class Epi, bool AT = false, bool F16 = false>
 int launch_gemm(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_total, int M, int N, int K, const Epi& epi,
                 hipStream_t st, const char* what, int splits = 1, int blk_m = 8) {
   if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<Epi, AT, F16>), kSmemBytes)) return rc;
   GemmArgs g{A, lda, Bp, kb_total, M, N, K, (M + BM - 1) / BM, (N + BN - 1) / BN, splits, blk_m};
+  g.blk_m = blk_m = fit_blk_m(blk_m, g.tiles_m, (int64_t)g.tiles_n * splits);
   if (AT && lda < (int64_t)g.tiles_m * BM) return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: row pitch %lld is shorter than %d tiles", what, (long long)lda, g.tiles_m);
   const int64_t tiles = raster_grid(g.tiles_m, g.tiles_n * splits, blk_m);
   gemm_nt_kernel<Epi, AT, F16><<<dim3((unsigned)tiles), dim3(kThreads), kSmemBytes, st>>>(g, epi);
@@ -743,13 +748,29 @@ int launch_gemm(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_tota
 // tiles: wider strips read it less often.
 constexpr int kBlkFwd = 4, kBlkRecompute = 2, kBlkDHidden = 4, kBlkDWeight = 8;
 
-// Two K runs when that fills the 256 compute units' last round noticeably better (896 tiles = 3.5 rounds become
-// 1792 = 7) and the GEMM is deep enough for the second fp32 buffer's extra pass not to matter.
-inline int pick_splits(int M, int N, int K) {
-  const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  auto eff = [](int64_t t) { return (double)t / (double)((t + 255) / 256 * 256); };
-  if (K / BK < 128) return 1;
-  return eff(2 * tiles) > eff(tiles) * 1.05 ? 2 : 1;
+// Number of K runs of the d-hidden GEMM, each with an fp32 buffer of its own that sum_convert_kernel adds up.  The
+// tiles of [T, H] alone rarely fill the 256 CUs: 896 tiles at T=16384, H=3584 are 3.5 rounds (two runs: 7), 14 tiles at
+// T=200 a fraction of one (18 runs: 252 workgroups, 1743 -> 190 us).  The run count is the one with the least time by
+// the kernel's measured 1.2 us per K-step and about 12 us per tile besides, plus the buffers' write and read at 5 TB/s.
+constexpr int kMaxSplits = 64;
+constexpr double kSplitBytes = 512.0 * 1048576.0;  // bound on the buffers beyond two
+// Up to 1024 tokens the choice does not look at T (it is the one for a single token tile; at T=1024, H=3584, K=152064
+// 18 runs model as 786 us against 710 us for the best 9), so that a row of d hidden keeps its bits whatever other rows
+// a small batch holds.
+inline int pick_splits(int64_t T, int64_t H, int64_t K) {
+  if (T <= 1024) T = BM;
+  const int64_t tiles = ((T + BM - 1) / BM) * ((H + BN - 1) / BN), KT = K / BK;
+  int best = 1;
+  double best_us = 0.;
+  for (int s = 1; s <= kMaxSplits && s <= KT; ++s) {
+    const double bytes = 4.0 * (double)T * (double)H * s;
+    if (s > 2 && bytes > kSplitBytes) break;
+    const int64_t per = (KT + s - 1) / s;
+    if ((s - 1) * per >= KT) continue;  // the last run would be empty
+    const double us = (double)((tiles * s + 255) / 256) * (1.2 * (double)per + 12.0) + 2.0 * bytes / 5e6;
+    if (s == 1 || us < best_us) best_us = us, best = s;
+  }
+  return best;
 }
 
 // K of the logits GEMM for operands of `dtype`: the hidden size, or three bf16 terms per fp32 element (split3_kernel)
@@ -758,7 +779,7 @@ inline int64_t logits_k(int dtype, int64_t H) { return dtype == SIIRL_F32 ? 3 * 
 int check_fused(const void* hidden, const void* weight, int64_t T, int64_t H, int64_t V, float inv_T, int dtype) {
   SIIRL_REQUIRE(dtype == SIIRL_BF16 || dtype == SIIRL_F16 || dtype == SIIRL_F32,
                 "fused lm_head path takes bf16, fp16 or fp32 operands (dtype %d given)", dtype);
-  // 32-bit byte offsets inside a 256-row tile bound the row pitch of every A operand (W: K, D: group of slabs + pad)
+  // 32-bit byte offsets inside a 256-row tile bound the row pitch of every A operand (W: K, D: group + pad)
   SIIRL_REQUIRE(T >= 1 && T < (1LL << 22) && V >= 1 && V < (1LL << 30), "T=%lld (< 4194304) V=%lld out of range",
                 (long long)T, (long long)V);
   SIIRL_REQUIRE(H >= BK && H % BK == 0 && logits_k(dtype, H) < (1 << 22),
@@ -793,21 +814,27 @@ FwdWs fwd_ws(int64_t T, int64_t H, int64_t V, int dtype) {
 
 struct BwdWs {
   size_t hp, wtp, htp, d, dh32, hs, wsp, total;
-  int64_t ldwt, ldt, hpad, ldd_row;  // ldt: token count padded to BK (the K of the d-weight GEMM); ldd_row: pitch of D
+  int64_t ldwt, ldt, hpad, group, ldd_row;  // ldt: token count padded to BK (the K of the d-weight GEMM); group: columns
+                                            // of a vocabulary group; ldd_row: pitch of D
+  int dh_splits;                            // K runs of the first (largest) group's d-hidden GEMM
 };
 BwdWs bwd_ws(int64_t T, int64_t H, int64_t V, bool want_dh, bool want_dw, int dtype) {
   BwdWs w;
   const int64_t Kc = logits_k(dtype, H);
   w.ldwt = round_up(V, BK);
   w.ldt = round_up(T, BK);
-  w.ldd_row = (int64_t)kDhGroup * kSlab + kLdPad;
+  int64_t n = kGroupTokens / w.ldt;  // at most 64: a tile's byte offsets into D have 32 bits
+  n = n < 1 ? 1 : (n > 64 ? 64 : n);
+  w.group = n * kGroupCols < V ? n * kGroupCols : round_up(V, BM);
+  w.ldd_row = w.group + kLdPad;
+  w.dh_splits = pick_splits(T, H, w.group < V ? w.group : w.ldwt);
   w.hpad = round_up(H, BN);
   size_t off = 0;
   w.hp = off; off += (size_t)round_up(T, BN) * Kc * 2;
   w.wtp = off; off += want_dh ? (size_t)w.hpad * w.ldwt * 2 : 0;
   w.htp = off; off += want_dw ? (size_t)w.hpad * w.ldt * 2 : 0;
   w.d = off; off += round_up((size_t)w.ldt * w.ldd_row * 2, 256);  // rows [T, ldt) are K-padding of d weight: zeros
-  w.dh32 = off; off += want_dh ? 2 * round_up((size_t)T * H * 4, 256) : 0;  // one buffer per K run
+  w.dh32 = off; off += want_dh ? w.dh_splits * round_up((size_t)T * H * 4, 256) : 0;  // one buffer per K run
   w.hs = off; off += dtype == SIIRL_F32 ? round_up((size_t)T * Kc * 2, 256) : 0;
   w.wsp = off; off += dtype == SIIRL_F32 ? round_up((size_t)V * Kc * 2, 256) : 0;
   w.total = off;
@@ -982,7 +1009,7 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
   u32x4* hp = (u32x4*)(base + ws.hp);          // packed hidden: B[n = token][k = K of the logits GEMM]
   u32x4* Wtp = (u32x4*)(base + ws.wtp);        // packed W^T:    B[n = H][k = vocabulary]
   u32x4* Htp = (u32x4*)(base + ws.htp);        // packed hidden^T: B[n = H][k = token]
-  uint16_t* D = (uint16_t*)(base + ws.d);      // [ldt][ldd_row]: kDhGroup slabs side by side
+  uint16_t* D = (uint16_t*)(base + ws.d);      // [ldt][ldd_row]: one vocabulary group
   float* dH32 = (float*)(base + ws.dh32);      // [T][H]
   const uint16_t* h = (const uint16_t*)hidden;
   const uint16_t* w = (const uint16_t*)weight;
@@ -1017,64 +1044,66 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
         reinterpret_cast<u32x4*>(D + T * ws.ldd_row), n16);
     SIIRL_LAUNCH_CHECK("zero_fill_kernel");
   }
-  int dh_splits = 1;
   const int64_t dh32_stride = (int64_t)(round_up((size_t)T * H * 4, 256) / 4);
-  int slab_idx = 0;
   const int tiles_t = (int)((T + BN - 1) / BN);
-  for (int64_t v0 = 0; v0 < V; v0 += kSlab, ++slab_idx) {
-    const int N = (int)((V - v0) < kSlab ? (V - v0) : kSlab);
+  // The recompute goes in launches of about 2048 workgroups (8192 columns at 16384 tokens, whose 59 MB of W stay in the
+  // memory-side cache while the token tiles pass over them: 0.4 % of the whole step faster than one launch per group).  At
+  // T=200 that is one launch of 594 workgroups; 19 launches of 8192 columns had 32 each (1766 against 330 us).
+  const int slab = 8192 * (tiles_t < 64 ? 64 / tiles_t : 1);
+  for (int64_t v0 = 0; v0 < V; v0 += ws.group) {
+    const int N = (int)(V - v0 < ws.group ? V - v0 : ws.group);
     const int Npad = (int)round_up(N, BK);
-    const int gs = slab_idx % kDhGroup;  // position of this slab in its group of D columns
     if (!saved_logits) {
-      DlogitsEpi epi{inv_temperature, (int)T, N, Npad, v0, lse, ex, g_logprob, g_entropy, labels,
-                     D + (int64_t)gs * kSlab, ws.ldd_row};
-      if (int rc = f16 ? launch_gemm<DlogitsEpi, false, true>(w + v0 * Kc, Kc, hp, Kc / 32, N, (int)T, (int)Kc, epi, st,
-                                                              "gemm_nt_kernel<DlogitsEpi, f16>", 1, kBlkRecompute)
-                       : launch_gemm(w + v0 * Kc, Kc, hp, Kc / 32, N, (int)T, (int)Kc, epi, st, "gemm_nt_kernel<DlogitsEpi>", 1,
-                                     kBlkRecompute))
-        return rc;
-    } else if (gs == 0) {
-      // the whole group's dlogits in one pass over the tiles the forward parked
-      const int64_t left = V - v0, cap = (int64_t)kDhGroup * kSlab;
-      const int Ng = (int)(left < cap ? left : cap);
-      DlogitsEpi epi{inv_temperature, (int)T, Ng, (int)round_up(Ng, BK), v0, lse, ex, g_logprob, g_entropy, labels,
-                     D, ws.ldd_row};
+      for (int s0 = 0; s0 < N; s0 += slab) {
+        const int Ns = N - s0 < slab ? N - s0 : slab;
+        const DlogitsEpi epi{inv_temperature, (int)T, Ns, (int)round_up(Ns, BK), v0 + s0, lse, ex, g_logprob, g_entropy,
+                             labels, D + s0, ws.ldd_row};
+        const uint16_t* ws0 = w + (v0 + s0) * Kc;
+        if (int rc = f16 ? launch_gemm<DlogitsEpi, false, true>(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st,
+                                                                "gemm_nt_kernel<DlogitsEpi, f16>", 1, kBlkRecompute)
+                         : launch_gemm(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st, "gemm_nt_kernel<DlogitsEpi>", 1,
+                                       kBlkRecompute))
+          return rc;
+      }
+    } else {
+      // the group's dlogits in one pass over the tiles the forward parked
+      const DlogitsEpi epi{inv_temperature, (int)T, N, Npad, v0, lse, ex, g_logprob, g_entropy, labels, D, ws.ldd_row};
       const void* fn = reinterpret_cast<const void*>(&replay_tiles_kernel<DlogitsEpi>);
       if (int rc = allow_dynamic_lds(fn, kSmemBytes)) return rc;
-      const int64_t wgs = (int64_t)((Ng + BM - 1) / BM) * tiles_t;
+      const int64_t wgs = (int64_t)((N + BM - 1) / BM) * tiles_t;
       replay_tiles_kernel<DlogitsEpi><<<dim3((unsigned)wgs), dim3(kThreads), kSmemBytes, st>>>(
           saved_logits, tiles_t, (int)(v0 / BM), epi);
       SIIRL_LAUNCH_CHECK("replay_tiles_kernel<DlogitsEpi>");
     }
-    if (want_dh && (gs == kDhGroup - 1 || v0 + kSlab >= V)) {
-      // dH[T, H] += D[T, K] . Wt[H, g0 : g0 + K]^T over the group's columns (only the last slab can be partial)
-      const int64_t g0 = v0 - (int64_t)gs * kSlab;
-      const int K = gs * kSlab + Npad;
-      // the first group decides whether d hidden is accumulated as two K runs; a shallower last group then still
-      // writes both buffers (its second run may be short, never empty: K >= 2 K-steps)
-      if (g0 == 0) dh_splits = pick_splits((int)T, (int)H, K);
-      const int splits = (K / BK >= 2) ? dh_splits : 1;
-      AccumF32Epi acc{dH32, H, dh32_stride, (int)T, (int)H, g0 > 0 ? 1 : 0};
-      if (int rc = launch_gemm(D, ws.ldd_row, Wtp + (g0 / 32) * 64, ws.ldwt / 32, (int)T, (int)H, K, acc, st,
+    if (want_dh) {
+      // dH[T, H] += D[T, K] . Wt[H, v0 : v0 + K]^T over the group's columns.  A shallower last group may take fewer runs
+      // than the first one: it then adds to the first buffers only.
+      int splits = ws.dh_splits;
+      if (v0 > 0) {
+        const int fit = pick_splits(T, H, Npad);
+        splits = fit < splits ? fit : splits;
+        const int KT = Npad / BK, per = (KT + splits - 1) / splits;
+        splits = (KT + per - 1) / per;  // no run is empty
+      }
+      AccumF32Epi acc{dH32, H, dh32_stride, (int)T, (int)H, v0 > 0 ? 1 : 0};
+      if (int rc = launch_gemm(D, ws.ldd_row, Wtp + (v0 / 32) * 64, ws.ldwt / 32, (int)T, (int)H, Npad, acc, st,
                                "gemm_nt_kernel<AccumF32Epi>", splits, kBlkDHidden))
         return rc;
     }
-    if (want_dw && (gs == kDhGroup - 1 || v0 + kSlab >= V)) {
-      // dW[g0 : g0 + M, H] = D[ldt, M]^T . Ht[H, ldt]^T over the group's vocabulary rows: D is the A operand given
-      // by its K-rows (tokens)
-      const int64_t g0 = v0 - (int64_t)gs * kSlab;
-      const int M = gs * kSlab + N;
-      StoreEpi sto{(char*)d_weight + g0 * H * (int64_t)dtype_size(dtype), H, M, (int)H, dtype};
-      if (int rc = launch_gemm<StoreEpi, true>(D, ws.ldd_row, Htp, ws.ldt / 32, M, (int)H, (int)ws.ldt, sto, st,
+    if (want_dw) {
+      // dW[v0 : v0 + N, H] = D[ldt, N]^T . Ht[H, ldt]^T over the group's vocabulary rows: D is the A operand given by its
+      // K-rows (tokens)
+      StoreEpi sto{(char*)d_weight + v0 * H * (int64_t)dtype_size(dtype), H, N, (int)H, dtype};
+      if (int rc = launch_gemm<StoreEpi, true>(D, ws.ldd_row, Htp, ws.ldt / 32, N, (int)H, (int)ws.ldt, sto, st,
                                                "gemm_nt_kernel<StoreEpi, A by K-rows>", 1, kBlkDWeight))
         return rc;
     }
   }
   if (want_dh) {
-    const int64_t n = T * H;
-    const unsigned blocks = (unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-    sum_convert_kernel<<<dim3(blocks), dim3(256), 0, st>>>(dH32, dh_splits > 1 ? dH32 + dh32_stride : nullptr, d_hidden, n,
-                                                           dtype);
+    const int64_t n4 = T * H / 4;  // H is a multiple of BK
+    const unsigned blocks = (unsigned)((n4 + 255) / 256 < 16384 ? (n4 + 255) / 256 : 16384);
+    sum_convert_kernel<<<dim3(blocks), dim3(256), 0, st>>>(reinterpret_cast<const f32x4*>(dH32), dh32_stride / 4, ws.dh_splits,
+                                                           d_hidden, n4, dtype);
     SIIRL_LAUNCH_CHECK("sum_convert_kernel");
   }
   return SIIRL_OK;

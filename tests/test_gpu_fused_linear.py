@@ -100,6 +100,33 @@ def test_fused_random_shapes_sweep(dev):
         FL.set_saved_logits_limit(0)
 
 
+@pytest.mark.parametrize("T,H,V", [(8200, 64, 65793), (8192, 128, 70000), (200, 320, 40000), (31, 64, 131073)])
+def test_column_groups_and_k_runs(dev, T, H, V):
+    """Vocabularies of more than one column group (8192 tokens and more: 65536 columns; the last group is shallower than
+    the first, down to 5 K-steps), and d hidden summed from many K runs (few token tiles).  Reference: float64 on the GPU."""
+    from siirl_amd.fused_linear import FusedLinearForPPO
+
+    h, w, y, g_lp, g_h = (t.to(dev) for t in _inputs(T, H, V, seed=T + V))
+    hd, wd = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    lp, ent = FusedLinearForPPO()(hd, wd, y)
+    torch.autograd.backward([lp, ent], [g_lp, g_h])
+    h64, w64 = h.double(), w.double()
+    dh64, dw64 = torch.empty_like(h64), torch.zeros_like(w64)
+    for lo in range(0, T, 2048):
+        rows = slice(lo, min(lo + 2048, T))
+        logp = torch.log_softmax(h64[rows] @ w64.t().contiguous(), dim=-1)
+        p = logp.exp()
+        ent64 = -(p * logp).sum(-1)
+        lp64 = logp.gather(-1, y[rows, None]).squeeze(-1)
+        assert (lp[rows].double() - lp64).abs().max() < 1e-4 and (ent[rows].double() - ent64).abs().max() < 1e-4
+        d = -g_lp[rows, None].double() * p - g_h[rows, None].double() * p * (logp + ent64[:, None])
+        d[torch.arange(d.shape[0], device=dev), y[rows]] += g_lp[rows].double()
+        dh64[rows] = d @ w64
+        dw64 += d.t().contiguous() @ h64[rows]
+    _check_grad(hd.grad, dh64, "d_hidden")
+    _check_grad(wd.grad, dw64, "d_weight")
+
+
 def test_single_branches_3d_and_linear_cross_entropy(dev):
     from siirl_amd.fused_linear import FusedLinearForPPO, linear_cross_entropy
 
