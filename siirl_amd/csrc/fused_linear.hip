@@ -29,6 +29,8 @@
 // one streaming pass.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace siirl {
 namespace {
 
@@ -183,23 +185,25 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(b[j][0]) : "v"(offB[j]), "s"(base));
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:1024" : "=v"(b[j][1]) : "v"(offB[j]), "s"(base));
   };
-  // waits until only this wave's last kDmaPerWave loads (one stage of DMA) are in flight and ties the B registers
-  // to the wait
+  // waits until only this wave's last N loads are in flight (N = kDmaPerWave: one stage of DMA) and ties the B
+  // registers to the wait
   static_assert(NJ * KS == 8 && kDmaPerWave % 2 == 0, "see the load schedule of a K-step");
-  auto bwait = [&](u32x4 (&b)[NJ][KS]) {
+  auto bwait = [&](u32x4 (&b)[NJ][KS], auto in_flight) {
     asm volatile("s_waitcnt vmcnt(%[n])"
                  : "+v"(b[0][0]), "+v"(b[0][1]), "+v"(b[1][0]), "+v"(b[1][1]), "+v"(b[2][0]), "+v"(b[2][1]),
                    "+v"(b[3][0]), "+v"(b[3][1])
-                 : [n] "n"(kDmaPerWave)
+                 : [n] "n"(decltype(in_flight)::value)
                  : "memory");
   };
+  using OneStage = std::integral_constant<int, kDmaPerWave>;
+  using Nothing = std::integral_constant<int, 0>;
 
 #pragma unroll
   for (int j = 0; j < NJ; ++j) bload(b0, 0, j);
   dma(0, 0);
   dma(1, KT > 1 ? 1 : 0);
   dma(2, KT > 2 ? 2 : 0);
-  bwait(b0);
+  bwait(b0, OneStage{});
   __syncthreads();
 
   // A fragments of MFMA group gq = 2 * s + hf: K slice s (32 columns), row blocks hf * 4 .. hf * 4 + 3 of the wave's
@@ -216,9 +220,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   const int tq = m15 >> 2;
   const int xt0 = (kq * 8 + tq) * 512 + wm * 256 + (lane & 3) * 8 + (tq << 5);  // row block ii: xt0 ^ (ii << 5)
 
-  // step kt: stage kt % 4 is read; B(kt + 1) and DMA(kt + 3) are issued (K-steps past the end are clamped to the
-  // last one: they land in stages that are not read again); the barrier at the end publishes stage
-  // (kt + 2) % 4, whose DMA was issued one step earlier, and frees stage kt % 4 for DMA(kt + 4).
+  // step kt: stage kt % 4 is read; B(kt + 1) and DMA(kt + 3) are issued; the barrier at the end publishes stage
+  // (kt + 2) % 4, whose DMA was issued one step earlier, and frees stage kt % 4 for DMA(kt + 4).  The last three steps
+  // have nothing left to fetch by DMA and wait for all loads instead; the last one fetches and publishes nothing.
   // A fragments are read one MFMA group ahead; the group after the last one of a step is the first of the next
   // step, whose stage was published by the previous barrier, so the reads cross the barrier.
   bf16x8 afa[4], afb[4];
@@ -267,33 +271,61 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
     mma(af, bc, gq);
     __builtin_amdgcn_s_setprio(0);
   };
-  auto step = [&](int kt, u32x4 (&bc)[NJ][KS], u32x4 (&bn)[NJ][KS]) {
+  enum { STEP_MAIN, STEP_TAIL, STEP_LAST };
+  auto step = [&](auto kind, int kt, u32x4 (&bc)[NJ][KS], u32x4 (&bn)[NJ][KS]) {
+    constexpr int kKind = decltype(kind)::value;
     const int stage = kt & 3;
-    const int ktb = kt + 1 < KT ? kt + 1 : KT - 1, kta = kt + 3 < KT ? kt + 3 : KT - 1;
+    if constexpr (kKind != STEP_LAST)
 #pragma unroll
-    for (int j = 0; j < NJ / 2; ++j) bload(bn, ktb, j);
+      for (int j = 0; j < NJ / 2; ++j) bload(bn, kt + 1, j);
     fread(afb, stage, 1);
     mma_prio(afa, bc, 0);
+    if constexpr (kKind != STEP_LAST)
 #pragma unroll
-    for (int j = NJ / 2; j < NJ; ++j) bload(bn, ktb, j);
+      for (int j = NJ / 2; j < NJ; ++j) bload(bn, kt + 1, j);
     fread(afa, stage, 2);
     mma_prio(afb, bc, 1);
-    dma((stage + 3) & 3, kta, 0, kDmaPerWave / 2);
+    if constexpr (kKind == STEP_MAIN) dma((stage + 3) & 3, kt + 3, 0, kDmaPerWave / 2);
     fread(afb, stage, 3);
     mma_prio(afa, bc, 2);
-    dma((stage + 3) & 3, kta, kDmaPerWave / 2, kDmaPerWave);
-    fread(afa, (stage + 1) & 3, 0);
+    if constexpr (kKind == STEP_MAIN) dma((stage + 3) & 3, kt + 3, kDmaPerWave / 2, kDmaPerWave);
+    if constexpr (kKind != STEP_LAST) fread(afa, (stage + 1) & 3, 0);
     mma_prio(afb, bc, 3);
-    bwait(bn);
-    __syncthreads();
+    if constexpr (kKind == STEP_MAIN) bwait(bn, OneStage{});
+    if constexpr (kKind == STEP_TAIL) bwait(bn, Nothing{});
+    if constexpr (kKind != STEP_LAST) __syncthreads();
+  };
+  using Main = std::integral_constant<int, STEP_MAIN>;
+  using Tail = std::integral_constant<int, STEP_TAIL>;
+  using Last = std::integral_constant<int, STEP_LAST>;
+  // The pairs of main steps swap the two B register sets by name.  What follows them moves the 32 registers instead: with
+  // a copy of the tail for each parity the compiler loses the accumulators' places where the copies join (1773 spills).
+  auto take_over = [&]() {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) b0[j][s] = b1[j][s];
   };
   int kt = 0;
-  for (; kt + 2 <= KT; kt += 2) {
-    step(kt, b0, b1);
-    step(kt + 1, b1, b0);
+  for (; kt + 5 <= KT; kt += 2) {
+    step(Main{}, kt, b0, b1);
+    step(Main{}, kt + 1, b1, b0);
   }
-  if (kt < KT) step(kt, b0, b1);
-  // the clamped DMA of the last steps may still be in flight and the epilogue reuses the LDS
+  if (kt + 4 <= KT) {
+    step(Main{}, kt++, b0, b1);
+    take_over();
+  }
+  if (KT >= 3) {
+    step(Tail{}, kt++, b0, b1);
+    take_over();
+  }
+  if (KT >= 2) {
+    step(Tail{}, kt++, b0, b1);
+    take_over();
+  }
+  step(Last{}, kt, b0, b1);
+  // nothing is in flight here but, with fewer than three K-steps, the spare DMA of the prologue; the epilogue reuses
+  // the LDS
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   epi(acc, m0, n0, tc.tm, split, wm, wn, lane, tid, smem);
