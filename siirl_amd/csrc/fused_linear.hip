@@ -108,6 +108,11 @@ __device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) {
   return wm * (MI * 16) + i * 16 + (lane >> 4) * 4 + r;
 }
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * (NJ * 16) + j * 16 + (lane & 15); }
+// An epilogue with kRowsPerLane takes the accumulator the other way round (the MFMA's operands are swapped): a lane owns
+// the rows row_of_lane(i) and, with B packed in the column order of transpose_pack_b_kernel, the 16 consecutive columns
+// from col_of_lane on: element r of acc[i][j] is column col_of_lane + 4 * j + r.
+__device__ __forceinline__ int row_of_lane(int wm, int i, int lane) { return wm * (MI * 16) + i * 16 + (lane & 15); }
+__device__ __forceinline__ int col_of_lane(int wn, int lane) { return wn * (NJ * 16) + (lane >> 4) * 16; }
 
 // m0 (the DMA's LDS base) is a reserved register: naming it in a clobber list is right but draws a warning
 #pragma clang diagnostic push
@@ -115,6 +120,7 @@ __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * (N
 // F16: the 16-bit operands are IEEE half instead of bf16 (the same data movement, the other MFMA)
 template <class Epi, bool AT = false, bool F16 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_nt_kernel(GemmArgs g, Epi epi) {
+  static_assert(!(F16 && Epi::kRowsPerLane), "the gradient GEMMs multiply bf16");
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w / WN, wn = w % WN;
@@ -257,6 +263,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
         floatx4& c = acc[hf * 4 + ii][j];
         if constexpr (F16)
           c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, af[ii]), __builtin_bit_cast(f16x8, bc[j][s]), c, 0, 0, 0);
+        else if constexpr (Epi::kRowsPerLane)
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bc[j][s]), af[ii], c, 0, 0, 0);
         else
           c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[ii], __builtin_bit_cast(bf16x8, bc[j][s]), c, 0, 0, 0);
       }
@@ -372,6 +380,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 // Per token of the tile: mx = max_v z, s = sum exp(z - mx), t = sum z * exp(z - mx) over the tile's 256
 // vocabulary rows, z = acc * inv_T; one (mx, s, t) per token is written to part[tm][.][token].
 struct SoftmaxPartialsEpi {
+  static constexpr bool kRowsPerLane = false;
   float inv_T;
   int T, V;
   float* part;  // [tiles_m][3][T]
@@ -458,6 +467,7 @@ struct SoftmaxPartialsEpi {
 // so the per-token coefficients are loaded once per lane and D gets 8-byte stores.  This one token-major layout
 // serves both consumers: d hidden reads it as its A[M = token][K = vocabulary], d weight as A given by K-rows.
 struct DlogitsEpi {
+  static constexpr bool kRowsPerLane = false;
   float inv_T;
   int T, Vs, Vpad;
   int64_t v0;  // first vocabulary column of the group
@@ -519,54 +529,78 @@ struct DlogitsEpi {
 
 // ------------------------------------------------------------------------------ epilogues: plain stores
 
+// Both take the accumulator by rows: a lane holds 16 consecutive columns of a row, 32 (16-bit) or 64 bytes, and the four
+// lanes of a row a whole 128-byte line or two.  With a column per lane each store instruction wrote 2-byte (d weight) or
+// 4-byte pieces, 128 per lane and tile instead of 16 or 32.  N is a multiple of 64, so a wave's columns are all inside
+// the matrix or all outside.
+
 struct AccumF32Epi {  // C_s[row][col] = (beta ? C_s : 0) + acc, one fp32 buffer C_s = C + s * split_stride per K run
+  static constexpr bool kRowsPerLane = true;
   float* C;
   int64_t ldc, split_stride;
   int M, N, beta;
   __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn, int lane, int tid,
                              char* smem) const {
+    const int col = n0 + col_of_lane(wn, lane);
+    if (col >= N) return;
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i) {
+      const int row = m0 + row_of_lane(wm, i, lane);
+      if (row >= M) continue;
+      f32x4* p = reinterpret_cast<f32x4*>(C + split * split_stride + (int64_t)row * ldc + col);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + acc_row(wm, i, r, lane);
-        if (row >= M) continue;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int col = n0 + acc_col(wn, j, lane);
-          if (col >= N) continue;
-          float* p = C + split * split_stride + (int64_t)row * ldc + col;
-          *p = beta ? *p + acc[i][j][r] : acc[i][j][r];
-        }
-      }
+      for (int j = 0; j < NJ; ++j) p[j] = beta ? p[j] + acc[i][j] : acc[i][j];
+    }
   }
 };
 
+// one value rounded to SIIRL_BF16, SIIRL_F16 or SIIRL_F32 and stored as element `at` of `out`
+__device__ __forceinline__ void store_one(void* out, int64_t at, float v, int out_dtype) {
+  if (out_dtype == SIIRL_BF16)
+    reinterpret_cast<uint16_t*>(out)[at] = (uint16_t)(pack_bf16(v, 0.f) & 0xffffu);
+  else if (out_dtype == SIIRL_F16)
+    reinterpret_cast<uint16_t*>(out)[at] = (uint16_t)(pack_f16(v, 0.f) & 0xffffu);
+  else
+    reinterpret_cast<float*>(out)[at] = v;
+}
+__device__ __forceinline__ uint2 pack4(floatx4 v, int out_dtype) {
+  return out_dtype == SIIRL_BF16 ? make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w))
+                                 : make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
+}
+
 struct StoreEpi {  // C[row][col] = acc, rounded to the output type (out_dtype: SIIRL_BF16, SIIRL_F16 or SIIRL_F32)
+  static constexpr bool kRowsPerLane = true;
   void* C;
   int64_t ldc;
   int M, N, out_dtype;
   __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn, int lane, int tid,
                              char* smem) const {
+    const int col = n0 + col_of_lane(wn, lane);
+    if (col >= N) return;
+    const bool aligned = ((uintptr_t)C & 15) == 0;  // (a caller's buffer need not be; ldc and col are multiples of 16)
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i) {
+      const int row = m0 + row_of_lane(wm, i, lane);
+      if (row >= M) continue;
+      const int64_t at = (int64_t)row * ldc + col;
+      if (!aligned) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + acc_row(wm, i, r, lane);
-        if (row >= M) continue;
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int col = n0 + acc_col(wn, j, lane);
-          if (col >= N) continue;
-          const int64_t at = (int64_t)row * ldc + col;
-          if (out_dtype == SIIRL_BF16)
-            reinterpret_cast<uint16_t*>(C)[at] = (uint16_t)(pack_bf16(acc[i][j][r], 0.f) & 0xffffu);
-          else if (out_dtype == SIIRL_F16)
-            reinterpret_cast<uint16_t*>(C)[at] = (uint16_t)(pack_f16(acc[i][j][r], 0.f) & 0xffffu);
-          else
-            reinterpret_cast<float*>(C)[at] = acc[i][j][r];
+          for (int r = 0; r < 4; ++r) store_one(C, at + j * 4 + r, acc[i][j][r], out_dtype);
+      } else if (out_dtype == SIIRL_F32) {
+        f32x4* p = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + at);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) p[j] = acc[i][j];
+      } else {
+        u32x4* p = reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(C) + at);
+#pragma unroll
+        for (int j = 0; j < NJ; j += 2) {
+          const uint2 a = pack4(acc[i][j], out_dtype), b = pack4(acc[i][j + 1], out_dtype);
+          p[j / 2] = u32x4{a.x, a.y, b.x, b.y};
         }
       }
+    }
   }
 };
 
@@ -589,7 +623,8 @@ __global__ __launch_bounds__(256) void pack_b_kernel(const uint16_t* __restrict_
 }
 
 // The same packing of the transpose: B[n][k] = in[k][n] with in of shape [R = K][C = N].  A workgroup stages a
-// 64 x 64 tile through LDS and emits its 512 chunks.
+// 64 x 64 tile through LDS and emits its 512 chunks.  Within each 64 columns, column n = 16 q + 4 j + r takes the place
+// of row 4 q + r of 16-row block j, so that an epilogue with kRowsPerLane finds 16 consecutive columns in a lane.
 // from_f16: the input holds IEEE halves, the packed output bf16 (round to nearest even).
 __device__ __forceinline__ uint32_t half2_to_bf16x2(uint32_t w) { return pack_bf16(f16_lo(w), f16_hi(w)); }
 __global__ __launch_bounds__(256) void transpose_pack_b_kernel(const uint16_t* __restrict__ in, int64_t ld_in, int R,
@@ -622,7 +657,9 @@ __global__ __launch_bounds__(256) void transpose_pack_b_kernel(const uint16_t* _
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = (uint32_t)tile[kc * 8 + 2 * e][nl] | ((uint32_t)tile[kc * 8 + 2 * e + 1][nl] << 16);
     const int64_t n = c0 + nl, k = r0 + kc * 8;
-    const int64_t ch = ((n >> 4) * KB + (k >> 5)) * 64 + (n & 15) + 16 * ((k >> 3) & 3);
+    const int64_t nb = (n >> 6) * 4 + ((n >> 2) & 3);                       // 16-row block
+    const int nr = (int)(((n >> 4) & 3) * 4 + (n & 3));                     // row in it
+    const int64_t ch = (nb * KB + (k >> 5)) * 64 + nr + 16 * ((k >> 3) & 3);
     out[ch] = u32x4{w[0], w[1], w[2], w[3]};
   }
 }
@@ -712,15 +749,18 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(const float* __rest
 // SIIRL_F32).  A pure stream: 16-byte loads, the buffers added in their order.
 __global__ __launch_bounds__(256) void sum_convert_kernel(const f32x4* __restrict__ in, int64_t stride, int splits,
                                                           void* __restrict__ out, int64_t n4, int out_dtype) {
+  const bool aligned = ((uintptr_t)out & 15) == 0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (int64_t)gridDim.x * 256) {
     f32x4 v = in[i];
     for (int s = 1; s < splits; ++s) v += in[s * stride + i];
-    if (out_dtype == SIIRL_BF16)
-      reinterpret_cast<uint2*>(out)[i] = make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
-    else if (out_dtype == SIIRL_F16)
-      reinterpret_cast<uint2*>(out)[i] = make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
-    else
+    if (!aligned) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) store_one(out, i * 4 + r, v[r], out_dtype);
+    } else if (out_dtype == SIIRL_F32) {
       reinterpret_cast<f32x4*>(out)[i] = v;
+    } else {
+      reinterpret_cast<uint2*>(out)[i] = pack4(v, out_dtype);
+    }
   }
 }
 
