@@ -386,6 +386,48 @@ struct SoftmaxPartialsEpi {
   float* part;  // [tiles_m][3][T]
   float* save;  // null, or the parked accumulator tiles (see saved_tile)
   int tiles_n;
+  // The wave's (mx, s, t) of each of its tokens, to sh[wm][token].  Works on the raw accumulator a (z = a * inv_T):
+  // a maximum, one fused multiply-add, one exp2 and two accumulations per logit; no matrix work runs beside this, so
+  // its length counts in full (FULL: no vocabulary row of the tile is past the end, nothing is compared or selected).
+  template <bool FULL>
+  __device__ __forceinline__ void reduce(floatx4 (&acc)[MI][NJ], int m0, int wm, int wn, int lane, float* sh) const {
+    const float ninf = -__builtin_inff();
+    const float ek = inv_T * kLog2e;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      float mx = ninf;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (FULL || m0 + acc_row(wm, i, r, lane) < V) mx = fmaxf(mx, acc[i][j][r]);
+      mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+      float s = 0.f, t = 0.f;
+      if (mx > ninf) {
+        const float nmk = -mx * ek;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (!FULL && m0 + acc_row(wm, i, r, lane) >= V) continue;
+            const float e = fast_exp2(fmaf(acc[i][j][r], ek, nmk));
+            s += e;
+            t = fmaf(acc[i][j][r], e, t);
+          }
+      }
+      s += __shfl_xor(s, 16, kWave);
+      t += __shfl_xor(t, 16, kWave);
+      s += __shfl_xor(s, 32, kWave);
+      t += __shfl_xor(t, 32, kWave);
+      if (lane < 16) {
+        float* d = sh + (wm * BN + acc_col(wn, j, lane)) * 3;
+        d[0] = mx * inv_T;
+        d[1] = s;
+        d[2] = t * inv_T;
+      }
+    }
+  }
   __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn,
                                              int lane, int tid, char* smem) const {
     // Parking costs about 11 us per tile (256 KB per workgroup): the workgroup's own drain, not a burst of the round.
@@ -399,44 +441,10 @@ struct SoftmaxPartialsEpi {
     float* sh = reinterpret_cast<float*>(smem);  // [WM][BN][3]; the main loop's last barrier freed the LDS
     const float k = kLog2e;
     const float ninf = -__builtin_inff();
-    const bool full = m0 + BM <= V;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      float mx = ninf;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const bool ok = full || (m0 + acc_row(wm, i, r, lane) < V);
-          mx = fmaxf(mx, ok ? acc[i][j][r] * inv_T : ninf);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-      float s = 0.f, t = 0.f;
-      if (mx > ninf) {
-        const float nmk = -mx * k;
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const bool ok = full || (m0 + acc_row(wm, i, r, lane) < V);
-            const float x = acc[i][j][r] * inv_T;
-            const float e = ok ? fast_exp2(fmaf(x, k, nmk)) : 0.f;
-            s += e;
-            t = fmaf(ok ? x : 0.f, e, t);
-          }
-      }
-      s += __shfl_xor(s, 16, kWave);
-      t += __shfl_xor(t, 16, kWave);
-      s += __shfl_xor(s, 32, kWave);
-      t += __shfl_xor(t, 32, kWave);
-      if (lane < 16) {
-        float* d = sh + (wm * BN + acc_col(wn, j, lane)) * 3;
-        d[0] = mx;
-        d[1] = s;
-        d[2] = t;
-      }
-    }
+    if (m0 + BM <= V)
+      reduce<true>(acc, m0, wm, wn, lane, sh);
+    else
+      reduce<false>(acc, m0, wm, wn, lane, sh);
     __syncthreads();
     const int tok = n0 + tid;
     if (tid < BN && tok < T) {
