@@ -8,12 +8,9 @@
 // are bit-identical to the reference's):
 //   delta = r_t + gamma * V_next - V_t ;  cand = delta + (gamma * lam) * A_next
 //   V_next <- V_t * m_t + (1 - m_t) * V_next ;  A_next <- cand * m_t + (1 - m_t) * A_next ;  A_t = A_next
-// A workgroup is one wave that owns 16 rows and walks them right to left in tiles of 128 columns: the tile's
-// rewards, values and mask are fetched with 16-byte loads (coalesced, four rows per wave instruction) into
-// registers while the previous tile is being scanned, pass through LDS, lanes 0-15 each walk one row of the tile
-// (the recurrence is sequential: ~12 dependent-ish float operations per token), and the results leave row-wise
-// again.  Rows are independent, so waves never synchronise with each other; 16 rows per wave gives B / 16 waves
-// (343 at B = 5488) to spread over the chip, each bound by the latency of its own chain.
+// The recurrence is sequential, so the time of one row is the latency of its chain; everything that is not the chain is
+// taken off it (gae_scan_kernel).  A scan over chunks of rows stitched through affine maps is there for callers that
+// do not need the reference's order (gae_compose_kernel, gae_carry_kernel).
 #include "common.hpp"
 #include "loss_token.hpp"
 
@@ -74,44 +71,260 @@ __device__ __forceinline__ void gae_compose(float r, float v, float m, float gam
   g.b1 = b1;
 }
 
-enum { MODE_SCAN = 0, MODE_COMPOSE = 1 };
+// Four masks as floats from the 16-byte (int64: 32-byte, u8: 4-byte) pieces of a quad.
+template <int MK, bool F32MASK>
+__device__ __forceinline__ float4 mask_quad(const u32x4& a, const u32x4& b) {
+  if (MK == MK_I64) {
+    // values that fit 32 bits (every mask in practice) convert with one instruction each
+    const bool wide = ((int32_t)a.y != ((int32_t)a.x >> 31)) | ((int32_t)a.w != ((int32_t)a.z >> 31)) |
+                      ((int32_t)b.y != ((int32_t)b.x >> 31)) | ((int32_t)b.w != ((int32_t)b.z >> 31));
+    if (__builtin_amdgcn_ballot_w64(wide) == 0)
+      return make_float4((float)(int32_t)a.x, (float)(int32_t)a.z, (float)(int32_t)b.x, (float)(int32_t)b.z);
+    return make_float4((float)(int64_t)(((uint64_t)a.y << 32) | a.x), (float)(int64_t)(((uint64_t)a.w << 32) | a.z),
+                       (float)(int64_t)(((uint64_t)b.y << 32) | b.x), (float)(int64_t)(((uint64_t)b.w << 32) | b.z));
+  }
+  if (MK == MK_B32)
+    return F32MASK ? make_float4(u2f(a.x), u2f(a.y), u2f(a.z), u2f(a.w))
+                   : make_float4((float)(int32_t)a.x, (float)(int32_t)a.y, (float)(int32_t)a.z, (float)(int32_t)a.w);
+  return make_float4((float)(a.x & 0xffu), (float)((a.x >> 8) & 0xffu), (float)((a.x >> 16) & 0xffu), (float)(a.x >> 24));
+}
+template <int MK>
+__device__ __forceinline__ void load_mask_pieces(const void* mask, int64_t idx, u32x4& a, u32x4& b) {
+  if (MK == MK_I64) {
+    a = reinterpret_cast<const u32x4*>((const int64_t*)mask + idx)[0];
+    b = reinterpret_cast<const u32x4*>((const int64_t*)mask + idx)[1];
+  } else if (MK == MK_B32) {
+    a = *reinterpret_cast<const u32x4*>((const uint32_t*)mask + idx);
+  } else {
+    a = u32x4{*reinterpret_cast<const uint32_t*>((const uint8_t*)mask + idx), 0u, 0u, 0u};
+  }
+}
 
-// MODE_SCAN: the recurrence itself, from the state `init` gives each row (zero when null).  MODE_COMPOSE: no output
-// per token; each row's tokens are folded into one GaeMap written to `maps`.  With rows that are chunks of the real
-// rows (B = rows x chunks, L = chunk length: chunks of a row are adjacent in memory) a compose pass, a carry over
-// the chunk maps and a scan pass evaluate the recurrence with a dependent chain of one chunk instead of one row.
-template <int MK, bool F32MASK, int MODE>
-__global__ __launch_bounds__(kWave) void gae_scan_vec_kernel(const float* __restrict__ rewards,
-                                                              const float* __restrict__ values,
-                                                              const void* __restrict__ mask, int64_t B, int64_t L,
-                                                              float gamma, float gamma_lam, float* __restrict__ adv,
-                                                              float* __restrict__ ret, double* __restrict__ part,
-                                                              const float* __restrict__ init,
-                                                              float* __restrict__ maps) {
-  __shared__ __align__(16) float s_r[kRows * kPitch], s_v[kRows * kPitch], s_m[kRows * kPitch], s_a[kRows * kPitch];
+// The exact-order scan.  What bounds it is the dependent chain of a row.  For masks of zeros and ones over finite data
+// the recurrence is, term for term and with the same roundings,
+//   A <- m ? delta + (gamma * lam) * A : A ,   delta = (r + gamma * V') - v ,   V' = the value of the nearest token to
+// the right with m = 1 (the row's entering state if there is none), so that only a product and a sum per token remain
+// on the chain:  A <- d + k * A  with d = delta, k = gamma * lam where m = 1 and d = 0, k = 1 where m = 0.  (Zeros may
+// differ in their sign.)  A workgroup owns four rows in tiles of 128 columns, right to left.  Its first wave walks the
+// chain, a row per lane; two more waves fetch the tiles four ahead (16-byte loads), prepare d and k a tile ahead and
+// store the tile behind with its whitening statistics.  Four rows per workgroup: 256 workgroups at B = 1024.
+// B = 1024, L = 8192, int64 mask: 91 us (2.6 TB/s); one wave per 16 rows that also loaded, converted and stored was 508 us
+// (149 cycles a token).
+// A tile with another mask value, or with a delta that is not finite and moderate, or that takes A out of the finite
+// numbers, is walked by the recurrence as it stands, and so is the rest of those rows (`slow`).
+constexpr int kScanRows = 4, kScanHelpers = kScanRows * kCols / 4, kScanThreads = kWave + kScanHelpers, kAhead = 4;
+static_assert(kScanHelpers % kWave == 0 && kCols / 4 == 32, "a helper wave holds two rows, a quad per lane");
+
+template <int MK, bool F32MASK>
+__global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __restrict__ rewards,
+                                                                const float* __restrict__ values,
+                                                                const void* __restrict__ mask, int64_t B, int64_t L,
+                                                                float gamma, float gamma_lam, float* __restrict__ adv,
+                                                                float* __restrict__ ret, double* __restrict__ part,
+                                                                const float* __restrict__ init) {
+  // two buffers of each: tile t + 1 is prepared and tile t - 1 stored while tile t is walked
+  __shared__ __align__(16) float s_d[2][kScanRows * kPitch], s_k[2][kScanRows * kPitch], s_a[2][kScanRows * kPitch];
+  __shared__ __align__(16) float s_r[2][kScanRows * kPitch], s_v[2][kScanRows * kPitch], s_m[2][kScanRows * kPitch];
+  __shared__ float s_nv[2][kScanRows];                          // V' entering the tile
+  __shared__ int s_slow[2][kScanHelpers / kWave];               // the tile needs the recurrence as it stands
+  __shared__ double s_st[kScanHelpers / kWave][kNStat];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int64_t row0 = (int64_t)blockIdx.x * kScanRows;
+  const int nrows = (int)((B - row0) < kScanRows ? (B - row0) : kScanRows);
+  const int NT = (int)((L + kCols - 1) / kCols);  // tile t covers the columns from (NT - 1 - t) * kCols
+
+  if (__builtin_amdgcn_readfirstlane(tid / kWave) == 0) {
+    // ---- the chain
+    float nv = 0.f, lg = 0.f;
+    if (init != nullptr && lane < nrows) lg = init[2 * (row0 + lane) + 1];
+    bool slow = !(fabsf(gamma_lam) <= 1.f);
+    bool first_slow = true;
+    const int row = lane < kScanRows ? lane : 0;  // (the other lanes walk row 0 again and store nothing)
+    for (int i = 0; i < (NT + 1) / kAhead * kAhead + kAhead; ++i) {  // (as many barriers as the helpers meet)
+      const int t = i - 1;
+      if (t >= 0 && t < NT) {
+        const int b = t & 1;
+        const float entering = lg;
+        slow |= __builtin_amdgcn_readfirstlane(s_slow[b][0] | s_slow[b][1]) != 0;
+        if (!slow) {
+          const float* d = s_d[b] + row * kPitch;
+          const float* k = s_k[b] + row * kPitch;
+          float* a = s_a[b] + row * kPitch;
+          // the LDS reads of the next 16 tokens are issued before the current 16 are walked
+          float4 dc[4], kc[4], dn[4], kn[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            dc[q] = *reinterpret_cast<const float4*>(d + kCols - 16 + 4 * q);
+            kc[q] = *reinterpret_cast<const float4*>(k + kCols - 16 + 4 * q);
+          }
+#pragma unroll
+          for (int cc = kCols - 16; cc >= 0; cc -= 16) {
+            const int nx = cc >= 16 ? cc - 16 : 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              dn[q] = *reinterpret_cast<const float4*>(d + nx + 4 * q);
+              kn[q] = *reinterpret_cast<const float4*>(k + nx + 4 * q);
+            }
+#pragma unroll
+            for (int q = 3; q >= 0; --q) {
+              float4 o;
+              lg = dc[q].w + kc[q].w * lg; o.w = lg;
+              lg = dc[q].z + kc[q].z * lg; o.z = lg;
+              lg = dc[q].y + kc[q].y * lg; o.y = lg;
+              lg = dc[q].x + kc[q].x * lg; o.x = lg;
+              if (lane < kScanRows) *reinterpret_cast<float4*>(a + cc + 4 * q) = o;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) dc[q] = dn[q], kc[q] = kn[q];
+          }
+          // an overflow stays: a tile that ends finite was finite throughout
+          if (__builtin_amdgcn_ballot_w64(!(lg - lg == 0.f)) != 0) slow = true, lg = entering;
+        }
+        if (slow) {
+          if (first_slow) nv = s_nv[b][row];
+          first_slow = false;
+          const int64_t c0 = (int64_t)(NT - 1 - t) * kCols;
+          const int ncols = (int)((L - c0) < kCols ? (L - c0) : kCols);  // a multiple of 4
+          const float *r = s_r[b] + row * kPitch, *v = s_v[b] + row * kPitch, *m = s_m[b] + row * kPitch;
+          if (lane < nrows)
+            for (int cc = ncols - 4; cc >= 0; cc -= 4) {
+              const float4 r4 = *reinterpret_cast<const float4*>(r + cc), v4 = *reinterpret_cast<const float4*>(v + cc),
+                           m4 = *reinterpret_cast<const float4*>(m + cc);
+              float4 o;
+              gae_step(r4.w, v4.w, m4.w, gamma, gamma_lam, nv, lg); o.w = lg;
+              gae_step(r4.z, v4.z, m4.z, gamma, gamma_lam, nv, lg); o.z = lg;
+              gae_step(r4.y, v4.y, m4.y, gamma, gamma_lam, nv, lg); o.y = lg;
+              gae_step(r4.x, v4.x, m4.x, gamma, gamma_lam, nv, lg); o.x = lg;
+              *reinterpret_cast<float4*>(s_a[b] + lane * kPitch + cc) = o;
+            }
+        }
+      }
+      __syncthreads();
+    }
+  } else {
+    // ---- loads, preparation, stores: quad `ch` of row `rr` in every tile
+    const int hl = tid - kWave, rr = hl >> 5, ch = hl & 31, half = lane & 32, hw = hl / kWave;
+    const bool row_in = rr < nrows;
+    const int64_t rbase = (row0 + (row_in ? rr : 0)) * L;  // (rows and columns past the edges load what is there)
+    const int o = rr * kPitch + 4 * ch;
+    float carry = init != nullptr && row_in ? init[2 * (row0 + rr)] : 0.f;
+    u32x4 pr[kAhead], pv[kAhead], pa[kAhead], pb[kAhead];
+    auto stat_add = [](double (&s)[kNStat], float x, float m) {
+      const double d = m != 0.f ? (double)x : 0.0, md = (double)m * d;
+      s[0] += md;
+      s[1] += md * d;
+      s[2] += (double)m;
+    };
+    auto issue = [&](int t, u32x4& r, u32x4& v, u32x4& a, u32x4& b) {
+      int64_t col = (int64_t)(t < NT ? NT - 1 - t : 0) * kCols + 4 * ch;
+      if (col >= L) col = L - 4;
+      r = *reinterpret_cast<const u32x4*>(rewards + rbase + col);
+      v = *reinterpret_cast<const u32x4*>(values + rbase + col);
+      load_mask_pieces<MK>(mask, rbase + col, a, b);
+    };
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) issue(u, pr[u], pv[u], pa[u], pb[u]);
+    float4 v1 = make_float4(0.f, 0.f, 0.f, 0.f), m1 = v1, v2 = v1, m2 = v1;  // of the tiles t and t - 1
+    double st[kNStat] = {0.0, 0.0, 0.0};  // whitening statistics of the advantages (pivot 0)
+#pragma unroll 1
+    for (int t0 = -1; t0 <= NT; t0 += kAhead) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int t = t0 + u;
+        // Every interval prepares and fetches, past the last tile too (of zeros, from clamped addresses; nothing reads
+        // them): with a fixed number of loads between a load and its use the wait for it leaves the later ones in flight.
+        {  // store tile t - 1
+          const int64_t col = (int64_t)(NT - t) * kCols + 4 * ch;
+          const float4 a = *reinterpret_cast<const float4*>(s_a[(t - 1) & 1] + o);
+          if (row_in && t >= 1 && t <= NT && col < L) {
+            *reinterpret_cast<float4*>(adv + rbase + col) = a;
+            *reinterpret_cast<float4*>(ret + rbase + col) = make_float4(a.x + v2.x, a.y + v2.y, a.z + v2.z, a.w + v2.w);
+          }
+          stat_add(st, a.x, m2.x);
+          stat_add(st, a.y, m2.y);
+          stat_add(st, a.z, m2.z);
+          stat_add(st, a.w, m2.w);
+        }
+        v2 = v1, m2 = m1;
+        {  // prepare tile t + 1
+          const int b = (t + 1) & 1;
+          const bool in = row_in && t + 1 < NT && (int64_t)(NT - 2 - t) * kCols + 4 * ch < L;
+          float4 r = make_float4(u2f(pr[u].x), u2f(pr[u].y), u2f(pr[u].z), u2f(pr[u].w));
+          float4 v = make_float4(u2f(pv[u].x), u2f(pv[u].y), u2f(pv[u].z), u2f(pv[u].w));
+          float4 m = mask_quad<MK, F32MASK>(pa[u], pb[u]);
+          if (!in) r = v = m = make_float4(0.f, 0.f, 0.f, 0.f);
+          issue(t + 1 + kAhead, pr[u], pv[u], pa[u], pb[u]);
+          const bool mx = m.x != 0.f, my = m.y != 0.f, mz = m.z != 0.f, mw = m.w != 0.f;
+          const float lead = mx ? v.x : my ? v.y : mz ? v.z : v.w;  // the quad's leftmost value with m != 0
+          const uint32_t have = (uint32_t)(__builtin_amdgcn_ballot_w64(mx | my | mz | mw) >> half);
+          const uint32_t right = have & ~((2u << ch) - 1u);  // quads of this row to the right
+          const float from_right = __shfl(lead, half + (right ? __builtin_ctz(right) : 0), kWave);
+          const float first = __shfl(lead, half + (have ? __builtin_ctz(have) : 0), kWave);
+          const float nw = right ? from_right : carry;  // V' of the quad's last token
+          const float nz = mw ? v.w : nw, ny = mz ? v.z : nz, nx = my ? v.y : ny;
+          const float4 d = make_float4((r.x + gamma * nx) - v.x, (r.y + gamma * ny) - v.y, (r.z + gamma * nz) - v.z,
+                                       (r.w + gamma * nw) - v.w);
+          constexpr float kBig = 1e30f;  // (added to a finite A it cannot leave the finite numbers for |gamma * lam| <= 1)
+          const bool plain = (!mx | (m.x == 1.f)) & (!my | (m.y == 1.f)) & (!mz | (m.z == 1.f)) & (!mw | (m.w == 1.f)) &
+                             (fabsf(d.x) <= kBig) & (fabsf(d.y) <= kBig) & (fabsf(d.z) <= kBig) & (fabsf(d.w) <= kBig);
+          const bool odd = __builtin_amdgcn_ballot_w64(in & !plain) != 0;
+          *reinterpret_cast<float4*>(s_d[b] + o) = make_float4(mx ? d.x : 0.f, my ? d.y : 0.f, mz ? d.z : 0.f, mw ? d.w : 0.f);
+          *reinterpret_cast<float4*>(s_k[b] + o) = make_float4(mx ? gamma_lam : 1.f, my ? gamma_lam : 1.f,
+                                                               mz ? gamma_lam : 1.f, mw ? gamma_lam : 1.f);
+          *reinterpret_cast<float4*>(s_r[b] + o) = r;
+          *reinterpret_cast<float4*>(s_v[b] + o) = v;
+          *reinterpret_cast<float4*>(s_m[b] + o) = m;
+          if (ch == 0) s_nv[b][rr] = carry;
+          if (lane == 0) s_slow[b][hw] = odd;
+          carry = have ? first : carry;
+          v1 = v, m1 = m;
+        }
+        __syncthreads();
+      }
+    }
+    if (part) {
+#pragma unroll
+      for (int k = 0; k < kNStat; ++k) {
+        const double s = wave_sum(st[k]);
+        if (lane == 0) s_st[hw][k] = s;
+      }
+    }
+  }
+  __syncthreads();
+  if (part && tid < kNStat) {
+    double s = 0.0;
+#pragma unroll
+    for (int h = 0; h < kScanHelpers / kWave; ++h) s += s_st[h][tid];
+    part[(int64_t)kNStat * blockIdx.x + tid] = s;
+  }
+}
+
+// Folds each row's tokens into one GaeMap, written to `maps`.  With rows that are chunks of the real rows (B = rows x
+// chunks, L = chunk length: chunks of a row are adjacent in memory) this pass, a carry over the chunk maps and a scan
+// pass evaluate the recurrence with a dependent chain of one chunk instead of one row.  One wave per 16 rows; the next
+// tile's loads are in flight while a tile, passed through LDS, is folded.
+template <int MK, bool F32MASK>
+__global__ __launch_bounds__(kWave) void gae_compose_kernel(const float* __restrict__ rewards,
+                                                            const float* __restrict__ values,
+                                                            const void* __restrict__ mask, int64_t B, int64_t L,
+                                                            float gamma, float gamma_lam, float* __restrict__ maps) {
+  __shared__ __align__(16) float s_r[kRows * kPitch], s_v[kRows * kPitch], s_m[kRows * kPitch];
   const int lane = threadIdx.x;
   const int64_t row0 = (int64_t)blockIdx.x * kRows;
   const int nrows = (int)((B - row0) < kRows ? (B - row0) : kRows);
   // chunk q = lane + 64 * k of a tile: row q / 32, columns 4 * (q % 32) .. + 3
-  u32x4 pr[kChunks], pv[kChunks], pm[kChunks][MK == MK_I64 ? 2 : 1];
+  u32x4 pr[kChunks], pv[kChunks], pa[kChunks], pb[kChunks];
   auto issue = [&](int64_t c0) {
 #pragma unroll
     for (int k = 0; k < kChunks; ++k) {
       const int q = lane + kWave * k, rr = q / (kCols / 4);
       const int64_t col = c0 + 4 * (q % (kCols / 4));
-      pr[k] = pv[k] = pm[k][0] = pm[k][MK == MK_I64 ? 1 : 0] = u32x4{0u, 0u, 0u, 0u};  // slots past the edges
+      pr[k] = pv[k] = pa[k] = pb[k] = u32x4{0u, 0u, 0u, 0u};  // slots past the edges
       if (rr < nrows && col < L) {
         const int64_t idx = (row0 + rr) * L + col;
         pr[k] = *reinterpret_cast<const u32x4*>(rewards + idx);
         pv[k] = *reinterpret_cast<const u32x4*>(values + idx);
-        if (MK == MK_I64) {
-          pm[k][0] = reinterpret_cast<const u32x4*>((const int64_t*)mask + idx)[0];
-          pm[k][MK == MK_I64 ? 1 : 0] = reinterpret_cast<const u32x4*>((const int64_t*)mask + idx)[1];
-        } else if (MK == MK_B32) {
-          pm[k][0] = *reinterpret_cast<const u32x4*>((const uint32_t*)mask + idx);
-        } else {
-          pm[k][0] = u32x4{*reinterpret_cast<const uint32_t*>((const uint8_t*)mask + idx), 0u, 0u, 0u};
-        }
+        load_mask_pieces<MK>(mask, idx, pa[k], pb[k]);
       }
     }
   };
@@ -121,109 +334,40 @@ __global__ __launch_bounds__(kWave) void gae_scan_vec_kernel(const float* __rest
       const int q = lane + kWave * k, rr = q / (kCols / 4), o = rr * kPitch + 4 * (q % (kCols / 4));
       *reinterpret_cast<u32x4*>(s_r + o) = pr[k];
       *reinterpret_cast<u32x4*>(s_v + o) = pv[k];
-      float4 m;
-      if (MK == MK_I64) {
-        const u32x4 a = pm[k][0], b = pm[k][MK == MK_I64 ? 1 : 0];
-        // values that fit 32 bits (every mask in practice) convert with one instruction each
-        const bool wide = ((int32_t)a.y != ((int32_t)a.x >> 31)) | ((int32_t)a.w != ((int32_t)a.z >> 31)) |
-                          ((int32_t)b.y != ((int32_t)b.x >> 31)) | ((int32_t)b.w != ((int32_t)b.z >> 31));
-        if (__builtin_amdgcn_ballot_w64(wide) == 0) {
-          m = make_float4((float)(int32_t)a.x, (float)(int32_t)a.z, (float)(int32_t)b.x, (float)(int32_t)b.z);
-        } else {
-          m.x = (float)(int64_t)(((uint64_t)a.y << 32) | a.x);
-          m.y = (float)(int64_t)(((uint64_t)a.w << 32) | a.z);
-          m.z = (float)(int64_t)(((uint64_t)b.y << 32) | b.x);
-          m.w = (float)(int64_t)(((uint64_t)b.w << 32) | b.z);
-        }
-      } else if (MK == MK_B32) {
-        const u32x4 a = pm[k][0];
-        if (F32MASK) m = make_float4(u2f(a.x), u2f(a.y), u2f(a.z), u2f(a.w));
-        else m = make_float4((float)(int32_t)a.x, (float)(int32_t)a.y, (float)(int32_t)a.z, (float)(int32_t)a.w);
-      } else {
-        const uint32_t u = pm[k][0].x;
-        m = make_float4((float)(u & 0xffu), (float)((u >> 8) & 0xffu), (float)((u >> 16) & 0xffu), (float)(u >> 24));
-      }
-      *reinterpret_cast<float4*>(s_m + o) = m;
+      *reinterpret_cast<float4*>(s_m + o) = mask_quad<MK, F32MASK>(pa[k], pb[k]);
     }
   };
-  float nv = 0.f, lg = 0.f;
-  if (MODE == MODE_SCAN && init != nullptr && lane < nrows) {
-    nv = init[2 * (row0 + lane)];
-    lg = init[2 * (row0 + lane) + 1];
-  }
   GaeMap gm{1.f, 0.f, 1.f, 0.f, 0.f};
-  double st[kNStat] = {0.0, 0.0, 0.0};  // whitening statistics of this wave's advantages (pivot 0)
   const int64_t c_last = (L - 1) / kCols * kCols;
   issue(c_last);
   for (int64_t c0 = c_last; c0 >= 0; c0 -= kCols) {
     const int ncols = (int)((L - c0) < kCols ? (L - c0) : kCols);  // a multiple of 4
     commit();  // waits for this tile's loads
-    if (c0 > 0) issue(c0 - kCols);  // in flight while this tile is scanned
+    if (c0 > 0) issue(c0 - kCols);  // in flight while this tile is folded
     __syncthreads();
     if (lane < nrows) {
       const float* r4 = s_r + lane * kPitch;
       const float* v4 = s_v + lane * kPitch;
       const float* m4 = s_m + lane * kPitch;
-      // the LDS reads of the next four tokens are issued before the current four are walked
+      // the LDS reads of the next four tokens are issued before the current four are folded
       float4 r = *reinterpret_cast<const float4*>(r4 + ncols - 4), v = *reinterpret_cast<const float4*>(v4 + ncols - 4),
              m = *reinterpret_cast<const float4*>(m4 + ncols - 4);
       for (int cc = ncols - 4; cc >= 0; cc -= 4) {
         const int nx = cc >= 4 ? cc - 4 : 0;
         const float4 rn = *reinterpret_cast<const float4*>(r4 + nx), vn = *reinterpret_cast<const float4*>(v4 + nx),
                      mn = *reinterpret_cast<const float4*>(m4 + nx);
-        if (MODE == MODE_SCAN) {
-          float4 a;
-          gae_step(r.w, v.w, m.w, gamma, gamma_lam, nv, lg); a.w = lg;
-          gae_step(r.z, v.z, m.z, gamma, gamma_lam, nv, lg); a.z = lg;
-          gae_step(r.y, v.y, m.y, gamma, gamma_lam, nv, lg); a.y = lg;
-          gae_step(r.x, v.x, m.x, gamma, gamma_lam, nv, lg); a.x = lg;
-          *reinterpret_cast<float4*>(s_a + lane * kPitch + cc) = a;
-        } else {
-          gae_compose(r.w, v.w, m.w, gamma, gamma_lam, gm);
-          gae_compose(r.z, v.z, m.z, gamma, gamma_lam, gm);
-          gae_compose(r.y, v.y, m.y, gamma, gamma_lam, gm);
-          gae_compose(r.x, v.x, m.x, gamma, gamma_lam, gm);
-        }
+        gae_compose(r.w, v.w, m.w, gamma, gamma_lam, gm);
+        gae_compose(r.z, v.z, m.z, gamma, gamma_lam, gm);
+        gae_compose(r.y, v.y, m.y, gamma, gamma_lam, gm);
+        gae_compose(r.x, v.x, m.x, gamma, gamma_lam, gm);
         r = rn; v = vn; m = mn;
       }
     }
-    __syncthreads();
-    if (MODE == MODE_SCAN) {
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      const int q = lane + kWave * k, rr = q / (kCols / 4), ch = q % (kCols / 4);
-      const int64_t col = c0 + 4 * ch;
-      if (rr < nrows && col < L) {
-        const int64_t idx = (row0 + rr) * L + col;
-        const float4 a = *reinterpret_cast<const float4*>(s_a + rr * kPitch + 4 * ch);
-        const float4 v = *reinterpret_cast<const float4*>(s_v + rr * kPitch + 4 * ch);
-        *reinterpret_cast<float4*>(adv + idx) = a;
-        *reinterpret_cast<float4*>(ret + idx) = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
-        if (part) {
-          const float4 m = *reinterpret_cast<const float4*>(s_m + rr * kPitch + 4 * ch);
-          stat_add(st, a.x, m.x, 0.0);
-          stat_add(st, a.y, m.y, 0.0);
-          stat_add(st, a.z, m.z, 0.0);
-          stat_add(st, a.w, m.w, 0.0);
-        }
-      }
-    }
-    }
-    __syncthreads();  // the next commit overwrites s_v / s_a
+    __syncthreads();  // the next commit overwrites the tile
   }
-  if (MODE == MODE_COMPOSE) {
-    if (lane < nrows) {
-      float* o = maps + 5 * (row0 + lane);
-      o[0] = gm.a00; o[1] = gm.a10; o[2] = gm.a11; o[3] = gm.b0; o[4] = gm.b1;
-    }
-    return;
-  }
-  if (part) {
-#pragma unroll
-    for (int k = 0; k < kNStat; ++k) {
-      const double t = wave_sum(st[k]);
-      if (lane == 0) part[kNStat * blockIdx.x + k] = t;
-    }
+  if (lane < nrows) {
+    float* o = maps + 5 * (row0 + lane);
+    o[0] = gm.a00; o[1] = gm.a10; o[2] = gm.a11; o[3] = gm.b0; o[4] = gm.b1;
   }
 }
 
@@ -247,11 +391,11 @@ __global__ __launch_bounds__(256) void gae_carry_kernel(const float* __restrict_
 
 // Scalar variant for rows that are not 16-byte aligned, lengths that are not a multiple of 4, or other mask
 // dtypes: same tiling, element-wise loads and stores, no prefetch.
-__global__ __launch_bounds__(kWave) void gae_scan_kernel(const float* __restrict__ rewards,
-                                                         const float* __restrict__ values, const void* mask,
-                                                         int mask_dtype, int64_t B, int64_t L, float gamma,
-                                                         float gamma_lam, float* __restrict__ adv,
-                                                         float* __restrict__ ret) {
+__global__ __launch_bounds__(kWave) void gae_scan_any_kernel(const float* __restrict__ rewards,
+                                                             const float* __restrict__ values, const void* mask,
+                                                             int mask_dtype, int64_t B, int64_t L, float gamma,
+                                                             float gamma_lam, float* __restrict__ adv,
+                                                             float* __restrict__ ret) {
   __shared__ float s_r[kRows * kPitch], s_v[kRows * kPitch], s_m[kRows * kPitch], s_a[kRows * kPitch];
   const int lane = threadIdx.x;
   const int64_t row0 = (int64_t)blockIdx.x * kRows;
@@ -287,7 +431,8 @@ __global__ __launch_bounds__(kWave) void gae_scan_kernel(const float* __restrict
 // ---------------------------------------------------------------------------- masked whitening
 
 constexpr int kThreads = 256;
-constexpr int kMaxParts = 8192;
+constexpr int kMaxParts = 8192;      // workgroups of whiten_stats_kernel
+constexpr int kWhitenSlots = 32768;  // partials that the workspace holds: the scan's workgroups of 131072 rows
 __global__ __launch_bounds__(kThreads) void whiten_stats_kernel(const float* __restrict__ v, const void* mask,
                                                                 int mask_dtype, int64_t n, int vec,
                                                                 double* __restrict__ part) {
@@ -360,7 +505,7 @@ int check_mask(int dt) {
   return SIIRL_OK;
 }
 
-constexpr size_t kWhitenWs = (size_t)kMaxParts * kNStat * sizeof(double);
+constexpr size_t kWhitenWs = (size_t)kWhitenSlots * kNStat * sizeof(double);
 
 int check_whiten_ws(const void* ws, size_t ws_bytes) {
   if (ws == nullptr || ws_bytes < kWhitenWs)
@@ -430,25 +575,24 @@ template <int MK, bool F32MASK>
 static int launch_gae_vec(const float* rewards, const float* values, const void* mask, int64_t B, int64_t L, float g,
                           float gl, float* adv, float* ret, void* ws, int chunks, int* parts_ready, hipStream_t st) {
   const int64_t rows = B * chunks, len = L / chunks;
-  const dim3 grid((unsigned)((rows + kRows - 1) / kRows)), block(kWave);
+  const dim3 grid((unsigned)((rows + kScanRows - 1) / kScanRows));
   // the scan leaves its whitening statistics in the workspace, one partial per workgroup, when they fit
-  const bool fused_stats = grid.x <= (unsigned)kMaxParts;
+  const bool fused_stats = grid.x <= (unsigned)kWhitenSlots;
   double* part = fused_stats ? (double*)ws : nullptr;
   *parts_ready = fused_stats ? (int)grid.x : 0;
   const float* init = nullptr;
   if (chunks > 1) {
     float* maps = reinterpret_cast<float*>((char*)ws + kWhitenWs);
     float* ini = maps + (size_t)rows * 5;
-    gae_scan_vec_kernel<MK, F32MASK, MODE_COMPOSE><<<grid, block, 0, st>>>(rewards, values, mask, rows, len, g, gl, nullptr,
-                                                                        nullptr, nullptr, nullptr, maps);
-    SIIRL_LAUNCH_CHECK("gae_scan_vec_kernel<compose>");
+    gae_compose_kernel<MK, F32MASK><<<dim3((unsigned)((rows + kRows - 1) / kRows)), dim3(kWave), 0, st>>>(
+        rewards, values, mask, rows, len, g, gl, maps);
+    SIIRL_LAUNCH_CHECK("gae_compose_kernel");
     gae_carry_kernel<<<dim3((unsigned)((B + 255) / 256)), dim3(256), 0, st>>>(maps, B, chunks, ini);
     SIIRL_LAUNCH_CHECK("gae_carry_kernel");
     init = ini;
   }
-  gae_scan_vec_kernel<MK, F32MASK, MODE_SCAN><<<grid, block, 0, st>>>(rewards, values, mask, rows, len, g, gl, adv, ret,
-                                                                   part, init, nullptr);
-  SIIRL_LAUNCH_CHECK("gae_scan_vec_kernel");
+  gae_scan_kernel<MK, F32MASK><<<grid, dim3(kScanThreads), 0, st>>>(rewards, values, mask, rows, len, g, gl, adv, ret, part, init);
+  SIIRL_LAUNCH_CHECK("gae_scan_kernel");
   return SIIRL_OK;
 }
 
@@ -485,9 +629,9 @@ extern "C" int siirl_gae_advantage_return(const float* token_level_rewards, cons
     rc = launch_gae_vec<MK_U8, false>(token_level_rewards, values, mask, B, L, g, gl, advantages, returns, workspace, chunks,
                                       &parts_ready, st);
   else {  // the scalar kernel walks whole rows in the reference's order, whatever `order` asks for
-    gae_scan_kernel<<<dim3((unsigned)((B + kRows - 1) / kRows)), dim3(kWave), 0, st>>>(
+    gae_scan_any_kernel<<<dim3((unsigned)((B + kRows - 1) / kRows)), dim3(kWave), 0, st>>>(
         token_level_rewards, values, mask, mask_dtype, B, L, g, gl, advantages, returns);
-    SIIRL_LAUNCH_CHECK("gae_scan_kernel");
+    SIIRL_LAUNCH_CHECK("gae_scan_any_kernel");
   }
   if (rc) return rc;
   return run_whiten(advantages, mask, mask_dtype, B * L, 1, advantages, stats3, workspace, parts_ready, st);

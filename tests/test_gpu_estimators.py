@@ -78,6 +78,42 @@ def test_gae(dev, B, L, kind, mdt, gamma, lam):
     assert (adv.cpu() - adv32).abs().max() < 1e-3
 
 
+@pytest.mark.parametrize("case", ["holes", "empty-rows", "fractional-late", "nan-padding", "inf-reward", "overflow",
+                                  "huge-value", "growing"])
+@pytest.mark.parametrize("B,L", [(1, 4), (3, 128), (5, 132), (4, 260), (9, 1156)])
+def test_gae_scan_paths(dev, B, L, case):
+    """The two-operation chain (0/1 masks, moderate numbers) and the recurrence as it stands, from the tile on that
+    needs it: the returns equal the oracle's, NaN where it has NaN."""
+    import siirl_amd.core_algos as CA
+
+    g = torch.Generator().manual_seed(B * 10000 + L)
+    r, v = torch.randn(B, L, generator=g), torch.randn(B, L, generator=g)
+    m = (torch.rand(B, L, generator=g) < 0.7).float()
+    m[:, 0], m[:, -1] = 1.0, 1.0
+    gamma, lam = 0.99, 0.95
+    b, at = B // 2, L // 3
+    if case == "empty-rows":
+        m[1:] = 0.0
+    elif case == "fractional-late":
+        m[b, at] = 0.5
+    elif case == "nan-padding":
+        m[b, at], v[b, at] = 0.0, float("nan")
+    elif case == "inf-reward":
+        r[b, at] = float("inf")
+    elif case == "overflow":  # A leaves the finite numbers although every delta is below 1e30
+        r[b], gamma, lam = 9e29, 1.0, 1.0
+    elif case == "huge-value":
+        v[b, at] = 3e38
+    elif case == "growing":
+        gamma, lam = 1.05, 1.0
+    adv, ret = CA.compute_gae_advantage_return(r.to(dev), v.to(dev), m.to(dev), gamma, lam)
+    _, ret_o = OC.gae_unwhitened(r, v, m, gamma, lam)
+    assert torch.equal(torch.nan_to_num(ret.cpu(), nan=7.0), torch.nan_to_num(ret_o, nan=7.0))
+    if case in ("holes", "empty-rows", "fractional-late"):
+        adv64, _ = OC.compute_gae_advantage_return(r.double(), v.double(), m.double(), gamma, lam)
+        assert (adv.cpu().double() - adv64).abs().max() <= 1e-4  # fp32 scan, then the division by the deviation
+
+
 def test_gae_host_tensors_errors_and_dispatch(dev):
     import siirl_amd.core_algos as CA
 
