@@ -643,7 +643,7 @@ size_t siirl_fused_linear_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, i
 size_t siirl_fused_linear_fwd_workspace_bytes_dtype(int dtype, int64_t T, int64_t H, int64_t V);
 size_t siirl_fused_linear_bwd_workspace_bytes_dtype(int dtype, int64_t T, int64_t H, int64_t V, int want_d_hidden,
                                                     int want_d_weight);
-/* Bytes of the optional saved_logits buffer of the two entry points below: 4 bytes per logit, whole 256 x 256 tiles. */
+/* Bytes of the optional saved_logits buffer of the two entry points below: 4 bytes per logit, whole 128 x 256 tiles. */
 size_t siirl_fused_linear_saved_logits_bytes(int64_t T, int64_t V);
 
 /*

@@ -6,12 +6,12 @@
 // (siirl/utils/kernel/linear_cross_entropy.py:40-117 -> siirl/utils/kernel/kernels.py:507-696,1378-1586); the
 // per-tile online-softmax state (max, sum exp, sum x*exp) is the one of kernels.py:254-266,343-350.
 //
-// One GEMM core, C[M,N] = A[M,K] . B[N,K]^T, 16-bit operands, fp32 accumulation, 256 x 256 x 64 workgroup tile,
-// 8 waves (2 x 4) of 128 x 64 (8 x 4 MFMA 16x16x32 tiles, 128 accumulator registers each).  The 16x16x32 shape moves
+// One GEMM core, C[M,N] = A[M,K] . B[N,K]^T, 16-bit operands, fp32 accumulation, 128 x 256 x 64 workgroup tile,
+// 4 waves of 128 x 64 (8 x 4 MFMA 16x16x32 tiles, 128 accumulator registers each), two workgroups per CU.  The 16x16x32 shape moves
 // half the accumulator data per flop of the 32x32x16 one; with random operand bits the matrix cores then sustain
 // 1.79 instead of 1.62 PFLOP/s in an LDS-fed loop at this part's power limit, which is what sets these kernels' time.
 //   * A (K-major rows) goes global -> LDS by DMA (global_load_lds_dwordx4, no staging registers, no ds_write)
-//     into a ring of four 32 KB stages.  Rows are unpadded; 16-byte chunks are XOR-swizzled by (row / 2) % 8 so
+//     into a ring of four 16 KB stages.  Rows are unpadded; 16-byte chunks are XOR-swizzled by (row / 2) % 8 so
 //     that the ds_read_b128 fragment reads are conflict-free.  A stage is issued three K-steps before it is read
 //     and published (barrier) one step before, so the first fragments of the next step are read ahead of the
 //     barrier and the matrix cores do not drain at it.
@@ -21,8 +21,11 @@
 //     would wait for every outstanding DMA before each LDS read.
 // Four epilogues: softmax partials (forward), dlogits in both layouts (backward), fp32 accumulate (d hidden),
 // bf16 store (d weight).  The backward walks the vocabulary in groups of columns: recompute the group's logits into
-// dlogits[T, group], then dH += dlogits . W_group and dW_group = dlogits^T . hidden as two more runs of the same core
-// against packed transposed copies of W and hidden.
+// dlogits[T, group], then dH += dlogits . W_group and dW_group = dlogits^T . hidden as two more runs of the same core.
+// dlogits are written fragment-packed, once, and serve both: as d hidden's B operand (its A is W as it lies in memory,
+// given by K-rows) and as d weight's A operand (its B a packed transposed copy of hidden).  A transposed copy of W, which
+// d hidden took as its B operand, cost 350 us a call at H=3584, V=152064 whatever the token count, and dlogits row by
+// row, as its A operand, 128 bytes of each of 256 rows per K-step: T=1500, H=2048, V=50257 503 -> 300 us.
 // Optionally the forward also parks the fp32 accumulator tiles in memory (4 bytes per logit, in the accumulator's
 // own lane order, so stores and loads are whole 1 KB wave accesses); the backward then replays the tiles through
 // the same dlogits epilogue instead of recomputing the GEMM: a third of the backward's matrix work is traded for
@@ -38,30 +41,30 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-// Workgroup tile 256 x 256 x 64, 8 waves as 2 (M) x 4 (N), two per SIMD, one workgroup per CU (the LDS ring).
-// (Measured alternatives at T=16384, H=3584, V=152064, with the 32x32x16 MFMA: 128-row tiles with two workgroups per
-// CU 1.5-4 % slower; 4 waves of 128 x 128, one per SIMD, 5-14 % slower.)
-constexpr int BM = 256, BN = 256, BK = 64;
-constexpr int WM = 2, WN = 4;  // wave grid over the workgroup tile
-constexpr int kThreads = WM * WN * 64;
-constexpr int kWavesPerSimd = kThreads / 256;
-constexpr int MI = BM / (WM * 16), NJ = BN / (WN * 16);  // 16x16 MFMA tiles per wave: 8 x 4
-constexpr int KS = BK / 32;                              // K = 32 slices per K-step
+// Workgroup tile 128 x 256 x 64, 4 waves along N, one per SIMD; two workgroups per CU (the LDS rings), which run through
+// their prologues and epilogues at different times.  Against tiles of 256 x 256 with 8 waves and one workgroup per CU, us:
+// forward T=200 345 -> 297, T=3001 (H=2048, fp16) 1710 -> 1660, T=16384 12990 -> 12500; recompute T=200 334 -> 289, a
+// slab at T=16384 717 -> 684; d weight T=200 542 -> 488, T=16384 the same (H=3584, V=152064 bf16 where not said).
+constexpr int BM = 128, BN = 256, BK = 64;
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * 64;
+constexpr int kWavesPerSimd = 2;
+constexpr int MI = BM / 16, NJ = BN / (kWaves * 16);  // 16x16 MFMA tiles per wave: 8 x 4
+constexpr int KS = BK / 32;                           // K = 32 slices per K-step
 static_assert(MI == 8 && NJ == 4 && KS == 2, "the K-step schedule is written for 8 x 4 tiles and two K slices");
-constexpr int kRowBytes = BK * 2;             // unpadded rows, 16-byte chunks XOR-swizzled by (row / 2) % 8
-constexpr int kTileBytes = BM * kRowBytes;    // 32768
-constexpr int kStageBytes = kTileBytes;       // A tile only: B goes global -> registers
+constexpr int kRowBytes = BK * 2;          // unpadded rows, 16-byte chunks XOR-swizzled by (row / 2) % 8
+constexpr int kStageBytes = BM * kRowBytes;  // 16 KB of A: B goes global -> registers
 constexpr int kStages = 4;
-constexpr int kSmemBytes = kStages * kStageBytes;  // 131072
-constexpr int kDmaPerWave = kTileBytes / 1024 / (kThreads / 64);  // 1 KB per wave instruction
+constexpr int kSmemBytes = kStages * kStageBytes;
+constexpr int kDmaPerWave = kStageBytes / 1024 / kWaves;  // 1 KB per wave instruction
 // The backward walks the vocabulary in groups: the group's logits are recomputed into dlogits, then d hidden and
-// d weight are updated from them.  A group is 65536 columns at 16384 tokens and above (256 x 64 tiles of dlogits and
-// 256 x 14 of d weight at H = 3584 fill whole rounds of the 256 CUs; 4 / 8 / 19 times 8192 columns measured 34.4 / 33.7
+// d weight are updated from them.  A group is 65536 columns at 16384 tokens and above (512 x 64 tiles of dlogits and
+// 512 x 14 of d weight at H = 3584 fill whole rounds of the 256 CUs, two workgroups each; 4 / 8 / 19 times 8192 columns measured 34.4 / 33.7
 // / 33.2 ms per backward at T=16384, V=152064), and as many times more with fewer tokens as keep the same bytes of
 // dlogits: at T=200, V=152064 one group instead of three.
 constexpr int64_t kGroupCols = 65536, kGroupTokens = 16384;
-constexpr int kLdPad = 64;                    // extra elements per row of D: keeps a tile's rows off a
-                                              // power-of-two stride, which would put them all in one memory channel
+constexpr int kPadBlocks = 2;  // extra 1 KB blocks per 16 tokens of D: keeps the token blocks of a stage off a power-of-two
+                               // stride, which would put them all in one memory channel
 
 struct GemmArgs {
   const uint16_t* A;
@@ -72,7 +75,14 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   int splits;  // K is cut into `splits` runs of K-steps; run s is tile column tn + s * tiles_n of the raster
   int blk_m;   // tiles along M of an XCD's block of 32 tiles
+  int chunk;   // tile places per XCD, or 0: whole blocks in turn
+  // A_KROWS: a last K-step that A does not fill is read from a copy of its rows, padded with zeros to BK of them
+  const uint16_t* A_tail;
+  int kt_tail;  // its index (the last step), or past it
 };
+// How the A operand lies in memory: [M][K] with K contiguous; [K][M] with M contiguous; or fragment-packed as the B
+// operand of a GEMM whose N is this one's K and whose K is this one's M (16-row blocks along K, 32-wide blocks along M).
+enum { A_ROWS = 0, A_KROWS = 1, A_PACKED = 2 };
 
 struct TileCoord {
   int tm, tn;
@@ -87,72 +97,97 @@ struct TileCoord {
 // operand from memory once rather than once per strip, measured 4 % slower forward and 8-17 % slower backward GEMMs
 // at T=16384, H=3584, V=152064: the L2 reuse inside a strip matters more than the bytes from memory.)
 constexpr int kXcd = 8, kBlkTiles = 32;
-__host__ __device__ inline int64_t raster_grid(int tiles_m, int tiles_n, int blk_m) {
-  const int blk_n = kBlkTiles / blk_m;
-  const int64_t blocks = (int64_t)((tiles_m + blk_m - 1) / blk_m) * ((tiles_n + blk_n - 1) / blk_n);
-  return (blocks + kXcd - 1) / kXcd * kXcd * kBlkTiles;
+// With few blocks that hand-out is uneven (9 or 10 blocks leave one or two XCDs a second round while the others stop): up
+// to kChunkBlocks of them, an XCD takes an eighth of all their tiles instead, consecutive in the same order (`chunk` tile
+// places).  d hidden at T=200, H=3584, V=152064 (28 x 18 tiles): 391 us in blocks of 8 x 4 in turn, 290 us as 32 x 1, chunked.
+constexpr int64_t kChunkBlocks = 64;
+inline int64_t raster_grid(GemmArgs& g) {
+  const int blk_n = kBlkTiles / g.blk_m;
+  const int64_t blocks = (int64_t)((g.tiles_m + g.blk_m - 1) / g.blk_m) * (((int64_t)g.tiles_n * g.splits + blk_n - 1) / blk_n);
+  g.chunk = blocks <= kChunkBlocks ? (int)((blocks * kBlkTiles + kXcd - 1) / kXcd) : 0;
+  return g.chunk ? (int64_t)g.chunk * kXcd : (blocks + kXcd - 1) / kXcd * kXcd * kBlkTiles;
 }
 __device__ __forceinline__ TileCoord tile_of(const GemmArgs& g, int id) {
   const int blk_m = g.blk_m, blk_n = kBlkTiles / blk_m;
   const int xcd = id % kXcd, l = id / kXcd;
-  const int blk = (l / kBlkTiles) * kXcd + xcd, j = l % kBlkTiles;
+  const int at = g.chunk ? xcd * g.chunk + l : ((l / kBlkTiles) * kXcd + xcd) * kBlkTiles + l % kBlkTiles;
+  const int blk = at / kBlkTiles, j = at % kBlkTiles;
   const int mb = (g.tiles_m + blk_m - 1) / blk_m;
   const int tm = (blk % mb) * blk_m + j % blk_m;
   const int tn = (blk / mb) * blk_n + j / blk_m;
   return {tm, tn, tm < g.tiles_m && tn < g.tiles_n * g.splits};
 }
 
-// Accumulator coordinates of lane `lane` in wave (wm, wn): element r (0..3) of acc[i][j] is
-//   row = wm*128 + i*16 + (lane/16)*4 + r ,  col = wn*64 + j*16 + lane%16   (tile-relative)
-__device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) {
-  return wm * (MI * 16) + i * 16 + (lane >> 4) * 4 + r;
+// Accumulator coordinates of lane `lane` in wave wn: element r (0..3) of acc[i][j] is
+//   row = i*16 + (lane/16)*4 + r ,  col = wn*64 + j*16 + lane%16   (tile-relative)
+__device__ __forceinline__ int acc_row(int i, int r, int lane) {
+  return i * 16 + (lane >> 4) * 4 + r;
 }
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * (NJ * 16) + j * 16 + (lane & 15); }
 // An epilogue with kRowsPerLane takes the accumulator the other way round (the MFMA's operands are swapped): a lane owns
 // the rows row_of_lane(i) and, with B packed in the column order of transpose_pack_b_kernel, the 16 consecutive columns
 // from col_of_lane on: element r of acc[i][j] is column col_of_lane + 4 * j + r.
-__device__ __forceinline__ int row_of_lane(int wm, int i, int lane) { return wm * (MI * 16) + i * 16 + (lane & 15); }
+__device__ __forceinline__ int row_of_lane(int i, int lane) { return i * 16 + (lane & 15); }
 __device__ __forceinline__ int col_of_lane(int wn, int lane) { return wn * (NJ * 16) + (lane >> 4) * 16; }
 
 // m0 (the DMA's LDS base) is a reserved register: naming it in a clobber list is right but draws a warning
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 // F16: the 16-bit operands are IEEE half instead of bf16 (the same data movement, the other MFMA)
-template <class Epi, bool AT = false, bool F16 = false>
+template <class Epi, int AL = A_ROWS, bool F16 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_nt_kernel(GemmArgs g, Epi epi) {
   static_assert(!(F16 && Epi::kRowsPerLane), "the gradient GEMMs multiply bf16");
   extern __shared__ __align__(16) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w / WN, wn = w % WN;
-  const TileCoord tc = tile_of(g, blockIdx.x);
+  const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
+  TileCoord tc = tile_of(g, blockIdx.x);
   if (!tc.valid) return;
-  const int split = tc.tn / g.tiles_n;
+  // (integer divisions leave their results in vector registers; these are the same in every lane)
+  tc.tm = __builtin_amdgcn_readfirstlane(tc.tm);
+  tc.tn = __builtin_amdgcn_readfirstlane(tc.tn);
+  const int split = __builtin_amdgcn_readfirstlane(tc.tn / g.tiles_n);
   const int m0 = tc.tm * BM, n0 = (tc.tn - split * g.tiles_n) * BN;
   // this workgroup's run of K-steps (the host keeps every run non-empty)
-  const int kt_per = (g.K / BK + g.splits - 1) / g.splits;
+  const int kt_per = __builtin_amdgcn_readfirstlane((g.K / BK + g.splits - 1) / g.splits);
   const int kt_first = split * kt_per;
   const int KT = (g.K / BK - kt_first < kt_per) ? g.K / BK - kt_first : kt_per;
 
   // A: global -> LDS by DMA (global_load_lds_dwordx4): wave instruction I = w * kDmaPerWave + i fills the 1 KB
   // [I * 1024, I * 1024 + 1024) of the stage.
-  //   A[M][K] (AT = false): 16-byte slot sl = I * 64 + lane holds row sl / 8, chunk (sl % 8) ^ ((row / 2) % 8).  Rows
+  //   A[M][K] (A_ROWS): 16-byte slot sl = I * 64 + lane holds row sl / 8, chunk (sl % 8) ^ ((row / 2) % 8).  Rows
   //     past the matrix edge are clamped to the last row.
-  //   A given as [K][M], M contiguous (AT = true): the stage is 64 K-rows of 512 bytes; slot sl holds K-row sl / 32,
-  //     chunk (sl % 32) ^ 2 * (row % 4), i.e. the 32-byte segments of a row are XOR-swizzled by the row so that the
-  //     four K-rows a transposing fragment read touches lie in different banks.  Columns past M are read as they are
-  //     (the row pitch covers whole tiles) and only reach output rows that the epilogue masks.
-  const int wu = __builtin_amdgcn_readfirstlane(w);
-  const char* gA = AT ? reinterpret_cast<const char*>(g.A + (int64_t)kt_first * BK * g.lda + m0)
-                      : reinterpret_cast<const char*>(g.A + (int64_t)m0 * g.lda + (int64_t)kt_first * BK);
-  const int64_t a_step = AT ? (int64_t)BK * g.lda * 2 : (int64_t)BK * 2;  // bytes from one K-step to the next
+  //   A[K][M] (A_KROWS): the stage is 64 K-rows of BM * 2 bytes; with c = BM / 8 chunks a row, slot sl holds
+  //     K-row sl / c, chunk (sl % c) ^ 2 * (row % 4), i.e. the 32-byte segments of a row are XOR-swizzled by the row so
+  //     that the four K-rows a transposing fragment read touches lie in different banks.  A chunk past M (a multiple of
+  //     64) is read as the tile's first one and only reaches output rows that the epilogue masks.
+  //   A_PACKED: the stage is 4 x BM / 32 packed blocks of 1 KB, one per wave instruction.  Slot 16 q + t of a block
+  //     holds the 8 M-entries from 8 q on of K-row t ^ 4 * (q % 2): the two chunks of a transposing fragment read that
+  //     are 256 bytes apart then lie in different banks.  Blocks past M are inside the buffer (its pitch covers tiles).
+  const int wu = __builtin_amdgcn_readfirstlane(wn);
+  const char* gA;
+  int64_t a_step;  // bytes from one K-step to the next
+  if constexpr (AL == A_ROWS) {
+    gA = reinterpret_cast<const char*>(g.A + (int64_t)m0 * g.lda + (int64_t)kt_first * BK);
+    a_step = (int64_t)BK * 2;
+  } else if constexpr (AL == A_KROWS) {
+    gA = reinterpret_cast<const char*>(g.A + (int64_t)kt_first * BK * g.lda + m0);
+    a_step = (int64_t)BK * g.lda * 2;
+  } else {  // lda: 32-wide blocks from one 16-row block to the next
+    gA = reinterpret_cast<const char*>(g.A) + ((int64_t)kt_first * (BK / 16) * g.lda + (m0 >> 5)) * 1024;
+    a_step = (int64_t)(BK / 16) * g.lda * 1024;
+  }
   uint32_t offA[kDmaPerWave];
 #pragma unroll
   for (int i = 0; i < kDmaPerWave; ++i) {
-    const int sl = (wu * kDmaPerWave + i) * 64 + lane;
-    if constexpr (AT) {
-      const int row = sl >> 5;
-      const int ch = (sl & 31) ^ ((row & 3) << 1);
+    const int I = wu * kDmaPerWave + i, sl = I * 64 + lane;
+    if constexpr (AL == A_KROWS) {
+      constexpr int kRowChunks = BM / 8;
+      const int row = sl / kRowChunks;
+      int ch = (sl % kRowChunks) ^ ((row & 3) << 1);
+      if (m0 + ch * 8 >= g.M) ch = 0;
       offA[i] = (uint32_t)row * (uint32_t)g.lda * 2u + ch * 16;
+    } else if constexpr (AL == A_PACKED) {
+      constexpr int kBlocks = BM / 32;
+      offA[i] = ((uint32_t)(I / kBlocks) * (uint32_t)g.lda + I % kBlocks) * 1024u + (lane ^ ((lane >> 2) & 4)) * 16;
     } else {
       int row = sl >> 3;
       const int ch = (sl & 7) ^ ((row >> 1) & 7);
@@ -178,8 +213,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
   u32x4 b0[NJ][KS], b1[NJ][KS];
+  const int kt_tail = g.kt_tail - kt_first;
+  const int64_t to_tail = reinterpret_cast<const char*>(g.A_tail + m0) - (gA + (int64_t)kt_tail * a_step);  // (kt_tail is the last step)
   auto dma = [&](int stage, int kt, int i0 = 0, int i1 = kDmaPerWave) {
+    // (No branch around the loads, and no register to spare: where the compiler copies or spills the B registers it does
+    // so before their wait.)
     const char* base = gA + (int64_t)kt * a_step;
+    if (AL == A_KROWS) base += to_tail & (int64_t)__builtin_amdgcn_readfirstlane((kt - kt_tail) >> 31 ^ -1);
 #pragma unroll
     for (int i = i0; i < i1; ++i) {
       const uint32_t dst = lds0 + stage * kStageBytes + (wu * kDmaPerWave + i) * 1024;
@@ -213,18 +253,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   __syncthreads();
 
   // A fragments of MFMA group gq = 2 * s + hf: K slice s (32 columns), row blocks hf * 4 .. hf * 4 + 3 of the wave's
-  // eight 16-row blocks.  AT = false: lane (m = lane % 16, 8-column chunk lane / 16 of the slice) reads its 8
-  // consecutive K entries as one 16-byte chunk of row m.  AT = true: the stage holds K-rows, so the 8 entries come
+  // eight 16-row blocks.  A_ROWS: lane (m = lane % 16, 8-column chunk lane / 16 of the slice) reads its 8
+  // consecutive K entries as one 16-byte chunk of row m.  Otherwise the stage holds K-rows, so the 8 entries come
   // from two transposing reads (ds_read_b64_tr_b16): in each block of 16 lanes, lane 4 e + c addresses the 8 bytes of
   // K-row e, M-chunk c, and receives the entries of K-rows 0..3 at M = its own index in the block; block lane / 16
   // takes the 8 K-rows lane / 16 * 8 .. + 7 of the slice.
   const int m15 = lane & 15, kq = lane >> 4, sw = m15 >> 1;
-  const int frag_row = (wm * (MI * 16) + m15) * kRowBytes;
+  const int frag_row = m15 * kRowBytes;
   int xk[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) xk[s] = frag_row + (((s * 4 + kq) ^ sw) << 4);
   const int tq = m15 >> 2;
-  const int xt0 = (kq * 8 + tq) * 512 + wm * 256 + (lane & 3) * 8 + (tq << 5);  // row block ii: xt0 ^ (ii << 5)
+  const int xt0 = (kq * 8 + tq) * (BM * 2) + (lane & 3) * 8 + (tq << 5);  // row block ii: xt0 ^ (ii << 5)
+  // A_PACKED: K-row t = (kq % 2) * 8 + tq of the 16-row block kq / 2 of the slice, the M-chunk's 8 bytes of its 16
+  const int mc = lane & 3;
+  const int xp0 = (kq >> 1) * (BM * 32) + ((kq & 1) * 8 + (mc & 2) * 2 + tq) * 16 + (mc >> 1) * 256 + (mc & 1) * 8;
 
   // step kt: stage kt % 4 is read; B(kt + 1) and DMA(kt + 3) are issued; the barrier at the end publishes stage
   // (kt + 2) % 4, whose DMA was issued one step earlier, and frees stage kt % 4 for DMA(kt + 4).  The last three steps
@@ -235,14 +278,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   auto fread = [&](bf16x8 (&af)[4], int stage, int gq) {
     const char* cur = smem + stage * kStageBytes;
     const int s = gq >> 1, hf = gq & 1;
-    if constexpr (AT) {
+    if constexpr (AL != A_ROWS) {
       typedef short s16x4 __attribute__((ext_vector_type(4)));
       typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) {
-        const char* at = cur + (xt0 ^ (ii << 5)) + s * (32 * 512) + hf * 128;
+        // K-rows 0 .. 3 and 4 .. 7 of the lane's eight
+        const int in_stage = s * (32 * BM * 2) + (AL == A_KROWS ? hf * 128 : (hf * 4 + ii) * 512);
+        const char* at = cur + in_stage + (AL == A_KROWS ? xt0 ^ (ii << 5) : xp0);
+        const char* at4 = AL == A_KROWS ? at + 4 * BM * 2 : cur + in_stage + (xp0 ^ 64);
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * 512));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at4));
         af[ii] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
     } else {
@@ -336,7 +382,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   // the LDS
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  epi(acc, m0, n0, tc.tm, split, wm, wn, lane, tid, smem);
+  int em0 = m0, en0 = n0, el = lane;
+  asm volatile("" : "+s"(em0), "+s"(en0), "+v"(el));  // (no address of the epilogue is computed before the main loop)
+  epi(acc, em0, en0, tc.tm, split, wn, el, tid, smem);
 }
 #pragma clang diagnostic pop
 
@@ -358,8 +406,7 @@ template <class Epi>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void replay_tiles_kernel(
     const float* __restrict__ saved, int tiles_n, int tm_first, Epi epi) {
   extern __shared__ __align__(16) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w / WN, wn = w % WN;
+  const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
   const int tml = blockIdx.x / tiles_n, tn = blockIdx.x - tml * tiles_n;
   const f32x4* src = saved_tile(const_cast<float*>(saved), tm_first + tml, tn, tiles_n) + tid;
   floatx4 acc[MI][NJ];
@@ -367,7 +414,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_nontemporal_load(src + (i * NJ + j) * kThreads);
-  epi(acc, tml * BM, tn * BN, tml, 0, wm, wn, lane, tid, smem);
+  epi(acc, tml * BM, tn * BN, tml, 0, wn, lane, tid, smem);
 }
 
 // ------------------------------------------------------------------------------ epilogue: softmax partials
@@ -375,9 +422,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 // The two fused GEMMs run "transposed": M is the vocabulary (A = W), N the tokens (B = hidden).  In the MFMA
 // accumulator layout a lane then owns one token (column) and its registers run over vocabulary rows, so the
 // softmax reductions over the vocabulary are in-register, followed by two exchanges between the four lanes that
-// share a token and a merge of the WM waves through LDS -- no 16-lane butterfly per row.
+// share a token -- no 16-lane butterfly per row.
 //
-// Per token of the tile: mx = max_v z, s = sum exp(z - mx), t = sum z * exp(z - mx) over the tile's 256
+// Per token of the tile: mx = max_v z, s = sum exp(z - mx), t = sum z * exp(z - mx) over the tile's 128
 // vocabulary rows, z = acc * inv_T; one (mx, s, t) per token is written to part[tm][.][token].
 struct SoftmaxPartialsEpi {
   static constexpr bool kRowsPerLane = false;
@@ -386,11 +433,11 @@ struct SoftmaxPartialsEpi {
   float* part;  // [tiles_m][3][T]
   float* save;  // null, or the parked accumulator tiles (see saved_tile)
   int tiles_n;
-  // The wave's (mx, s, t) of each of its tokens, to sh[wm][token].  Works on the raw accumulator a (z = a * inv_T):
+  // The (mx, s, t) of each of the wave's tokens.  Works on the raw accumulator a (z = a * inv_T):
   // a maximum, one fused multiply-add, one exp2 and two accumulations per logit; no matrix work runs beside this, so
   // its length counts in full (FULL: no vocabulary row of the tile is past the end, nothing is compared or selected).
   template <bool FULL>
-  __device__ __forceinline__ void reduce(floatx4 (&acc)[MI][NJ], int m0, int wm, int wn, int lane, float* sh) const {
+  __device__ __forceinline__ void reduce(floatx4 (&acc)[MI][NJ], int m0, int n0, int wn, int lane, float* o) const {
     const float ninf = -__builtin_inff();
     const float ek = inv_T * kLog2e;
 #pragma unroll
@@ -400,7 +447,7 @@ struct SoftmaxPartialsEpi {
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (FULL || m0 + acc_row(wm, i, r, lane) < V) mx = fmaxf(mx, acc[i][j][r]);
+          if (FULL || m0 + acc_row(i, r, lane) < V) mx = fmaxf(mx, acc[i][j][r]);
       mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
       mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
       float s = 0.f, t = 0.f;
@@ -410,7 +457,7 @@ struct SoftmaxPartialsEpi {
         for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            if (!FULL && m0 + acc_row(wm, i, r, lane) >= V) continue;
+            if (!FULL && m0 + acc_row(i, r, lane) >= V) continue;
             const float e = fast_exp2(fmaf(acc[i][j][r], ek, nmk));
             s += e;
             t = fmaf(acc[i][j][r], e, t);
@@ -420,17 +467,17 @@ struct SoftmaxPartialsEpi {
       t += __shfl_xor(t, 16, kWave);
       s += __shfl_xor(s, 32, kWave);
       t += __shfl_xor(t, 32, kWave);
-      if (lane < 16) {
-        float* d = sh + (wm * BN + acc_col(wn, j, lane)) * 3;
-        d[0] = mx * inv_T;
-        d[1] = s;
-        d[2] = t * inv_T;
+      const int tok = n0 + acc_col(wn, j, lane);
+      if (lane < 16 && tok < T) {
+        o[tok] = mx * inv_T;
+        o[(int64_t)T + tok] = s;
+        o[2 * (int64_t)T + tok] = t * inv_T;
       }
     }
   }
-  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn,
-                                             int lane, int tid, char* smem) const {
-    // Parking costs about 11 us per tile (256 KB per workgroup): the workgroup's own drain, not a burst of the round.
+  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wn, int lane,
+                                             int tid, char* smem) const {
+    // Parking costs about 11 us per 256 KB: the workgroup's own drain, not a burst of the round.
     if (save) {
       f32x4* dst = saved_tile(save, tm, n0 / BN, tiles_n) + tid;
 #pragma unroll
@@ -438,66 +485,56 @@ struct SoftmaxPartialsEpi {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) dst[(i * NJ + j) * kThreads] = acc[i][j];
     }
-    float* sh = reinterpret_cast<float*>(smem);  // [WM][BN][3]; the main loop's last barrier freed the LDS
-    const float k = kLog2e;
-    const float ninf = -__builtin_inff();
+    float* o = part + (int64_t)tm * 3 * T;
     if (m0 + BM <= V)
-      reduce<true>(acc, m0, wm, wn, lane, sh);
+      reduce<true>(acc, m0, n0, wn, lane, o);
     else
-      reduce<false>(acc, m0, wm, wn, lane, sh);
-    __syncthreads();
-    const int tok = n0 + tid;
-    if (tid < BN && tok < T) {
-      float M = ninf;
-#pragma unroll
-      for (int q = 0; q < WM; ++q) M = fmaxf(M, sh[(q * BN + tid) * 3]);
-      float ss = 0.f, tt = 0.f;
-#pragma unroll
-      for (int q = 0; q < WM; ++q) {
-        const float* a = sh + (q * BN + tid) * 3;
-        const float f = a[0] > ninf ? fast_exp2((a[0] - M) * k) : 0.f;
-        ss += a[1] * f;
-        tt += a[2] * f;
-      }
-      float* o = part + (int64_t)tm * 3 * T;
-      o[tok] = M;
-      o[(int64_t)T + tok] = ss;
-      o[2 * (int64_t)T + tok] = tt;
-    }
+      reduce<false>(acc, m0, n0, wn, lane, o);
   }
 };
 
 // ------------------------------------------------------------------------------ epilogue: dlogits
 
 // d raw_logit = inv_T * ( g_lp * (1[v == y] - p) - g_h * p * (z - ex) ),  p = exp(z - lse), z = acc * inv_T,
-// written as bf16 to D[token][v] (ld = ldd); v is group-relative and is the M dimension of this GEMM.  Rows v in
-// [Vs, Vpad) are written as zeros: they are K-padding of the d-hidden GEMM that consumes D.  A lane owns one token,
-// so the per-token coefficients are loaded once per lane and D gets 8-byte stores.  This one token-major layout
-// serves both consumers: d hidden reads it as its A[M = token][K = vocabulary], d weight as A given by K-rows.
+// written as bf16, fragment-packed like a B operand B[n = token][k = v]: block (token / 16, v / 32) is the 1 KB
+// D + ((token / 16) * kb_total + v / 32) * 1 KB.  v is group-relative and is the M dimension of this GEMM.  Rows v in
+// [Vs, Vpad) are written as zeros: they are K-padding of the d-hidden GEMM that consumes D; so are the tokens in
+// [T, Tpad) for d weight.  A lane owns one token, so the per-token coefficients are loaded once per lane, and a wave
+// writes D in runs of 512 bytes.  The one layout serves both consumers: d hidden takes it as its B operand, d weight
+// as an A operand given by packed K-rows.
 struct DlogitsEpi {
   static constexpr bool kRowsPerLane = false;
   float inv_T;
-  int T, Vs, Vpad;
+  int T, Tpad, Vs, Vpad;
   int64_t v0;  // first vocabulary column of the group
   const float* lse;
   const float* ex;
   const float* g_lp;  // may be null
   const float* g_h;   // may be null
   const int64_t* labels;
-  uint16_t* D;
-  int64_t ldd;
+  char* D;
+  int64_t kb_total;
   // One lane's part of the tile.  With a = raw accumulator (z = a * inv_T) the gradient is
   //   d = p * (c0 + c1 * a) + [v == y] * cy,   p = exp2(a * ek + nl),
   // ek = inv_T * log2(e), nl = -lse * log2(e), c1 = -g_h * inv_T^2, c0 = inv_T * (g_h * ex - g_lp), cy = g_lp * inv_T:
   // two fused multiply-adds, one exp2 and one multiply per logit.  FULL: every vocabulary row of the tile is inside
   // the group.
   template <bool FULL>
-  __device__ __forceinline__ void tile(floatx4 (&acc)[MI][NJ], int m0, int n0, int wm, int wn, int lane) const {
+  __device__ __forceinline__ void tile(floatx4 (&acc)[MI][NJ], int m0, int n0, int wn, int lane) const {
     const float ek = inv_T * kLog2e;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int tok = n0 + acc_col(wn, j, lane);
-      if (tok >= T) continue;
+      if (tok >= Tpad) continue;
+      // chunk (token % 16) + 16 * (v % 32 / 8) of the block; the lane's four rows are half a chunk
+      char* dblk = D + ((int64_t)(tok >> 4) * kb_total + (m0 >> 5)) * 1024 + (lane & 15) * 16 +
+                   (lane >> 5) * 256 + ((lane >> 4) & 1) * 8;
+      if (tok >= T) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          if (FULL || m0 + acc_row(i, 0, lane) < Vpad) *reinterpret_cast<uint2*>(dblk + i * 512) = make_uint2(0u, 0u);
+        continue;
+      }
       const float g1 = g_lp ? g_lp[tok] : 0.f;
       const float g2 = g_h ? g_h[tok] : 0.f;
       const float nl = -lse[tok] * kLog2e;
@@ -508,10 +545,9 @@ struct DlogitsEpi {
         const int64_t yl = labels[tok] - v0;
         if (yl >= 0 && yl < Vs) y = (int)yl;
       }
-      uint16_t* drow = D + (int64_t)tok * ldd;
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        const int v = m0 + acc_row(wm, i, 0, lane);  // 4 consecutive vocabulary rows of the group
+        const int v = m0 + acc_row(i, 0, lane);  // 4 consecutive vocabulary rows of the group
         float d[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -521,43 +557,43 @@ struct DlogitsEpi {
           if (v + e == y) g += cy;
           d[e] = (FULL || v + e < Vs) ? g : 0.f;
         }
-        // the four lanes that share the token hold 16 consecutive rows: 32 contiguous bytes per token and store
-        if (FULL || v < Vpad) *reinterpret_cast<uint2*>(drow + v) = make_uint2(pack_bf16(d[0], d[1]), pack_bf16(d[2], d[3]));
+        if (FULL || v < Vpad)
+          *reinterpret_cast<uint2*>(dblk + i * 512) = make_uint2(pack_bf16(d[0], d[1]), pack_bf16(d[2], d[3]));
       }
     }
   }
-  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn,
+  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wn,
                                              int lane, int tid, char* smem) const {
     if (m0 + BM <= Vs)
-      tile<true>(acc, m0, n0, wm, wn, lane);
+      tile<true>(acc, m0, n0, wn, lane);
     else
-      tile<false>(acc, m0, n0, wm, wn, lane);
+      tile<false>(acc, m0, n0, wn, lane);
   }
 };
 
 // ------------------------------------------------------------------------------ epilogues: plain stores
 
-// Both take the accumulator by rows: a lane holds 16 consecutive columns of a row, 32 (16-bit) or 64 bytes, and the four
-// lanes of a row a whole 128-byte line or two.  With a column per lane each store instruction wrote 2-byte (d weight) or
-// 4-byte pieces, 128 per lane and tile instead of 16 or 32.  N is a multiple of 64, so a wave's columns are all inside
-// the matrix or all outside.
-
-struct AccumF32Epi {  // C_s[row][col] = (beta ? C_s : 0) + acc, one fp32 buffer C_s = C + s * split_stride per K run
-  static constexpr bool kRowsPerLane = true;
+// d hidden: C_s[token][h] = (beta ? C_s : 0) + acc, one fp32 buffer C_s = C + s * split_stride per K run.  M is the hidden
+// index, N the token: the four lanes of a token hold 16 consecutive columns of its row.
+struct AccumF32Epi {
+  static constexpr bool kRowsPerLane = false;
   float* C;
   int64_t ldc, split_stride;
   int M, N, beta;
-  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn, int lane, int tid,
+  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wn, int lane, int tid,
                              char* smem) const {
-    const int col = n0 + col_of_lane(wn, lane);
-    if (col >= N) return;
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int row = m0 + row_of_lane(wm, i, lane);
-      if (row >= M) continue;
-      f32x4* p = reinterpret_cast<f32x4*>(C + split * split_stride + (int64_t)row * ldc + col);
+    for (int j = 0; j < NJ; ++j) {
+      const int tok = n0 + acc_col(wn, j, lane);
+      if (tok >= N) continue;
+      float* p = C + split * split_stride + (int64_t)tok * ldc;
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) p[j] = beta ? p[j] + acc[i][j] : acc[i][j];
+      for (int i = 0; i < MI; ++i) {
+        const int h = m0 + acc_row(i, 0, lane);
+        if (h >= M) continue;
+        f32x4* q = reinterpret_cast<f32x4*>(p + h);
+        *q = beta ? *q + acc[i][j] : acc[i][j];
+      }
     }
   }
 };
@@ -576,19 +612,23 @@ __device__ __forceinline__ uint2 pack4(floatx4 v, int out_dtype) {
                                  : make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
 }
 
-struct StoreEpi {  // C[row][col] = acc, rounded to the output type (out_dtype: SIIRL_BF16, SIIRL_F16 or SIIRL_F32)
+// C[row][col] = acc, rounded to the output type (out_dtype: SIIRL_BF16, SIIRL_F16 or SIIRL_F32).  Takes the accumulator
+// by rows: a lane holds 16 consecutive columns of a row, 32 (16-bit) or 64 bytes, and the four lanes of a row a whole
+// 128-byte line or two.  With a column per lane each store instruction wrote 2-byte pieces, 128 per lane and tile instead
+// of 16 or 32.  N is a multiple of 64, so a wave's columns are all inside the matrix or all outside.
+struct StoreEpi {
   static constexpr bool kRowsPerLane = true;
   void* C;
   int64_t ldc;
   int M, N, out_dtype;
-  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wm, int wn, int lane, int tid,
+  __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wn, int lane, int tid,
                              char* smem) const {
     const int col = n0 + col_of_lane(wn, lane);
     if (col >= N) return;
     const bool aligned = ((uintptr_t)C & 15) == 0;  // (a caller's buffer need not be; ldc and col are multiples of 16)
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-      const int row = m0 + row_of_lane(wm, i, lane);
+      const int row = m0 + row_of_lane(i, lane);
       if (row >= M) continue;
       const int64_t at = (int64_t)row * ldc + col;
       if (!aligned) {
@@ -672,6 +712,21 @@ __global__ __launch_bounds__(256) void transpose_pack_b_kernel(const uint16_t* _
   }
 }
 
+// out = in rounded from IEEE half to bf16; eight elements per thread and pass
+__global__ __launch_bounds__(256) void f16_to_bf16_kernel(const u32x4* __restrict__ in, u32x4* __restrict__ out, int64_t n8) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (int64_t)gridDim.x * 256) {
+    const u32x4 v = __builtin_nontemporal_load(in + i);
+    out[i] = u32x4{half2_to_bf16x2(v.x), half2_to_bf16x2(v.y), half2_to_bf16x2(v.z), half2_to_bf16x2(v.w)};
+  }
+}
+
+// 16-byte pieces: the first `have` of them copied, the others zero
+__global__ __launch_bounds__(256) void copy_padded_kernel(const u32x4* __restrict__ in, int64_t have, u32x4* __restrict__ out,
+                                                          int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = i < have ? in[i] : u32x4{0u, 0u, 0u, 0u};
+}
+
 // label_logit[row] = inv_T * <hidden[row], W[labels[row]]>, one wave per row (NaN for a label outside [0, V))
 __global__ __launch_bounds__(256) void label_logit_kernel(const uint16_t* __restrict__ hidden,
                                                           const uint16_t* __restrict__ W,
@@ -704,25 +759,47 @@ __global__ __launch_bounds__(256) void label_logit_kernel(const uint16_t* __rest
 
 // folds the per-tile partials of each token: lse, ex, entropy, logprob.  A workgroup handles kMergeTok tokens;
 // kMergeGrp thread groups each merge every kMergeGrp-th tile online, then the states are merged through LDS.
-constexpr int kMergeTok = 16, kMergeGrp = 16;
-static_assert(kMergeTok * kMergeGrp == 256, "one thread per (token, group)");
-__global__ __launch_bounds__(256) void merge_partials_kernel(const float* __restrict__ part, int nparts, int T,
-                                                             const float* __restrict__ label_logit,
-                                                             float* __restrict__ logprob, float* __restrict__ entropy,
-                                                             float* __restrict__ lse_out, float* __restrict__ ex_out) {
+// Bound by the latency of its loads at few tokens (13 workgroups at T=200) and by the read of the partials at many: 64
+// groups, whose loads do not depend on each other, four tiles at a time.  1188 tiles: T=200 68 -> 13 us, T=16384
+// 95 -> 78 us against 16 groups that waited for a tile's maximum before they read its sums.
+constexpr int kMergeTok = 16, kMergeGrp = 64, kMergeThreads = kMergeTok * kMergeGrp, kMergeFold = 8, kMergeAhead = 4;
+__global__ __launch_bounds__(kMergeThreads) void merge_partials_kernel(const float* __restrict__ part, int nparts, int T,
+                                                                       const float* __restrict__ label_logit,
+                                                                       float* __restrict__ logprob,
+                                                                       float* __restrict__ entropy,
+                                                                       float* __restrict__ lse_out,
+                                                                       float* __restrict__ ex_out) {
   __shared__ float sh[kMergeGrp][kMergeTok][3];
+  __shared__ double shd[kMergeFold][kMergeTok][2];
+  const float ninf = -__builtin_inff();
   const int tl = threadIdx.x % kMergeTok, grp = threadIdx.x / kMergeTok;
   const int row = blockIdx.x * kMergeTok + tl;
-  float M = -__builtin_inff(), s = 0.f, t = 0.f;
+  float M = ninf, s = 0.f, t = 0.f;
   if (row < T) {
-    for (int p = grp; p < nparts; p += kMergeGrp) {
-      const float* q = part + (int64_t)p * 3 * T;
-      const float m = q[row];
-      if (m > -__builtin_inff()) {
-        const float Mn = fmaxf(M, m);
-        const float fo = fast_exp2((M - Mn) * kLog2e), fn = fast_exp2((m - Mn) * kLog2e);
-        s = s * fo + q[(int64_t)T + row] * fn;
-        t = t * fo + q[2 * (int64_t)T + row] * fn;
+    for (int p0 = grp; p0 < nparts; p0 += kMergeAhead * kMergeGrp) {
+      float m[kMergeAhead], ps[kMergeAhead], pt[kMergeAhead], Mn = M;
+#pragma unroll
+      for (int k = 0; k < kMergeAhead; ++k) {
+        const int p = p0 + k * kMergeGrp;
+        const float* q = part + (int64_t)(p < nparts ? p : p0) * 3 * T + row;
+        m[k] = q[0];
+        ps[k] = q[T];
+        pt[k] = q[2 * (int64_t)T];
+        if (p >= nparts) m[k] = ninf;
+      }
+#pragma unroll
+      for (int k = 0; k < kMergeAhead; ++k) Mn = fmaxf(Mn, m[k]);
+      if (Mn > ninf) {
+        const float fo = fast_exp2((M - Mn) * kLog2e);
+        s *= fo;
+        t *= fo;
+#pragma unroll
+        for (int k = 0; k < kMergeAhead; ++k) {
+          if (!(m[k] > ninf)) continue;
+          const float fn = fast_exp2((m[k] - Mn) * kLog2e);
+          s += ps[k] * fn;
+          t += pt[k] * fn;
+        }
         M = Mn;
       }
     }
@@ -731,19 +808,29 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(const float* __rest
   sh[grp][tl][1] = s;
   sh[grp][tl][2] = t;
   __syncthreads();
-  if (grp != 0 || row >= T) return;
-  float Mx = M;
-#pragma unroll
-  for (int g = 1; g < kMergeGrp; ++g) Mx = fmaxf(Mx, sh[g][tl][0]);
+  float Mx = ninf;
   double ss = 0.0, tt = 0.0;
+  if (grp < kMergeFold) {
 #pragma unroll
-  for (int g = 0; g < kMergeGrp; ++g) {
-    const float m = sh[g][tl][0];
-    if (m > -__builtin_inff()) {
-      const float f = fast_exp2((m - Mx) * kLog2e);
-      ss += (double)(sh[g][tl][1] * f);
-      tt += (double)(sh[g][tl][2] * f);
+    for (int g = 0; g < kMergeGrp; ++g) Mx = fmaxf(Mx, sh[g][tl][0]);
+#pragma unroll
+    for (int g = 0; g < kMergeGrp / kMergeFold; ++g) {
+      const float* a = sh[grp * (kMergeGrp / kMergeFold) + g][tl];
+      if (a[0] > ninf) {
+        const float f = fast_exp2((a[0] - Mx) * kLog2e);
+        ss += (double)(a[1] * f);
+        tt += (double)(a[2] * f);
+      }
     }
+    shd[grp][tl][0] = ss;
+    shd[grp][tl][1] = tt;
+  }
+  __syncthreads();
+  if (grp != 0 || row >= T) return;
+#pragma unroll
+  for (int g = 1; g < kMergeFold; ++g) {
+    ss += shd[g][tl][0];
+    tt += shd[g][tl][1];
   }
   const float lse = Mx + logf((float)ss);
   const float exv = (float)(tt / ss);
@@ -798,7 +885,6 @@ __global__ __launch_bounds__(256) void split3_kernel(const float* __restrict__ i
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-// AT: A is given by its K-rows (A[K][M], M contiguous, row pitch lda >= tiles_m * BM, K readable rows)
 // Shape of an XCD's block: `blk_m` tiles along M where the grid has room for it.  A grid narrower than the block in one
 // direction would leave most of the block's workgroup ids without a tile (a token count of one tile in blocks of 4 x 8:
 // 7 of 8 ids start and leave, each holding the CU's LDS meanwhile), so the block is made longer in the other one.
@@ -808,38 +894,41 @@ inline int fit_blk_m(int blk_m, int64_t tiles_m, int64_t tiles_n) {
   return blk_m;
 }
 
-template <class Epi, bool AT = false, bool F16 = false>
+template <class Epi, int AL = A_ROWS, bool F16 = false>
 int launch_gemm(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_total, int M, int N, int K, const Epi& epi,
-                hipStream_t st, const char* what, int splits = 1, int blk_m = 8) {
-  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<Epi, AT, F16>), kSmemBytes)) return rc;
-  GemmArgs g{A, lda, Bp, kb_total, M, N, K, (M + BM - 1) / BM, (N + BN - 1) / BN, splits, blk_m};
-  g.blk_m = blk_m = fit_blk_m(blk_m, g.tiles_m, (int64_t)g.tiles_n * splits);
-  if (AT && lda < (int64_t)g.tiles_m * BM) return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: row pitch %lld is shorter than %d tiles", what, (long long)lda, g.tiles_m);
-  const int64_t tiles = raster_grid(g.tiles_m, g.tiles_n * splits, blk_m);
-  gemm_nt_kernel<Epi, AT, F16><<<dim3((unsigned)tiles), dim3(kThreads), kSmemBytes, st>>>(g, epi);
+                hipStream_t st, const char* what, int splits = 1, int blk_m = 8, const uint16_t* A_tail = nullptr) {
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<Epi, AL, F16>), kSmemBytes)) return rc;
+  GemmArgs g{A, lda, Bp, kb_total, M, N, K, (M + BM - 1) / BM, (N + BN - 1) / BN, splits, blk_m, 0,
+             A_tail, A_tail ? K / BK - 1 : K / BK};
+  g.blk_m = fit_blk_m(blk_m, g.tiles_m, (int64_t)g.tiles_n * splits);
+  if (AL == A_PACKED && lda * 32 < (int64_t)g.tiles_m * BM) return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: row pitch %lld is shorter than %d tiles", what, (long long)lda, g.tiles_m);
+  const int64_t grid = raster_grid(g);
+  gemm_nt_kernel<Epi, AL, F16><<<dim3((unsigned)grid), dim3(kThreads), kSmemBytes, st>>>(g, epi);
   SIIRL_LAUNCH_CHECK(what);
   return SIIRL_OK;
 }
 
-// Tiles along M of an XCD's block, per GEMM of the fused path.  Measured at T=16384, H=3584, V=152064 (ms per step
-// for blocks of 2 x 16 / 4 x 8 / 8 x 4 / 16 x 2 tiles): forward 13.34 / 13.32 / 13.67 / 15.16; recompute + dlogits
-// 13.97 / 14.17 / 14.30 / 14.90 (1 x 32: slower again); d hidden 13.49 / 13.31 / 13.50 / 13.74; d weight 13.77 /
-// 13.50 / 13.40 / 14.24.  The A operand of the first two is W, streamed from memory once per strip of blk_n token
-// tiles: wider strips read it less often.
+// Tiles along M of an XCD's block, per GEMM of the fused path.  Measured at T=16384, H=3584, V=152064 with 256 x 256 tiles
+// (ms per step for blocks of 2 x 16 / 4 x 8 / 8 x 4 / 16 x 2 tiles): forward 13.34 / 13.32 / 13.67 / 15.16; recompute +
+// dlogits 13.97 / 14.17 / 14.30 / 14.90 (1 x 32: slower again); d weight 13.77 / 13.50 / 13.40 / 14.24.  The A operand
+// of the first two is W, streamed from memory once per strip of blk_n token tiles: wider strips read it less often.
+// d hidden with 128 x 256 tiles (us, first group): 7192 / 5574 / 6115 for blocks of 2 x 16 / 4 x 8 / 8 x 4; with one token
+// tile the tiles of a K run share nothing but its dlogits, so they go to one XCD: 649 / 437 / 410 / 304 / 300 us for 2 x 16
+// .. 32 x 1 at T=200.
 constexpr int kBlkFwd = 4, kBlkRecompute = 2, kBlkDHidden = 4, kBlkDWeight = 8;
 
 // Number of K runs of the d-hidden GEMM, each with an fp32 buffer of its own that sum_convert_kernel adds up.  The
-// tiles of [T, H] alone rarely fill the 256 CUs: 896 tiles at T=16384, H=3584 are 3.5 rounds (two runs: 7), 14 tiles at
-// T=200 a fraction of one (18 runs: 252 workgroups, 1743 -> 190 us).  The run count is the one with the least time by
-// the kernel's measured 1.2 us per K-step and about 12 us per tile besides, plus the buffers' write and read at 5 TB/s.
+// tiles of [T, H] alone rarely fill the 256 CUs, two each: 1792 tiles at T=16384, H=3584 are 3.5 rounds (two runs: 7), 28
+// tiles at T=200 a fraction of one (18 runs: 504 workgroups).  The run count is the one with the least time by
+// the kernel's measured 1.2 us per K-step of the two tiles on a CU and about 12 us per tile besides, plus the buffers' write and read at 5 TB/s.
 constexpr int kMaxSplits = 64;
 constexpr double kSplitBytes = 512.0 * 1048576.0;  // bound on the buffers beyond two
 // Up to 1024 tokens the choice does not look at T (it is the one for a single token tile; at T=1024, H=3584, K=152064
 // 18 runs model as 786 us against 710 us for the best 9), so that a row of d hidden keeps its bits whatever other rows
 // a small batch holds.
 inline int pick_splits(int64_t T, int64_t H, int64_t K) {
-  if (T <= 1024) T = BM;
-  const int64_t tiles = ((T + BM - 1) / BM) * ((H + BN - 1) / BN), KT = K / BK;
+  if (T <= 1024) T = BN;
+  const int64_t tiles = ((T + BN - 1) / BN) * ((H + BM - 1) / BM), KT = K / BK;
   int best = 1;
   double best_us = 0.;
   for (int s = 1; s <= kMaxSplits && s <= KT; ++s) {
@@ -847,7 +936,7 @@ inline int pick_splits(int64_t T, int64_t H, int64_t K) {
     if (s > 2 && bytes > kSplitBytes) break;
     const int64_t per = (KT + s - 1) / s;
     if ((s - 1) * per >= KT) continue;  // the last run would be empty
-    const double us = (double)((tiles * s + 255) / 256) * (1.2 * (double)per + 12.0) + 2.0 * bytes / 5e6;
+    const double us = (double)((tiles * s + 511) / 512) * (1.2 * (double)per + 12.0) + 2.0 * bytes / 5e6;
     if (s == 1 || us < best_us) best_us = us, best = s;
   }
   return best;
@@ -893,27 +982,27 @@ FwdWs fwd_ws(int64_t T, int64_t H, int64_t V, int dtype) {
 }
 
 struct BwdWs {
-  size_t hp, wtp, htp, d, dh32, hs, wsp, total;
-  int64_t ldwt, ldt, hpad, group, ldd_row;  // ldt: token count padded to BK (the K of the d-weight GEMM); group: columns
-                                            // of a vocabulary group; ldd_row: pitch of D
+  size_t hp, w16, wtail, htp, d, dh32, hs, wsp, total;
+  int64_t ldt, hpad, group, kb_d;  // ldt: token count padded to BK (the K of the d-weight GEMM); group: columns of a
+                                   // vocabulary group; kb_d: 1 KB blocks of D per 16 tokens
   int dh_splits;                            // K runs of the first (largest) group's d-hidden GEMM
 };
 BwdWs bwd_ws(int64_t T, int64_t H, int64_t V, bool want_dh, bool want_dw, int dtype) {
   BwdWs w;
   const int64_t Kc = logits_k(dtype, H);
-  w.ldwt = round_up(V, BK);
   w.ldt = round_up(T, BK);
   int64_t n = kGroupTokens / w.ldt;  // at most 64: a tile's byte offsets into D have 32 bits
   n = n < 1 ? 1 : (n > 64 ? 64 : n);
-  w.group = n * kGroupCols < V ? n * kGroupCols : round_up(V, BM);
-  w.ldd_row = w.group + kLdPad;
-  w.dh_splits = pick_splits(T, H, w.group < V ? w.group : w.ldwt);
+  w.group = n * kGroupCols < V ? n * kGroupCols : round_up(V, 256);
+  w.kb_d = w.group / 32 + kPadBlocks;
+  w.dh_splits = pick_splits(T, H, w.group < V ? w.group : round_up(V, BK));
   w.hpad = round_up(H, BN);
   size_t off = 0;
   w.hp = off; off += (size_t)round_up(T, BN) * Kc * 2;
-  w.wtp = off; off += want_dh ? (size_t)w.hpad * w.ldwt * 2 : 0;
+  w.w16 = off; off += want_dh && dtype == SIIRL_F16 ? round_up((size_t)V * H * 2, 256) : 0;
+  w.wtail = off; off += want_dh && V % BK ? round_up((size_t)BK * Kc * 2, 256) : 0;
   w.htp = off; off += want_dw ? (size_t)w.hpad * w.ldt * 2 : 0;
-  w.d = off; off += round_up((size_t)w.ldt * w.ldd_row * 2, 256);  // rows [T, ldt) are K-padding of d weight: zeros
+  w.d = off; off += (size_t)(round_up(T, BN) / 16) * w.kb_d * 1024;  // tokens [T, ldt) are K-padding of d weight: zeros
   w.dh32 = off; off += want_dh ? w.dh_splits * round_up((size_t)T * H * 4, 256) : 0;  // one buffer per K run
   w.hs = off; off += dtype == SIIRL_F32 ? round_up((size_t)T * Kc * 2, 256) : 0;
   w.wsp = off; off += dtype == SIIRL_F32 ? round_up((size_t)V * Kc * 2, 256) : 0;
@@ -930,10 +1019,6 @@ int stage_f32(const void* hidden, const void* weight, int64_t T, int64_t H, int6
   split3_kernel<<<dim3((unsigned)((qw + 255) / 256)), dim3(256), 0, st>>>((const float*)weight, V, H, wsp, 0);
   SIIRL_LAUNCH_CHECK("split3_kernel(weight)");
   return SIIRL_OK;
-}
-
-__global__ __launch_bounds__(256) void zero_fill_kernel(u32x4* __restrict__ p, int64_t n16) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256) p[i] = u32x4{0u, 0u, 0u, 0u};
 }
 
 int pack_hidden(const uint16_t* h, int64_t T, int64_t H, u32x4* out, hipStream_t st) {
@@ -1054,13 +1139,13 @@ extern "C" int siirl_fused_linear_logprob_entropy_fwd(const void* hidden, const 
   u32x4* hp = reinterpret_cast<u32x4*>((char*)workspace + ws.hp);
   if (int rc = pack_hidden(h, T, Kc, hp, st)) return rc;
   SoftmaxPartialsEpi epi{inv_temperature, (int)T, (int)V, part, saved_logits, (int)((T + BN - 1) / BN)};
-  if (int rc = f16 ? launch_gemm<SoftmaxPartialsEpi, false, true>(w, Kc, hp, Kc / 32, (int)V, (int)T, (int)Kc, epi, st,
+  if (int rc = f16 ? launch_gemm<SoftmaxPartialsEpi, A_ROWS, true>(w, Kc, hp, Kc / 32, (int)V, (int)T, (int)Kc, epi, st,
                                                                   "gemm_nt_kernel<SoftmaxPartialsEpi, f16>", 1, kBlkFwd)
                    : launch_gemm(w, Kc, hp, Kc / 32, (int)V, (int)T, (int)Kc, epi, st, "gemm_nt_kernel<SoftmaxPartialsEpi>", 1,
                                  kBlkFwd))
     return rc;
   const int tiles_v = (int)((V + BM - 1) / BM);
-  merge_partials_kernel<<<dim3((unsigned)((T + kMergeTok - 1) / kMergeTok)), dim3(256), 0, st>>>(part, tiles_v, (int)T, label_logit,
+  merge_partials_kernel<<<dim3((unsigned)((T + kMergeTok - 1) / kMergeTok)), dim3(kMergeThreads), 0, st>>>(part, tiles_v, (int)T, label_logit,
                                                                                logprob, entropy, lse, ex);
   SIIRL_LAUNCH_CHECK("merge_partials_kernel");
   return SIIRL_OK;
@@ -1087,9 +1172,9 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
   hipStream_t st = (hipStream_t)stream;
   char* base = (char*)workspace;
   u32x4* hp = (u32x4*)(base + ws.hp);          // packed hidden: B[n = token][k = K of the logits GEMM]
-  u32x4* Wtp = (u32x4*)(base + ws.wtp);        // packed W^T:    B[n = H][k = vocabulary]
+  u32x4* W16 = (u32x4*)(base + ws.w16);        // fp16 operands: bf16 copy of W
   u32x4* Htp = (u32x4*)(base + ws.htp);        // packed hidden^T: B[n = H][k = token]
-  uint16_t* D = (uint16_t*)(base + ws.d);      // [ldt][ldd_row]: one vocabulary group
+  char* D = base + ws.d;                       // packed dlogits of one vocabulary group
   float* dH32 = (float*)(base + ws.dh32);      // [T][H]
   const uint16_t* h = (const uint16_t*)hidden;
   const uint16_t* w = (const uint16_t*)weight;
@@ -1108,27 +1193,31 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
 
   if (!saved_logits)
     if (int rc = pack_hidden(h, T, Kc, hp, st)) return rc;
-  if (want_dh) {
-    transpose_pack_b_kernel<<<dim3((unsigned)(ws.ldwt / 64), (unsigned)(ws.hpad / 64)), dim3(256), 0, st>>>(
-        w, Kc, (int)V, (int)H, Wtp, ws.ldwt / 32, (int)f16);
-    SIIRL_LAUNCH_CHECK("transpose_pack_b_kernel(W)");
+  uint16_t* Wtail = (uint16_t*)(base + ws.wtail);  // the last V % BK rows of W and zeros
+  const uint16_t* wg = w;  // W as the gradient GEMM reads it: bf16 rows of pitch Kc, H of them used
+  if (want_dh && f16) {
+    const int64_t n8 = V * H / 8;
+    f16_to_bf16_kernel<<<dim3((unsigned)((n8 + 255) / 256 < 65536 ? (n8 + 255) / 256 : 65536)), dim3(256), 0, st>>>(
+        reinterpret_cast<const u32x4*>(w), W16, n8);
+    SIIRL_LAUNCH_CHECK("f16_to_bf16_kernel");
+    wg = reinterpret_cast<const uint16_t*>(W16);
+  }
+  if (want_dh && V % BK) {
+    const int64_t n8 = BK * Kc / 8, have8 = V % BK * Kc / 8;  // (Kc is a multiple of BK)
+    copy_padded_kernel<<<dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st>>>(
+        reinterpret_cast<const u32x4*>(wg + V / BK * BK * Kc), have8, reinterpret_cast<u32x4*>(Wtail), n8);
+    SIIRL_LAUNCH_CHECK("copy_padded_kernel");
   }
   if (want_dw) {
     transpose_pack_b_kernel<<<dim3((unsigned)(ws.ldt / 64), (unsigned)(ws.hpad / 64)), dim3(256), 0, st>>>(
         h, Kc, (int)T, (int)H, Htp, ws.ldt / 32, (int)f16);
     SIIRL_LAUNCH_CHECK("transpose_pack_b_kernel(hidden)");
   }
-  if (want_dw && ws.ldt > T) {  // the token rows that only pad the K of the d-weight GEMM (ldd_row * 2 % 16 == 0)
-    const int64_t n16 = (ws.ldt - T) * ws.ldd_row * 2 / 16;
-    zero_fill_kernel<<<dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)), dim3(256), 0, st>>>(
-        reinterpret_cast<u32x4*>(D + T * ws.ldd_row), n16);
-    SIIRL_LAUNCH_CHECK("zero_fill_kernel");
-  }
   const int64_t dh32_stride = (int64_t)(round_up((size_t)T * H * 4, 256) / 4);
   const int tiles_t = (int)((T + BN - 1) / BN);
-  // The recompute goes in launches of about 2048 workgroups (8192 columns at 16384 tokens, whose 59 MB of W stay in the
+  // The recompute goes in launches of about 4096 workgroups (8192 columns at 16384 tokens, whose 59 MB of W stay in the
   // memory-side cache while the token tiles pass over them: 0.4 % of the whole step faster than one launch per group).  At
-  // T=200 that is one launch of 594 workgroups; 19 launches of 8192 columns had 32 each (1766 against 330 us).
+  // T=200 that is one launch of 1188 workgroups; 19 launches of 8192 columns had 32 each (1766 against 330 us).
   const int slab = 8192 * (tiles_t < 64 ? 64 / tiles_t : 1);
   for (int64_t v0 = 0; v0 < V; v0 += ws.group) {
     const int N = (int)(V - v0 < ws.group ? V - v0 : ws.group);
@@ -1136,10 +1225,10 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
     if (!saved_logits) {
       for (int s0 = 0; s0 < N; s0 += slab) {
         const int Ns = N - s0 < slab ? N - s0 : slab;
-        const DlogitsEpi epi{inv_temperature, (int)T, Ns, (int)round_up(Ns, BK), v0 + s0, lse, ex, g_logprob, g_entropy,
-                             labels, D + s0, ws.ldd_row};
+        const DlogitsEpi epi{inv_temperature, (int)T, (int)ws.ldt, Ns, (int)round_up(Ns, BK), v0 + s0, lse, ex, g_logprob,
+                             g_entropy, labels, D + (s0 >> 5) * 1024, ws.kb_d};
         const uint16_t* ws0 = w + (v0 + s0) * Kc;
-        if (int rc = f16 ? launch_gemm<DlogitsEpi, false, true>(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st,
+        if (int rc = f16 ? launch_gemm<DlogitsEpi, A_ROWS, true>(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st,
                                                                 "gemm_nt_kernel<DlogitsEpi, f16>", 1, kBlkRecompute)
                          : launch_gemm(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st, "gemm_nt_kernel<DlogitsEpi>", 1,
                                        kBlkRecompute))
@@ -1147,7 +1236,7 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
       }
     } else {
       // the group's dlogits in one pass over the tiles the forward parked
-      const DlogitsEpi epi{inv_temperature, (int)T, N, Npad, v0, lse, ex, g_logprob, g_entropy, labels, D, ws.ldd_row};
+      const DlogitsEpi epi{inv_temperature, (int)T, (int)ws.ldt, N, Npad, v0, lse, ex, g_logprob, g_entropy, labels, D, ws.kb_d};
       const void* fn = reinterpret_cast<const void*>(&replay_tiles_kernel<DlogitsEpi>);
       if (int rc = allow_dynamic_lds(fn, kSmemBytes)) return rc;
       const int64_t wgs = (int64_t)((N + BM - 1) / BM) * tiles_t;
@@ -1156,8 +1245,9 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
       SIIRL_LAUNCH_CHECK("replay_tiles_kernel<DlogitsEpi>");
     }
     if (want_dh) {
-      // dH[T, H] += D[T, K] . Wt[H, v0 : v0 + K]^T over the group's columns.  A shallower last group may take fewer runs
-      // than the first one: it then adds to the first buffers only.
+      // dH[T, H] += D[T, K] . W[v0 : v0 + K, H] over the group's columns, as its transpose: W is the A operand given by its
+      // K-rows, as it lies in memory, the packed D the B operand.  A shallower last group may take fewer runs than the
+      // first one: it then adds to the first buffers only.
       int splits = ws.dh_splits;
       if (v0 > 0) {
         const int fit = pick_splits(T, H, Npad);
@@ -1165,17 +1255,18 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
         const int KT = Npad / BK, per = (KT + splits - 1) / splits;
         splits = (KT + per - 1) / per;  // no run is empty
       }
-      AccumF32Epi acc{dH32, H, dh32_stride, (int)T, (int)H, v0 > 0 ? 1 : 0};
-      if (int rc = launch_gemm(D, ws.ldd_row, Wtp + (v0 / 32) * 64, ws.ldwt / 32, (int)T, (int)H, Npad, acc, st,
-                               "gemm_nt_kernel<AccumF32Epi>", splits, kBlkDHidden))
+      AccumF32Epi acc{dH32, H, dh32_stride, (int)H, (int)T, v0 > 0 ? 1 : 0};
+      if (int rc = launch_gemm<AccumF32Epi, A_KROWS>(wg + v0 * Kc, Kc, reinterpret_cast<const u32x4*>(D), ws.kb_d, (int)H,
+                                                     (int)T, Npad, acc, st, "gemm_nt_kernel<AccumF32Epi, A by K-rows>",
+                                                     splits, T <= BN ? kBlkTiles : kBlkDHidden, N < Npad ? Wtail : nullptr))
         return rc;
     }
     if (want_dw) {
       // dW[v0 : v0 + N, H] = D[ldt, N]^T . Ht[H, ldt]^T over the group's vocabulary rows: D is the A operand given by its
-      // K-rows (tokens)
+      // packed K-rows (tokens)
       StoreEpi sto{(char*)d_weight + v0 * H * (int64_t)dtype_size(dtype), H, N, (int)H, dtype};
-      if (int rc = launch_gemm<StoreEpi, true>(D, ws.ldd_row, Htp, ws.ldt / 32, N, (int)H, (int)ws.ldt, sto, st,
-                                               "gemm_nt_kernel<StoreEpi, A by K-rows>", 1, kBlkDWeight))
+      if (int rc = launch_gemm<StoreEpi, A_PACKED>(reinterpret_cast<const uint16_t*>(D), ws.kb_d, Htp, ws.ldt / 32, N,
+                                                   (int)H, (int)ws.ldt, sto, st, "gemm_nt_kernel<StoreEpi, packed A>", 1, kBlkDWeight))
         return rc;
     }
   }

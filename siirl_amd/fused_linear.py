@@ -58,7 +58,7 @@ def set_skip_zero_rows(flag: bool) -> None:
 
 
 def _saved_logits_bytes(T: int, V: int) -> int:
-    return ((V + 255) // 256) * ((T + 255) // 256) * (256 * 256 * 4)
+    return ((V + 127) // 128) * ((T + 255) // 256) * (128 * 256 * 4)
 
 
 def _apply(hidden2d, weight, labels1d, temperature):
