@@ -58,6 +58,8 @@ constexpr int64_t kSkipRow = SIIRL_LABEL_SKIP_ROW;
 #define SIIRL_LPE_BWD_NT_STORE 1
 #endif
 constexpr int kFwdThreads = SIIRL_LPE_FWD_THREADS;  // waves per row = threads / 64
+constexpr int kFwdWideThreads = 1024;               // with few long rows
+constexpr int64_t kWideRows = 256;
 constexpr int kFwdUnroll = SIIRL_LPE_FWD_UNROLL;    // 16-byte loads in flight per lane
 constexpr int kBwdThreads = SIIRL_LPE_BWD_THREADS;
 constexpr int kBwdUnroll = SIIRL_LPE_BWD_UNROLL;
@@ -192,8 +194,8 @@ __device__ __forceinline__ void absorb_vecs(SoftState& st, const u32x4* buf, flo
 
 // NT: the row is streamed with non-temporal loads (worth 12 % when the logits are many times the memory-side cache);
 // without them a tensor that fits that cache is still there when the backward reads it again.
-template <class E, bool ENT, bool NT>
-__global__ __launch_bounds__(kFwdThreads) void lpe_fwd_kernel(const typename E::elem_t* __restrict__ logits,
+template <class E, bool ENT, bool NT, int kThreads>
+__global__ __launch_bounds__(kThreads) void lpe_fwd_kernel(const typename E::elem_t* __restrict__ logits,
                                                            int64_t row_stride, int V,
                                                            const int64_t* __restrict__ labels, float inv_T,
                                                            float* __restrict__ logprob, float* __restrict__ entropy,
@@ -218,21 +220,28 @@ __global__ __launch_bounds__(kFwdThreads) void lpe_fwd_kernel(const typename E::
 
   SoftState st{-1e30f, 0.f, 0.f};
 
-  for (int i = tid; i < sp.head; i += kFwdThreads) absorb1<ENT>(st, E::load1(x + i), k);
-  for (int i = sp.tail0 + tid; i < V; i += kFwdThreads) absorb1<ENT>(st, E::load1(x + i), k);
+  for (int i = tid; i < sp.head; i += kThreads) absorb1<ENT>(st, E::load1(x + i), k);
+  for (int i = sp.tail0 + tid; i < V; i += kThreads) absorb1<ENT>(st, E::load1(x + i), k);
 
   const u32x4* __restrict__ xv = reinterpret_cast<const u32x4*>(x + sp.head);
-  constexpr int kTile = kFwdThreads * kFwdUnroll;
+  constexpr int kTile = kThreads * kFwdUnroll;
   const int nfull = sp.nvec / kTile * kTile;
   for (int base = 0; base < nfull; base += kTile) {
     u32x4 buf[kFwdUnroll];
 #pragma unroll
-    for (int u = 0; u < kFwdUnroll; ++u) buf[u] = ld16<NT>(xv + base + u * kFwdThreads + tid);
+    for (int u = 0; u < kFwdUnroll; ++u) buf[u] = ld16<NT>(xv + base + u * kThreads + tid);
     absorb_vecs<E, ENT, kFwdUnroll>(st, buf, k);
   }
-  for (int i = nfull + tid; i < sp.nvec; i += kFwdThreads) {
-    u32x4 b = ld16<NT>(xv + i);
-    absorb_vecs<E, ENT, 1>(st, &b, k);
+  {  // the ragged end: its loads are in flight together as well (one at a time: [512, 32000] bf16 8.6 us instead of 7.9)
+    u32x4 buf[kFwdUnroll];
+#pragma unroll
+    for (int u = 0; u < kFwdUnroll; ++u) {
+      const int i = nfull + u * kThreads + tid;
+      if (i < sp.nvec) buf[u] = ld16<NT>(xv + i);
+    }
+#pragma unroll
+    for (int u = 0; u < kFwdUnroll; ++u)
+      if (nfull + u * kThreads + tid < sp.nvec) absorb_vecs<E, ENT, 1>(st, buf + u, k);
   }
 
   // wave merge
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(kFwdThreads) void lpe_fwd_kernel(const typename E::
     const float ot = __shfl_xor(st.t, o, kWave);
     merge(st, omx, os, ot, k);
   }
-  __shared__ float sm[3 * (kFwdThreads / kWave)];
+  __shared__ float sm[3 * (kThreads / kWave)];
   const int lane = tid & (kWave - 1), wid = tid / kWave;
   if (lane == 0) {
     sm[wid * 3 + 0] = st.mx;
@@ -253,7 +262,7 @@ __global__ __launch_bounds__(kFwdThreads) void lpe_fwd_kernel(const typename E::
   __syncthreads();
   if (tid == 0) {
 #pragma unroll
-    for (int w = 1; w < kFwdThreads / kWave; ++w) merge(st, sm[w * 3], sm[w * 3 + 1], sm[w * 3 + 2], k);
+    for (int w = 1; w < kThreads / kWave; ++w) merge(st, sm[w * 3], sm[w * 3 + 1], sm[w * 3 + 2], k);
     const float lse = st.mx * inv_T + logf(st.s);
     lse_out[row] = lse;
     if (ENT) {
@@ -716,16 +725,28 @@ template <class E>
 int launch_fwd(const void* logits, int64_t T, int V, int64_t row_stride, const int64_t* labels, float inv_T,
                float* logprob, float* entropy, float* lse, float* ex, hipStream_t st) {
   using elem_t = typename E::elem_t;
-  dim3 grid((unsigned)T), block(kFwdThreads);
+  dim3 grid((unsigned)T);
   // Logits of up to kCacheResidentBytes (the part's 256 MB memory-side cache and a little more) are read with
   // ordinary loads, so that the backward pass that follows finds them cached: measured on [2048, 32000] fp32
   // (250 MiB) forward + backward 128 -> 117 us, [768, 152064] bf16 (223 MiB) 114 -> 103 us, the forward alone
   // unchanged; from 375 MiB upwards the non-temporal loads win (forward alone 60 against 70 us at that size).
   const bool nt = SIIRL_LPE_FWD_NT_LOAD && streams_past_cache((double)T * (double)V * (double)sizeof(elem_t));
-  auto go = [&](auto ent_tag, auto nt_tag) {
-    lpe_fwd_kernel<E, decltype(ent_tag)::value, decltype(nt_tag)::value><<<grid, block, 0, st>>>(
+  // With no more rows than CUs a row's workgroup has its CU to itself, and four waves keep too few loads in flight: 1024
+  // threads where a row gives each of them four vectors four times.  Forward alone, 256 / 1024 threads (us): V=152064
+  // bf16 32 rows 12.2 / 10.7, 256 rows 18.3 / 15.5, 400 rows 21.9 / 24.4; fp32 128 rows 25.3 / 15.3; V=32000 bf16 32 rows
+  // 5.4 / 5.7, fp32 128 rows 6.9 / 8.0.
+  const bool wide = T <= kWideRows && V / E::VEC >= 4 * kFwdWideThreads * kFwdUnroll;
+  auto launch = [&](auto ent_tag, auto nt_tag, auto threads) {
+    constexpr int kThreads = decltype(threads)::value;
+    lpe_fwd_kernel<E, decltype(ent_tag)::value, decltype(nt_tag)::value, kThreads><<<grid, dim3(kThreads), 0, st>>>(
         (const elem_t*)logits, row_stride, V, labels, inv_T, logprob, decltype(ent_tag)::value ? entropy : nullptr, lse,
         decltype(ent_tag)::value ? ex : nullptr);
+  };
+  auto go = [&](auto ent_tag, auto nt_tag) {
+    if (wide)
+      launch(ent_tag, nt_tag, std::integral_constant<int, kFwdWideThreads>{});
+    else
+      launch(ent_tag, nt_tag, std::integral_constant<int, kFwdThreads>{});
   };
   using Yes = std::true_type;
   using No = std::false_type;

@@ -100,7 +100,8 @@ def test_fused_random_shapes_sweep(dev):
         FL.set_saved_logits_limit(0)
 
 
-@pytest.mark.parametrize("T,H,V", [(8200, 64, 65793), (8192, 128, 70000), (200, 320, 40000), (31, 64, 131073)])
+@pytest.mark.parametrize("T,H,V", [(8200, 64, 65793), (8192, 128, 70000), (200, 320, 40000), (31, 64, 131073),
+                                   (257, 448, 33003)])
 def test_column_groups_and_k_runs(dev, T, H, V):
     """Vocabularies of more than one column group (8192 tokens and more: 65536 columns; the last group is shallower than
     the first, down to 5 K-steps), and d hidden summed from many K runs (few token tiles).  Reference: float64 on the GPU."""

@@ -71,6 +71,19 @@ def test_forward_backward_matches_oracle(dev, dtype, T, V):
         assert torch.count_nonzero(dx[1]) == 0
 
 
+@pytest.mark.parametrize("dtype,T,V", [(torch.bfloat16, 3, 131071), (torch.bfloat16, 3, 131072), (torch.bfloat16, 2, 163843),
+                                       (torch.float32, 2, 65536), (torch.float32, 256, 65540), (torch.float32, 257, 65540)])
+def test_forward_few_long_rows(dev, dtype, T, V):
+    """Both sides of the line between four and sixteen waves a row, with ragged ends and rows of every alignment."""
+    import siirl_amd.torch_functional as SF
+
+    x, y = _make(T, V, dtype, seed=T + V)
+    lp, ent = SF.logprobs_and_entropy_from_logits(x.to(dev), y.to(dev))
+    logp = torch.log_softmax(x.to(dev).double(), dim=-1)
+    assert (lp.double() - logp.gather(-1, y.to(dev)[:, None]).squeeze(-1)).abs().max() < 1e-4
+    assert (ent.double() + (logp.exp() * logp).sum(-1)).abs().max() < 1e-4
+
+
 @pytest.mark.parametrize("temperature", [0.6, 1.0, 1.7])
 def test_temperature_folded(dev, temperature):
     import siirl_amd.torch_functional as SF
