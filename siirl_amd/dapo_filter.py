@@ -116,7 +116,7 @@ def filter_tensordict(batch, indices: List[int]):
     anything else is metadata and is kept.  An empty list gives an empty batch.  Works on a ``dict`` and on
     a ``TensorDict`` (returned as the same kind)."""
     is_td = hasattr(batch, "batch_size") and not isinstance(batch, dict)
-    if not indices:
+    if indices is None or len(indices) == 0:
         if is_td:
             return type(batch)({}, batch_size=(0,))
         return {}
@@ -133,7 +133,7 @@ def filter_tensordict(batch, indices: List[int]):
         elif isinstance(data, np.ndarray) and len(data) == bsz:
             out[key] = data[idx_np]
         elif isinstance(data, (list, tuple)) and len(data) == bsz:
-            out[key] = [data[i] for i in indices]
+            out[key] = [data[i] for i in idx_np.tolist()]
         else:
             out[key] = value
     if is_td:
@@ -218,11 +218,15 @@ def dynamic_sampling(config, batch, **kwargs) -> NodeOutput:
                        f"Available non-tensor keys: {keys}")
     uids = batch["uid"]
     keep, gsz = group_keep_mask(metric, uids, return_group_size=True)
-    kept = torch.nonzero(keep).flatten().tolist()
-    inv = 1.0 / gsz.double()  # each group of n members contributes n * (1/n) = 1
-    total_groups = int(torch.round(inv.sum()).item())
-    kept_groups = int(torch.round((inv * keep).sum()).item())
-    filtered = filter_tensordict(batch, kept)
+    # one copy to the host, and one wait for the GPU, for everything that the host has to know: 2 * group size + kept
+    codes = torch.add(keep, gsz, alpha=2).cpu().numpy()
+    mask = (codes & 1).astype(bool)
+    kept_rows = np.flatnonzero(mask)
+    kept = kept_rows.tolist()
+    inv = 1.0 / (codes >> 1)  # each group of n members contributes n * (1/n) = 1
+    total_groups = int(np.rint(inv.sum()))
+    kept_groups = int(np.rint(inv[mask].sum()))
+    filtered = filter_tensordict(batch, kept_rows)
     final = len(kept)
     metrics = {
         "dapo_sampling/kept_trajectories_ratio": final / initial if initial > 0 else 1.0,
