@@ -125,10 +125,12 @@ __device__ __forceinline__ int acc_row(int i, int r, int lane) {
 }
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * (NJ * 16) + j * 16 + (lane & 15); }
 // An epilogue with kRowsPerLane takes the accumulator the other way round (the MFMA's operands are swapped): a lane owns
-// the rows row_of_lane(i) and, with B packed in the column order of transpose_pack_b_kernel, the 16 consecutive columns
-// from col_of_lane on: element r of acc[i][j] is column col_of_lane + 4 * j + r.
+// the rows row_of_lane(i) and, with B packed in the column order of transpose_pack_b_kernel, 8 consecutive columns from
+// col_of_lane(j) on of each pair j, j + 1 (j even) of N-tiles: element r of acc[i][j] is column col_of_lane(j) + r.
 __device__ __forceinline__ int row_of_lane(int i, int lane) { return i * 16 + (lane & 15); }
-__device__ __forceinline__ int col_of_lane(int wn, int lane) { return wn * (NJ * 16) + (lane >> 4) * 16; }
+__device__ __forceinline__ int col_of_lane(int wn, int j, int lane) {
+  return wn * (NJ * 16) + (j >> 1) * 32 + (lane >> 4) * 8 + (j & 1) * 4;
+}
 
 // m0 (the DMA's LDS base) is a reserved register: naming it in a clobber list is right but draws a warning
 #pragma clang diagnostic push
@@ -388,6 +390,83 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 }
 #pragma clang diagnostic pop
 
+// The same product for a K of at most four K-steps and a packed A (d weight at up to 256 tokens).  A tile of it is one to
+// four K-steps of matrix work between a fetch and a store of 64 KB, and gemm_nt_kernel starts a workgroup for each: at
+// T=200, H=3584, V=152064 it wrote d weight at 2.2 TB/s.  Here the four stages of the ring hold a row tile's whole K, and
+// the workgroup walks n_per tiles along N with it: no barrier after the first, so that its waves, and the CU's other
+// workgroup, multiply while some of them store.  What remains is matrix work
+// (200 us at the rate of the large GEMMs) and the store of C (180 us) hardly overlapping.  d weight, us: T=200 485 -> 440, and
+// 43 at T=64, H=2048, V=50257 (4.8 TB/s).  Fetching B two steps ahead with branch-free stores, so that no fetch waits behind a
+// store, measured the same (439); non-temporal stores 454, and 129 at T=64.
+constexpr int kShortSteps = kStages;
+template <class Epi>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_short_k_kernel(
+    GemmArgs g, int n_per, Epi epi) {
+  static_assert(Epi::kRowsPerLane, "the MFMA operands are swapped");
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wn = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tm = blockIdx.x % g.tiles_m, tn0 = (int)(blockIdx.x / g.tiles_m) * n_per;
+  const int tn1 = tn0 + n_per < g.tiles_n ? tn0 + n_per : g.tiles_n;
+  const int m0 = tm * BM, KT = g.K / BK;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const char* gA = reinterpret_cast<const char*>(g.A) + (int64_t)(m0 >> 5) * 1024;
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < kDmaPerWave; ++i) {  // slots as in gemm_nt_kernel, A_PACKED
+      constexpr int kBlocks = BM / 32;
+      const int I = wn * kDmaPerWave + i;
+      const char* base = gA + ((int64_t)(kt * (BK / 16) + I / kBlocks) * g.lda + I % kBlocks) * 1024;
+      const uint32_t dst = lds0 + kt * kStageBytes + I * 1024, off = (lane ^ ((lane >> 2) & 4)) * 16;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "m0", "memory");
+    }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  const int kq = lane >> 4, mc = lane & 3, tq = (lane & 15) >> 2;
+  const char* frag = smem + (kq >> 1) * (BM * 32) + ((kq & 1) * 8 + (mc & 2) * 2 + tq) * 16 + (mc >> 1) * 256 + (mc & 1) * 8;
+  const char* frag4 = smem + ((uint32_t)(frag - smem) ^ 64u);
+  auto fetch = [&](u32x4 (&b)[NJ][KS], int tn, int kt) {
+    const u32x4* p = g.Bp + ((int64_t)(tn * (BN / 16) + wn * NJ) * g.kb_total + kt * KS) * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) b[j][s] = p[(int64_t)j * g.kb_total * 64 + s * 64];
+  };
+  u32x4 b[NJ][KS], bn[NJ][KS];
+  fetch(b, tn0, 0);
+  for (int tn = tn0; tn < tn1; ++tn) {
+    floatx4 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < KT; ++kt) {
+      // the next step's B, of this tile or the next one (past the end: of the last step again)
+      const bool same = kt + 1 < KT, more = same || tn + 1 < tn1;
+      fetch(bn, more && !same ? tn + 1 : tn, same ? kt + 1 : (more ? 0 : kt));
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          typedef short s16x4 __attribute__((ext_vector_type(4)));
+          typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+          const int at = kt * kStageBytes + s * (32 * BM * 2) + i * 512;
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(frag + at));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(frag4 + at));
+          const bf16x8 af = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b[j][s]), af, acc[i][j], 0, 0, 0);
+        }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int s = 0; s < KS; ++s) b[j][s] = bn[j][s];
+    }
+    epi(acc, m0, tn * BN, tm, 0, wn, lane, tid, smem);
+  }
+}
+
 // ------------------------------------------------------------------------------ parked accumulator tiles
 
 // Tile (tm, tn) of the forward GEMM occupies kQuads * kThreads 16-byte slots; slot c * kThreads + tid holds thread
@@ -613,9 +692,10 @@ __device__ __forceinline__ uint2 pack4(floatx4 v, int out_dtype) {
 }
 
 // C[row][col] = acc, rounded to the output type (out_dtype: SIIRL_BF16, SIIRL_F16 or SIIRL_F32).  Takes the accumulator
-// by rows: a lane holds 16 consecutive columns of a row, 32 (16-bit) or 64 bytes, and the four lanes of a row a whole
-// 128-byte line or two.  With a column per lane each store instruction wrote 2-byte pieces, 128 per lane and tile instead
-// of 16 or 32.  N is a multiple of 64, so a wave's columns are all inside the matrix or all outside.
+// by rows: the four lanes of a row write 64 consecutive bytes per instruction (16-bit types).  With 16 columns a lane an
+// instruction wrote 16 bytes of every 32, and the L2 had to hold the half-written lines until their other half came:
+// T=16384, H=3584,
+// V=152064 forward + backward 54.2 -> 53.2 ms, d weight at T=64, H=2048, V=50257 47 -> 43 us.  N is a multiple of 64, so a wave's columns are all inside the matrix or all outside.
 struct StoreEpi {
   static constexpr bool kRowsPerLane = true;
   void* C;
@@ -623,29 +703,27 @@ struct StoreEpi {
   int M, N, out_dtype;
   __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wn, int lane, int tid,
                              char* smem) const {
-    const int col = n0 + col_of_lane(wn, lane);
-    if (col >= N) return;
-    const bool aligned = ((uintptr_t)C & 15) == 0;  // (a caller's buffer need not be; ldc and col are multiples of 16)
+    if (n0 + col_of_lane(wn, 0, lane) >= N) return;
+    const bool aligned = ((uintptr_t)C & 15) == 0;  // (a caller's buffer need not be; ldc and a pair's columns are multiples of 8)
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       const int row = m0 + row_of_lane(i, lane);
       if (row >= M) continue;
-      const int64_t at = (int64_t)row * ldc + col;
+      const int64_t at = (int64_t)row * ldc + n0;
       if (!aligned) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) store_one(C, at + j * 4 + r, acc[i][j][r], out_dtype);
+          for (int r = 0; r < 4; ++r) store_one(C, at + col_of_lane(wn, j, lane) + r, acc[i][j][r], out_dtype);
       } else if (out_dtype == SIIRL_F32) {
-        f32x4* p = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + at);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) p[j] = acc[i][j];
+        for (int j = 0; j < NJ; ++j)
+          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + at + col_of_lane(wn, j, lane)) = acc[i][j];
       } else {
-        u32x4* p = reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(C) + at);
 #pragma unroll
         for (int j = 0; j < NJ; j += 2) {
           const uint2 a = pack4(acc[i][j], out_dtype), b = pack4(acc[i][j + 1], out_dtype);
-          p[j / 2] = u32x4{a.x, a.y, b.x, b.y};
+          *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(C) + at + col_of_lane(wn, j, lane)) = u32x4{a.x, a.y, b.x, b.y};
         }
       }
     }
@@ -671,8 +749,8 @@ __global__ __launch_bounds__(256) void pack_b_kernel(const uint16_t* __restrict_
 }
 
 // The same packing of the transpose: B[n][k] = in[k][n] with in of shape [R = K][C = N].  A workgroup stages a
-// 64 x 64 tile through LDS and emits its 512 chunks.  Within each 64 columns, column n = 16 q + 4 j + r takes the place
-// of row 4 q + r of 16-row block j, so that an epilogue with kRowsPerLane finds 16 consecutive columns in a lane.
+// 64 x 64 tile through LDS and emits its 512 chunks.  Within each 64 columns, column n = 32 h + 8 q + 4 e + r takes the place
+// of row 4 q + r of 16-row block 2 h + e, so that an epilogue with kRowsPerLane finds 8 consecutive columns in a lane.
 // from_f16: the input holds IEEE halves, the packed output bf16 (round to nearest even).
 __device__ __forceinline__ uint32_t half2_to_bf16x2(uint32_t w) { return pack_bf16(f16_lo(w), f16_hi(w)); }
 __global__ __launch_bounds__(256) void transpose_pack_b_kernel(const uint16_t* __restrict__ in, int64_t ld_in, int R,
@@ -705,8 +783,8 @@ __global__ __launch_bounds__(256) void transpose_pack_b_kernel(const uint16_t* _
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = (uint32_t)tile[kc * 8 + 2 * e][nl] | ((uint32_t)tile[kc * 8 + 2 * e + 1][nl] << 16);
     const int64_t n = c0 + nl, k = r0 + kc * 8;
-    const int64_t nb = (n >> 6) * 4 + ((n >> 2) & 3);                       // 16-row block
-    const int nr = (int)(((n >> 4) & 3) * 4 + (n & 3));                     // row in it
+    const int64_t nb = (n >> 6) * 4 + ((n >> 5) & 1) * 2 + ((n >> 2) & 1);  // 16-row block
+    const int nr = (int)(((n >> 3) & 3) * 4 + (n & 3));                     // row in it
     const int64_t ch = (nb * KB + (k >> 5)) * 64 + nr + 16 * ((k >> 3) & 3);
     out[ch] = u32x4{w[0], w[1], w[2], w[3]};
   }
@@ -904,6 +982,23 @@ int launch_gemm(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_tota
   if (AL == A_PACKED && lda * 32 < (int64_t)g.tiles_m * BM) return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: row pitch %lld is shorter than %d tiles", what, (long long)lda, g.tiles_m);
   const int64_t grid = raster_grid(g);
   gemm_nt_kernel<Epi, AL, F16><<<dim3((unsigned)grid), dim3(kThreads), kSmemBytes, st>>>(g, epi);
+  SIIRL_LAUNCH_CHECK(what);
+  return SIIRL_OK;
+}
+
+// C = A . B^T with a packed A and K of at most kShortSteps K-steps.  The tiles along N are cut into as many equal runs as
+// make four rounds of the CUs' 512 workgroups, or less where N has fewer tiles.
+template <class Epi>
+int launch_short_k(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_total, int M, int N, int K, const Epi& epi,
+                   hipStream_t st, const char* what) {
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_short_k_kernel<Epi>), kSmemBytes)) return rc;
+  const GemmArgs g{A, lda, Bp, kb_total, M, N, K, (M + BM - 1) / BM, (N + BN - 1) / BN, 1, 1, 0, nullptr, K / BK};
+  if (K > kShortSteps * BK || lda * 32 < (int64_t)g.tiles_m * BM)
+    return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: K=%d or row pitch %lld does not fit %d tiles", what, K, (long long)lda, g.tiles_m);
+  const int64_t want = (4 * 512 + g.tiles_m - 1) / g.tiles_m;  // runs along N
+  const int runs = (int)(want < g.tiles_n ? want : g.tiles_n), n_per = (g.tiles_n + runs - 1) / runs;
+  const int64_t grid = (int64_t)g.tiles_m * ((g.tiles_n + n_per - 1) / n_per);
+  gemm_short_k_kernel<Epi><<<dim3((unsigned)grid), dim3(kThreads), kSmemBytes, st>>>(g, n_per, epi);
   SIIRL_LAUNCH_CHECK(what);
   return SIIRL_OK;
 }
@@ -1265,8 +1360,12 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
       // dW[v0 : v0 + N, H] = D[ldt, N]^T . Ht[H, ldt]^T over the group's vocabulary rows: D is the A operand given by its
       // packed K-rows (tokens)
       StoreEpi sto{(char*)d_weight + v0 * H * (int64_t)dtype_size(dtype), H, N, (int)H, dtype};
-      if (int rc = launch_gemm<StoreEpi, A_PACKED>(reinterpret_cast<const uint16_t*>(D), ws.kb_d, Htp, ws.ldt / 32, N,
-                                                   (int)H, (int)ws.ldt, sto, st, "gemm_nt_kernel<StoreEpi, packed A>", 1, kBlkDWeight))
+      const uint16_t* Da = reinterpret_cast<const uint16_t*>(D);
+      if (int rc = ws.ldt <= kShortSteps * BK
+                       ? launch_short_k(Da, ws.kb_d, Htp, ws.ldt / 32, N, (int)H, (int)ws.ldt, sto, st,
+                                        "gemm_short_k_kernel<StoreEpi>")
+                       : launch_gemm<StoreEpi, A_PACKED>(Da, ws.kb_d, Htp, ws.ldt / 32, N, (int)H, (int)ws.ldt, sto, st,
+                                                         "gemm_nt_kernel<StoreEpi, packed A>", 1, kBlkDWeight))
         return rc;
     }
   }

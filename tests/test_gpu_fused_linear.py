@@ -128,6 +128,26 @@ def test_column_groups_and_k_runs(dev, T, H, V):
     _check_grad(wd.grad, dw64, "d_weight")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T", [1, 64, 65, 129, 192, 193, 256, 257])
+@pytest.mark.parametrize("H,V", [(64, 129), (320, 1000), (576, 70000)])
+def test_few_tokens_weight_gradient(dev, dtype, T, H, V):
+    """d weight with a K of one to four K-steps held in the LDS (up to 256 tokens; 257: the general kernel), row and column
+    remainders of the tiles, one and several runs along H.  Reference: float64 on the GPU."""
+    from siirl_amd.fused_linear import FusedLinearForPPO
+
+    h, w, y, g_lp, g_h = (t.to(dev) for t in _inputs(T, H, V, seed=T + V))
+    h, w = h.to(dtype), w.to(dtype)
+    wd = w.clone().requires_grad_(True)
+    lp, ent = FusedLinearForPPO()(h, wd, y)
+    torch.autograd.backward([lp, ent], [g_lp, g_h])
+    logp = torch.log_softmax(h.double() @ w.double().t().contiguous(), dim=-1)
+    p = logp.exp()
+    d = -g_lp[:, None].double() * p - g_h[:, None].double() * p * (logp - (p * logp).sum(-1)[:, None])
+    d[torch.arange(T, device=dev), y] += g_lp.double()
+    _check_grad(wd.grad, d.t().contiguous() @ h.double(), "d_weight")
+
+
 def test_single_branches_3d_and_linear_cross_entropy(dev):
     from siirl_amd.fused_linear import FusedLinearForPPO, linear_cross_entropy
 
