@@ -672,7 +672,7 @@ int siirl_fused_linear_logprob_entropy_fwd(const void* hidden, const void* weigh
  * d_hidden[T, H] and / or d_weight[V, H] in the operands' dtype (either may be NULL).  The vocabulary is walked in
  * groups of columns: the group's logits are recomputed -- or, when saved_logits holds what the forward call with
  * the same hidden, weight and inv_temperature parked there, read back --, dlogits = inv_T * (g_lp (onehot - p)
- * - g_H p (z - ex)) is written to scratch as bf16 (token-major, one layout for both consumers), then
+ * - g_H p (z - ex)) is written to scratch as bf16 (packed blocks, one layout for both consumers), then
  * d_hidden += dlogits . W_group (fp32 accumulation across groups, rounded once) and d_weight_group = dlogits^T . hidden.
  * Both routes give the same bits.  For SIIRL_F16 and SIIRL_F32 operands the logits are recomputed as in the forward;
  * the two gradient GEMMs multiply the bf16 dlogits (bf16 for its range: a softmax gradient underflows fp16) with

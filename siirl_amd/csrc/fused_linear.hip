@@ -90,7 +90,7 @@ struct TileCoord {
 };
 // XCD-aware rasterisation.  Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2, so
 // workgroup id runs on XCD id % 8 as that XCD's (id / 8)-th workgroup.  The tile grid is cut into blocks of
-// blk_m x blk_n tiles (32 tiles: one XCD's resident set; blk_m is the launch's choice among the powers of two); block b
+// blk_m x blk_n tiles (32 tiles: half of one XCD's resident set; blk_m is the launch's choice among the powers of two); block b
 // goes to XCD b % 8 and its tiles to 32 consecutive workgroups of that XCD, so the workgroups sharing an L2 at any
 // time share blk_m A-tiles and blk_n B-tiles instead of streaming 32 different A-tiles.  Blocks sweep M fastest
 // inside a strip of blk_n N-tiles, which keeps a strip's B-tiles hot across the 8 XCDs.  (Sweeping N fastest instead, which would stream the big
