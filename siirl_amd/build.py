@@ -9,10 +9,13 @@ from __future__ import annotations
 
 import argparse
 import os
+import re
 import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
+
+from . import asm_check
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
@@ -47,6 +50,29 @@ def _filter(stderr: str) -> str:
     return "\n".join(keep)
 
 
+def listing(src: Path) -> Path:
+    """The gfx950 assembly of ``src`` as it is compiled for the library, in ``build/``."""
+    out = PKG / "build" / (src.stem + ".s")
+    out.parent.mkdir(exist_ok=True)
+    cmd = [HIPCC, *CXXFLAGS, *EXTRA.get(src.name, []), "-S", "--cuda-device-only", str(src), "-o", str(out)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"hipcc -S failed on {src}:\n{_filter(r.stderr)}")
+    return out
+
+
+def has_asm_loads(src: Path) -> bool:
+    return re.search(r'asm volatile\("[^"]*_load_', src.read_text()) is not None
+
+
+def check_asm_loads(src: Path) -> None:
+    """Refuses a build whose register allocation uses the target of an inline-assembly load before its wait."""
+    bad = asm_check.check(listing(src).read_text())
+    if bad:
+        raise RuntimeError(f"{src.name}: registers of loads in flight are used: "
+                           + "; ".join(f"{k}: {v[0]} ({len(v)} places)" for k, v in bad.items()))
+
+
 def build(force: bool = False, verbose: bool = True) -> Path:
     LIBDIR.mkdir(exist_ok=True)
     objdir = PKG / "build"
@@ -65,6 +91,7 @@ def build(force: bool = False, verbose: bool = True) -> Path:
         return src, r.returncode, _filter(r.stderr)
 
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
+        checks = [ex.submit(check_asm_loads, src) for src, _ in jobs if has_asm_loads(src)]
         for src, rc, err in ex.map(compile_one, jobs):
             if verbose:
                 print(f"[siirl_amd.build] hipcc {src.name}: {'ok' if rc == 0 else 'FAILED'}", flush=True)
@@ -72,6 +99,8 @@ def build(force: bool = False, verbose: bool = True) -> Path:
                 print(err, file=sys.stderr)
             if rc != 0:
                 raise RuntimeError(f"hipcc failed on {src}")
+        for check in checks:
+            check.result()
     out = LIBDIR / LIBNAME
     objs = [str(objdir / (s.stem + ".o")) for s in sources()]
     if force or jobs or not out.exists():

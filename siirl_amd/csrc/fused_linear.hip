@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   const int64_t to_tail = reinterpret_cast<const char*>(g.A_tail + m0) - (gA + (int64_t)kt_tail * a_step);  // (kt_tail is the last step)
   auto dma = [&](int stage, int kt, int i0 = 0, int i1 = kDmaPerWave) {
     // (No branch around the loads, and no register to spare: where the compiler copies or spills the B registers it does
-    // so before their wait.)
+    // so before their wait.  The build reads its own listing for that, siirl_amd/asm_check.py, and refuses it.)
     const char* base = gA + (int64_t)kt * a_step;
     if (AL == A_KROWS) base += to_tail & (int64_t)__builtin_amdgcn_readfirstlane((kt - kt_tail) >> 31 ^ -1);
 #pragma unroll
