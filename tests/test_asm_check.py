@@ -1,5 +1,7 @@
-"""The check of inline-assembly loads in the compiler's listing (CPU only): what it accepts, what it refuses, and that
-the kernels as they are built here pass."""
+"""What the compiler's listings say (CPU only).  Inline-assembly loads: what the check accepts, what it refuses, and that
+the kernels as they are built here pass.  Log-prob forward: the loads that are meant to be in flight together are."""
+
+import re
 
 import pytest
 
@@ -74,3 +76,15 @@ def test_a_copy_in_the_real_kernel_is_seen(fused_linear):
             out += [";;#ASMEND", f"\tv_mov_b32_e32 v0, v{first}", ";;#ASMSTART"]
     bad = asm_check.check("\n".join(out))
     assert sum("gemm_nt_kernel" in k for k in bad) == 6
+
+
+def test_log_prob_forward_waits_for_no_load_of_the_ragged_end_alone():
+    """Every variant issues the ragged end's four loads together, waits for them and only then branches on what a lane has."""
+    text = build.listing(build.CSRC / "logprob_entropy.hip").read_text()
+    variants = {k: v for k, v in asm_check.kernels(text).items() if "lpe_fwd_kernel" in k}
+    assert len(variants) == 24
+    for name, body in variants.items():
+        marks = "".join("L" if line.startswith("global_load_dwordx4") else "w" if "vmcnt" in line else "e" if "v_exp" in line
+                        else "|" if line.endswith(":") or line.startswith(("s_branch", "s_cbranch")) else ""
+                        for line, _ in body)
+        assert re.search(r"LLLLw+\|", marks), (name, marks)
