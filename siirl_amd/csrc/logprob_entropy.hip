@@ -58,8 +58,10 @@ constexpr int64_t kSkipRow = SIIRL_LABEL_SKIP_ROW;
 #define SIIRL_LPE_BWD_NT_STORE 1
 #endif
 constexpr int kFwdThreads = SIIRL_LPE_FWD_THREADS;  // waves per row = threads / 64
-constexpr int kFwdWideThreads = 1024;               // with few long rows
-constexpr int64_t kWideRows = 256;
+// With no more rows than CUs, a row of more than kDeepTiles tiles of kFwdThreads x kFwdUnroll vectors keeps kRing tiles in
+// flight.  See launch_fwd for where the lines lie.
+constexpr int kRing = 4, kDeepTiles = kRing + 1;
+constexpr int64_t kDeepRows = 256;
 constexpr int kFwdUnroll = SIIRL_LPE_FWD_UNROLL;    // 16-byte loads in flight per lane
 constexpr int kBwdThreads = SIIRL_LPE_BWD_THREADS;
 constexpr int kBwdUnroll = SIIRL_LPE_BWD_UNROLL;
@@ -194,8 +196,10 @@ __device__ __forceinline__ void absorb_vecs(SoftState& st, const u32x4* buf, flo
 
 // NT: the row is streamed with non-temporal loads (worth 12 % when the logits are many times the memory-side cache);
 // without them a tensor that fits that cache is still there when the backward reads it again.
-template <class E, bool ENT, bool NT, int kThreads>
-__global__ __launch_bounds__(kThreads) void lpe_fwd_kernel(const typename E::elem_t* __restrict__ logits,
+// DEEP: kRing tiles of loads in flight instead of one, for rows too few to hide the latency of each other's loads.  The
+// order of the arithmetic is the same, so that a row's outputs do not depend on how many rows the call has.
+template <class E, bool ENT, bool NT, bool DEEP>
+__global__ __launch_bounds__(kFwdThreads) void lpe_fwd_kernel(const typename E::elem_t* __restrict__ logits,
                                                            int64_t row_stride, int V,
                                                            const int64_t* __restrict__ labels, float inv_T,
                                                            float* __restrict__ logprob, float* __restrict__ entropy,
@@ -220,36 +224,68 @@ __global__ __launch_bounds__(kThreads) void lpe_fwd_kernel(const typename E::ele
 
   SoftState st{-1e30f, 0.f, 0.f};
 
-  for (int i = tid; i < sp.head; i += kThreads) absorb1<ENT>(st, E::load1(x + i), k);
-  for (int i = sp.tail0 + tid; i < V; i += kThreads) absorb1<ENT>(st, E::load1(x + i), k);
+  for (int i = tid; i < sp.head; i += kFwdThreads) absorb1<ENT>(st, E::load1(x + i), k);
+  for (int i = sp.tail0 + tid; i < V; i += kFwdThreads) absorb1<ENT>(st, E::load1(x + i), k);
 
   const u32x4* __restrict__ xv = reinterpret_cast<const u32x4*>(x + sp.head);
-  constexpr int kTile = kThreads * kFwdUnroll;
-  const int nfull = sp.nvec / kTile * kTile;
-  for (int base = 0; base < nfull; base += kTile) {
-    u32x4 buf[kFwdUnroll];
+  constexpr int kTile = kFwdThreads * kFwdUnroll;
+  const int ntiles = sp.nvec / kTile, nfull = ntiles * kTile, last = sp.nvec - 1;
+  auto load_tile = [&](u32x4 (&buf)[kFwdUnroll], int t) {
 #pragma unroll
-    for (int u = 0; u < kFwdUnroll; ++u) buf[u] = ld16<NT>(xv + base + u * kThreads + tid);
-    // (fp32: all four loads before the first wait; the scheduler had put the fourth behind it.  [2048, 152064] 187 -> 182 us;
-    // the 16-bit types, with twice the arithmetic per vector, do not gain: [3000, 16000] bf16 22.3 -> 22.7)
-    if constexpr (E::VEC == 4) __builtin_amdgcn_sched_barrier(0);
-    absorb_vecs<E, ENT, kFwdUnroll>(st, buf, k);
-  }
-  if (nfull < sp.nvec) {
-    // The ragged end: every lane loads (past the end: the last vector again), so that all of it is in flight together.
-    // (Loads under a condition each were waited for one by one in the fp16 kernels: [6000, 16000] 34.4 us against 31.5.)
-    u32x4 buf[kFwdUnroll];
-    const int last = sp.nvec - 1;
+    for (int u = 0; u < kFwdUnroll; ++u) buf[u] = ld16<NT>(xv + t * kTile + u * kFwdThreads + tid);
+  };
+  // The ragged end: every lane loads (past the end: the last vector again), so that all of it is in flight together.
+  // (Loads under a condition each were waited for one by one in the fp16 kernels: [6000, 16000] 34.4 us against 31.5.)
+  auto load_end = [&](u32x4 (&buf)[kFwdUnroll]) {
 #pragma unroll
     for (int u = 0; u < kFwdUnroll; ++u) {
-      const int i = nfull + u * kThreads + tid;
+      const int i = nfull + u * kFwdThreads + tid;
       buf[u] = ld16<NT>(xv + (i < last ? i : last));
     }
-#pragma unroll
-    for (int u = 0; u < kFwdUnroll; ++u) asm volatile("" : "+v"(buf[u]));  // (no load moves down to its use)
+  };
+  auto absorb_end = [&](u32x4 (&buf)[kFwdUnroll]) {
 #pragma unroll
     for (int u = 0; u < kFwdUnroll; ++u)
-      if (nfull + u * kThreads + tid <= last) absorb_vecs<E, ENT, 1>(st, buf + u, k);
+      if (nfull + u * kFwdThreads + tid <= last) absorb_vecs<E, ENT, 1>(st, buf + u, k);
+  };
+  u32x4 end[kFwdUnroll];
+  if constexpr (DEEP) {  // (the launch sees to it that there are kRing tiles, whatever the row's alignment)
+    u32x4 ring[kRing][kFwdUnroll];
+    auto fetch = [&](u32x4 (&buf)[kFwdUnroll], int t) {
+      load_tile(buf, t < ntiles ? t : ntiles - 1);
+      __builtin_amdgcn_sched_barrier(0);  // (the loads stay in this order: a wait for one leaves the later ones in flight)
+    };
+#pragma unroll
+    for (int r = 0; r < kRing; ++r) fetch(ring[r], r);
+    const int rest = ntiles % kRing;
+    for (int t0 = 0; t0 < ntiles - rest; t0 += kRing) {
+#pragma unroll
+      for (int r = 0; r < kRing; ++r) {
+        absorb_vecs<E, ENT, kFwdUnroll>(st, ring[r], k);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(ring[r], t0 + r + kRing);
+      }
+    }
+    load_end(end);
+#pragma unroll
+    for (int r = 0; r < kRing - 1; ++r)
+      if (r < rest) absorb_vecs<E, ENT, kFwdUnroll>(st, ring[r], k);
+    absorb_end(end);
+  } else {
+    for (int t = 0; t < ntiles; ++t) {
+      u32x4 buf[kFwdUnroll];
+      load_tile(buf, t);
+      // (fp32: all four loads before the first wait; the scheduler had put the fourth behind it.  [2048, 152064] 187 -> 182 us;
+      // the 16-bit types, with twice the arithmetic per vector, do not gain: [3000, 16000] bf16 22.3 -> 22.7)
+      if constexpr (E::VEC == 4) __builtin_amdgcn_sched_barrier(0);
+      absorb_vecs<E, ENT, kFwdUnroll>(st, buf, k);
+    }
+    if (nfull <= last) {
+      load_end(end);
+#pragma unroll
+      for (int u = 0; u < kFwdUnroll; ++u) asm volatile("" : "+v"(end[u]));  // (no load moves down to its use)
+      absorb_end(end);
+    }
   }
 
   // wave merge
@@ -260,7 +296,7 @@ __global__ __launch_bounds__(kThreads) void lpe_fwd_kernel(const typename E::ele
     const float ot = __shfl_xor(st.t, o, kWave);
     merge(st, omx, os, ot, k);
   }
-  __shared__ float sm[3 * (kThreads / kWave)];
+  __shared__ float sm[3 * (kFwdThreads / kWave)];
   const int lane = tid & (kWave - 1), wid = tid / kWave;
   if (lane == 0) {
     sm[wid * 3 + 0] = st.mx;
@@ -270,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void lpe_fwd_kernel(const typename E::ele
   __syncthreads();
   if (tid == 0) {
 #pragma unroll
-    for (int w = 1; w < kThreads / kWave; ++w) merge(st, sm[w * 3], sm[w * 3 + 1], sm[w * 3 + 2], k);
+    for (int w = 1; w < kFwdThreads / kWave; ++w) merge(st, sm[w * 3], sm[w * 3 + 1], sm[w * 3 + 2], k);
     const float lse = st.mx * inv_T + logf(st.s);
     lse_out[row] = lse;
     if (ENT) {
@@ -739,22 +775,23 @@ int launch_fwd(const void* logits, int64_t T, int V, int64_t row_stride, const i
   // (250 MiB) forward + backward 128 -> 117 us, [768, 152064] bf16 (223 MiB) 114 -> 103 us, the forward alone
   // unchanged; from 375 MiB upwards the non-temporal loads win (forward alone 60 against 70 us at that size).
   const bool nt = SIIRL_LPE_FWD_NT_LOAD && streams_past_cache((double)T * (double)V * (double)sizeof(elem_t));
-  // With no more rows than CUs a row's workgroup has its CU to itself, and four waves keep too few loads in flight: 1024
-  // threads where a row gives each of them four vectors four times.  Forward alone, 256 / 1024 threads (us): V=152064
-  // bf16 32 rows 12.2 / 10.7, 256 rows 18.3 / 15.5, 400 rows 21.9 / 24.4; fp32 128 rows 25.3 / 15.3; V=32000 bf16 32 rows
-  // 5.4 / 5.7, fp32 128 rows 6.9 / 8.0.
-  const bool wide = T <= kWideRows && V / E::VEC >= 4 * kFwdWideThreads * kFwdUnroll;
-  auto launch = [&](auto ent_tag, auto nt_tag, auto threads) {
-    constexpr int kThreads = decltype(threads)::value;
-    lpe_fwd_kernel<E, decltype(ent_tag)::value, decltype(nt_tag)::value, kThreads><<<grid, dim3(kThreads), 0, st>>>(
+  // Few rows: the ring of loads.  Forward alone, one tile / the ring in flight (us) on logits that no cache holds and, in
+  // brackets, on logits that the memory-side cache does.  bf16: V=152064 32 rows 20.6 / 11.7 (12.2 / 11.1), 256 rows
+  // 22.7 / 16.6 (17.1 / 14.6), 384 rows 25.6 / 25.8 (20.7 / 23.3); V=50257 (6 tiles) 32 rows 7.7 / 7.0 (6.9 / 7.0), 256
+  // rows 10.3 / 9.0 (7.2 / 7.2).  fp32: V=152064 32 rows 43.7 / 14.7 (16.7 / 11.6), 300 rows 38.3 / 39.6 (27.8 / 31.8).
+  // Rings of 2, 3, 6 and 8 tiles, 32 rows, V=152064 bf16: 13.0 / 12.2 / 12.7 / 12.8.  1024 threads a row, which makes
+  // a row's bits depend on the number of rows: 13.1 (10.9).
+  const bool deep = T <= kDeepRows && V / E::VEC > kDeepTiles * kFwdThreads * kFwdUnroll;
+  auto launch = [&](auto ent_tag, auto nt_tag, auto deep_tag) {
+    lpe_fwd_kernel<E, decltype(ent_tag)::value, decltype(nt_tag)::value, decltype(deep_tag)::value><<<grid, dim3(kFwdThreads), 0, st>>>(
         (const elem_t*)logits, row_stride, V, labels, inv_T, logprob, decltype(ent_tag)::value ? entropy : nullptr, lse,
         decltype(ent_tag)::value ? ex : nullptr);
   };
   auto go = [&](auto ent_tag, auto nt_tag) {
-    if (wide)
-      launch(ent_tag, nt_tag, std::integral_constant<int, kFwdWideThreads>{});
+    if (deep)
+      launch(ent_tag, nt_tag, std::true_type{});
     else
-      launch(ent_tag, nt_tag, std::integral_constant<int, kFwdThreads>{});
+      launch(ent_tag, nt_tag, std::false_type{});
   };
   using Yes = std::true_type;
   using No = std::false_type;

@@ -72,9 +72,12 @@ def test_forward_backward_matches_oracle(dev, dtype, T, V):
 
 
 @pytest.mark.parametrize("dtype,T,V", [(torch.bfloat16, 3, 131071), (torch.bfloat16, 3, 131072), (torch.bfloat16, 2, 163843),
-                                       (torch.float32, 2, 65536), (torch.float32, 256, 65540), (torch.float32, 257, 65540)])
+                                       (torch.float32, 2, 65536), (torch.float32, 256, 65540), (torch.float32, 257, 65540),
+                                       (torch.float16, 3, 40960), (torch.float16, 3, 40968), (torch.bfloat16, 3, 49159),
+                                       (torch.float32, 3, 20484), (torch.float32, 3, 24580)])
 def test_forward_few_long_rows(dev, dtype, T, V):
-    """Both sides of the line between four and sixteen waves a row, with ragged ends and rows of every alignment."""
+    """Both sides of the lines (256 rows, five tiles of loads) between one tile of loads in flight and a ring of four, every
+    remainder of the ring, with ragged ends and rows of every alignment."""
     import siirl_amd.torch_functional as SF
 
     x, y = _make(T, V, dtype, seed=T + V)
@@ -82,6 +85,23 @@ def test_forward_few_long_rows(dev, dtype, T, V):
     logp = torch.log_softmax(x.to(dev).double(), dim=-1)
     assert (lp.double() - logp.gather(-1, y.to(dev)[:, None]).squeeze(-1)).abs().max() < 1e-4
     assert (ent.double() + (logp.exp() * logp).sum(-1)).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 40960), (torch.bfloat16, 40968), (torch.bfloat16, 152064),
+                                     (torch.bfloat16, 131071), (torch.float16, 152064), (torch.float16, 65537),
+                                     (torch.float32, 20484), (torch.float32, 90001)])
+def test_a_row_does_not_depend_on_the_number_of_rows(dev, dtype, V):
+    """Log-probs scored in a small call equal, bit for bit, those of the same rows in a large one."""
+    import siirl_amd.torch_functional as SF
+
+    rows = 40 + 400_000_000 // (V * dtype.itemsize)  # the large call streams past the memory-side cache as well
+    x = torch.empty(rows, V, dtype=dtype, device=dev).normal_(0.0, 3.0, generator=torch.Generator(dev).manual_seed(V))
+    y = torch.randint(0, V, (rows,), device=dev, generator=torch.Generator(dev).manual_seed(V + 1))
+    lp, ent = SF.logprobs_and_entropy_from_logits(x, y)
+    for n in (1, 7, 256, 257):
+        n = min(n, rows)
+        lp_n, ent_n = SF.logprobs_and_entropy_from_logits(x[:n].clone(), y[:n])
+        assert torch.equal(lp_n, lp[:n]) and torch.equal(ent_n, ent[:n]), n
 
 
 @pytest.mark.parametrize("temperature", [0.6, 1.0, 1.7])
