@@ -5,12 +5,12 @@
 //
 // The scan is the reference's recurrence, evaluated per row in the same float32 operation order (this file is
 // compiled with -ffp-contract=off, so no multiply-add is fused and the un-whitened advantages and the returns
-// are bit-identical to the reference's):
+// equal the reference's; the sign of a zero may differ):
 //   delta = r_t + gamma * V_next - V_t ;  cand = delta + (gamma * lam) * A_next
 //   V_next <- V_t * m_t + (1 - m_t) * V_next ;  A_next <- cand * m_t + (1 - m_t) * A_next ;  A_t = A_next
 // The recurrence is sequential, so the time of one row is the latency of its chain; everything that is not the chain is
 // taken off it (gae_scan_kernel).  A scan over chunks of rows stitched through affine maps is there for callers that
-// do not need the reference's order (gae_compose_kernel, gae_carry_kernel).
+// do not need the reference's order (MODE_COMPOSE, gae_carry_kernel).
 #include "common.hpp"
 #include "loss_token.hpp"
 
@@ -108,8 +108,7 @@ __device__ __forceinline__ void load_mask_pieces(const void* mask, int64_t idx, 
 // differ in their sign.)  A workgroup owns four rows in tiles of 128 columns, right to left.  Its first wave walks the
 // chain, a row per lane; two more waves fetch the tiles four ahead (16-byte loads), prepare d and k a tile ahead and
 // store the tile behind with its whitening statistics.  Four rows per workgroup: 256 workgroups at B = 1024.
-// B = 1024, L = 8192, int64 mask: 91 us (2.6 TB/s); one wave per 16 rows that also loaded, converted and stored was 508 us
-// (149 cycles a token).
+// B = 1024, L = 8192, int64 mask: 91 us (2.6 TB/s), gae_rows_kernel 508 us (149 cycles a token).
 // A tile with another mask value, or with a delta that is not finite and moderate, or that takes A out of the finite
 // numbers, is walked by the recurrence as it stands, and so is the rest of those rows (`slow`).
 constexpr int kScanRows = 4, kScanHelpers = kScanRows * kCols / 4, kScanThreads = kWave + kScanHelpers, kAhead = 4;
@@ -299,16 +298,22 @@ __global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __r
   }
 }
 
-// Folds each row's tokens into one GaeMap, written to `maps`.  With rows that are chunks of the real rows (B = rows x
-// chunks, L = chunk length: chunks of a row are adjacent in memory) this pass, a carry over the chunk maps and a scan
-// pass evaluate the recurrence with a dependent chain of one chunk instead of one row.  One wave per 16 rows; the next
-// tile's loads are in flight while a tile, passed through LDS, is folded.
-template <int MK, bool F32MASK>
-__global__ __launch_bounds__(kWave) void gae_compose_kernel(const float* __restrict__ rewards,
-                                                            const float* __restrict__ values,
-                                                            const void* __restrict__ mask, int64_t B, int64_t L,
-                                                            float gamma, float gamma_lam, float* __restrict__ maps) {
-  __shared__ __align__(16) float s_r[kRows * kPitch], s_v[kRows * kPitch], s_m[kRows * kPitch];
+enum { MODE_SCAN = 0, MODE_COMPOSE = 1 };
+
+// One wave per 16 rows, which loads, converts, walks and stores by itself: the next tile's loads are in flight while a
+// tile, passed through LDS, is walked.  16 rows a wave and 64 a CU make it a stream where there are rows enough.
+// MODE_SCAN: the recurrence itself, from the state `init` gives each row (zero when null).  MODE_COMPOSE: no output
+// per token; each row's tokens are folded into one GaeMap written to `maps`.  With rows that are chunks of the real
+// rows (B = rows x chunks, L = chunk length: chunks of a row are adjacent in memory) a compose pass, a carry over
+// the chunk maps and a scan pass evaluate the recurrence with a dependent chain of one chunk instead of one row.
+template <int MK, bool F32MASK, int MODE>
+__global__ __launch_bounds__(kWave) void gae_rows_kernel(const float* __restrict__ rewards,
+                                                         const float* __restrict__ values,
+                                                         const void* __restrict__ mask, int64_t B, int64_t L,
+                                                         float gamma, float gamma_lam, float* __restrict__ adv,
+                                                         float* __restrict__ ret, double* __restrict__ part,
+                                                         const float* __restrict__ init, float* __restrict__ maps) {
+  __shared__ __align__(16) float s_r[kRows * kPitch], s_v[kRows * kPitch], s_m[kRows * kPitch], s_a[kRows * kPitch];
   const int lane = threadIdx.x;
   const int64_t row0 = (int64_t)blockIdx.x * kRows;
   const int nrows = (int)((B - row0) < kRows ? (B - row0) : kRows);
@@ -337,37 +342,84 @@ __global__ __launch_bounds__(kWave) void gae_compose_kernel(const float* __restr
       *reinterpret_cast<float4*>(s_m + o) = mask_quad<MK, F32MASK>(pa[k], pb[k]);
     }
   };
+  float nv = 0.f, lg = 0.f;
+  if (MODE == MODE_SCAN && init != nullptr && lane < nrows) {
+    nv = init[2 * (row0 + lane)];
+    lg = init[2 * (row0 + lane) + 1];
+  }
   GaeMap gm{1.f, 0.f, 1.f, 0.f, 0.f};
+  double st[kNStat] = {0.0, 0.0, 0.0};  // whitening statistics of this wave's advantages (pivot 0)
   const int64_t c_last = (L - 1) / kCols * kCols;
   issue(c_last);
   for (int64_t c0 = c_last; c0 >= 0; c0 -= kCols) {
     const int ncols = (int)((L - c0) < kCols ? (L - c0) : kCols);  // a multiple of 4
     commit();  // waits for this tile's loads
-    if (c0 > 0) issue(c0 - kCols);  // in flight while this tile is folded
+    if (c0 > 0) issue(c0 - kCols);  // in flight while this tile is walked
     __syncthreads();
     if (lane < nrows) {
       const float* r4 = s_r + lane * kPitch;
       const float* v4 = s_v + lane * kPitch;
       const float* m4 = s_m + lane * kPitch;
-      // the LDS reads of the next four tokens are issued before the current four are folded
+      // the LDS reads of the next four tokens are issued before the current four are walked
       float4 r = *reinterpret_cast<const float4*>(r4 + ncols - 4), v = *reinterpret_cast<const float4*>(v4 + ncols - 4),
              m = *reinterpret_cast<const float4*>(m4 + ncols - 4);
       for (int cc = ncols - 4; cc >= 0; cc -= 4) {
         const int nx = cc >= 4 ? cc - 4 : 0;
         const float4 rn = *reinterpret_cast<const float4*>(r4 + nx), vn = *reinterpret_cast<const float4*>(v4 + nx),
                      mn = *reinterpret_cast<const float4*>(m4 + nx);
-        gae_compose(r.w, v.w, m.w, gamma, gamma_lam, gm);
-        gae_compose(r.z, v.z, m.z, gamma, gamma_lam, gm);
-        gae_compose(r.y, v.y, m.y, gamma, gamma_lam, gm);
-        gae_compose(r.x, v.x, m.x, gamma, gamma_lam, gm);
+        if (MODE == MODE_SCAN) {
+          float4 a;
+          gae_step(r.w, v.w, m.w, gamma, gamma_lam, nv, lg); a.w = lg;
+          gae_step(r.z, v.z, m.z, gamma, gamma_lam, nv, lg); a.z = lg;
+          gae_step(r.y, v.y, m.y, gamma, gamma_lam, nv, lg); a.y = lg;
+          gae_step(r.x, v.x, m.x, gamma, gamma_lam, nv, lg); a.x = lg;
+          *reinterpret_cast<float4*>(s_a + lane * kPitch + cc) = a;
+        } else {
+          gae_compose(r.w, v.w, m.w, gamma, gamma_lam, gm);
+          gae_compose(r.z, v.z, m.z, gamma, gamma_lam, gm);
+          gae_compose(r.y, v.y, m.y, gamma, gamma_lam, gm);
+          gae_compose(r.x, v.x, m.x, gamma, gamma_lam, gm);
+        }
         r = rn; v = vn; m = mn;
       }
     }
-    __syncthreads();  // the next commit overwrites the tile
+    __syncthreads();
+    if (MODE == MODE_SCAN) {
+#pragma unroll
+      for (int k = 0; k < kChunks; ++k) {
+        const int q = lane + kWave * k, rr = q / (kCols / 4), ch = q % (kCols / 4);
+        const int64_t col = c0 + 4 * ch;
+        if (rr < nrows && col < L) {
+          const int64_t idx = (row0 + rr) * L + col;
+          const float4 a = *reinterpret_cast<const float4*>(s_a + rr * kPitch + 4 * ch);
+          const float4 v = *reinterpret_cast<const float4*>(s_v + rr * kPitch + 4 * ch);
+          *reinterpret_cast<float4*>(adv + idx) = a;
+          *reinterpret_cast<float4*>(ret + idx) = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
+          if (part) {
+            const float4 m = *reinterpret_cast<const float4*>(s_m + rr * kPitch + 4 * ch);
+            stat_add(st, a.x, m.x, 0.0);
+            stat_add(st, a.y, m.y, 0.0);
+            stat_add(st, a.z, m.z, 0.0);
+            stat_add(st, a.w, m.w, 0.0);
+          }
+        }
+      }
+      __syncthreads();  // the next commit overwrites s_v / s_m / s_a
+    }
   }
-  if (lane < nrows) {
-    float* o = maps + 5 * (row0 + lane);
-    o[0] = gm.a00; o[1] = gm.a10; o[2] = gm.a11; o[3] = gm.b0; o[4] = gm.b1;
+  if (MODE == MODE_COMPOSE) {
+    if (lane < nrows) {
+      float* o = maps + 5 * (row0 + lane);
+      o[0] = gm.a00; o[1] = gm.a10; o[2] = gm.a11; o[3] = gm.b0; o[4] = gm.b1;
+    }
+    return;
+  }
+  if (part) {
+#pragma unroll
+    for (int k = 0; k < kNStat; ++k) {
+      const double t = wave_sum(st[k]);
+      if (lane == 0) part[(int64_t)kNStat * blockIdx.x + k] = t;
+    }
   }
 }
 
@@ -431,8 +483,7 @@ __global__ __launch_bounds__(kWave) void gae_scan_any_kernel(const float* __rest
 // ---------------------------------------------------------------------------- masked whitening
 
 constexpr int kThreads = 256;
-constexpr int kMaxParts = 8192;      // workgroups of whiten_stats_kernel
-constexpr int kWhitenSlots = 32768;  // partials that the workspace holds: the scan's workgroups of 131072 rows
+constexpr int kMaxParts = 8192;
 __global__ __launch_bounds__(kThreads) void whiten_stats_kernel(const float* __restrict__ v, const void* mask,
                                                                 int mask_dtype, int64_t n, int vec,
                                                                 double* __restrict__ part) {
@@ -505,7 +556,7 @@ int check_mask(int dt) {
   return SIIRL_OK;
 }
 
-constexpr size_t kWhitenWs = (size_t)kWhitenSlots * kNStat * sizeof(double);
+constexpr size_t kWhitenWs = (size_t)kMaxParts * kNStat * sizeof(double);
 
 int check_whiten_ws(const void* ws, size_t ws_bytes) {
   if (ws == nullptr || ws_bytes < kWhitenWs)
@@ -571,28 +622,50 @@ extern "C" size_t siirl_gae_workspace_bytes(int64_t B, int64_t L) {
   return B < 1 ? 0 : gae_ws_bytes(B);
 }
 
+// Which scan.  gae_scan_kernel gives a row's chain a wave that does nothing else, but a CU holds only 8 rows of it (16
+// with masks of up to four bytes: registers), and a workgroup pays four intervals however short its rows are;
+// gae_rows_kernel holds 64 rows a CU and streams.  So the first for up to three rounds of long rows (two, with the narrower
+// masks), the second beyond, and for rows of one tile from the end of the first round on.  GAE with whitening, first /
+// second (us), int64 mask: [1024, 128] 14.8 / 17.2, [2048, 128] 15.4 / 17.4, [3072, 128] 18.6 / 17.7, [4096, 32] 19.3 / 14.7,
+// [6144, 256] 30.2 / 31.9, [6144, 8192] 384 / 589, [8192, 256] 38.5 / 33.7, [8192, 1024] 90.3 / 90.5, [8192, 8192] 506 / 616,
+// [12000, 256] 53.5 / 36.1, [131072, 32] 382 / 77; in chunks of rows [1024, 8192] 161 / 118, [5488, 8192] 753 / 488.
+// float32 mask: [3072, 128] 16.2 / 17.1, [4096, 64] 16.4 / 14.7, [8192, 256] 31.0 / 32.2, [8192, 4096] 222 / 291, [12000, 256]
+// 40.7 / 32.4.  (Masks of other values than 0 and 1 would rather have the second from 3000 rows on, [4096, 8192] 554 / 494.)
+static bool few_rows(int64_t rows, int64_t len, bool mask64) {
+  if (len <= kCols) return rows <= (mask64 ? 2048 : 3072);
+  return rows <= (mask64 && len < 1024 ? 6144 : 8192);
+}
+
 template <int MK, bool F32MASK>
 static int launch_gae_vec(const float* rewards, const float* values, const void* mask, int64_t B, int64_t L, float g,
                           float gl, float* adv, float* ret, void* ws, int chunks, int* parts_ready, hipStream_t st) {
   const int64_t rows = B * chunks, len = L / chunks;
-  const dim3 grid((unsigned)((rows + kScanRows - 1) / kScanRows));
+  const bool few = few_rows(rows, len, MK == MK_I64);
+  const dim3 grid16((unsigned)((rows + kRows - 1) / kRows));
+  const dim3 grid = few ? dim3((unsigned)((rows + kScanRows - 1) / kScanRows)) : grid16;
   // the scan leaves its whitening statistics in the workspace, one partial per workgroup, when they fit
-  const bool fused_stats = grid.x <= (unsigned)kWhitenSlots;
+  const bool fused_stats = grid.x <= (unsigned)kMaxParts;
   double* part = fused_stats ? (double*)ws : nullptr;
   *parts_ready = fused_stats ? (int)grid.x : 0;
   const float* init = nullptr;
   if (chunks > 1) {
     float* maps = reinterpret_cast<float*>((char*)ws + kWhitenWs);
     float* ini = maps + (size_t)rows * 5;
-    gae_compose_kernel<MK, F32MASK><<<dim3((unsigned)((rows + kRows - 1) / kRows)), dim3(kWave), 0, st>>>(
-        rewards, values, mask, rows, len, g, gl, maps);
-    SIIRL_LAUNCH_CHECK("gae_compose_kernel");
+    gae_rows_kernel<MK, F32MASK, MODE_COMPOSE><<<grid16, dim3(kWave), 0, st>>>(rewards, values, mask, rows, len, g, gl, nullptr,
+                                                                             nullptr, nullptr, nullptr, maps);
+    SIIRL_LAUNCH_CHECK("gae_rows_kernel<MODE_COMPOSE>");
     gae_carry_kernel<<<dim3((unsigned)((B + 255) / 256)), dim3(256), 0, st>>>(maps, B, chunks, ini);
     SIIRL_LAUNCH_CHECK("gae_carry_kernel");
     init = ini;
   }
-  gae_scan_kernel<MK, F32MASK><<<grid, dim3(kScanThreads), 0, st>>>(rewards, values, mask, rows, len, g, gl, adv, ret, part, init);
-  SIIRL_LAUNCH_CHECK("gae_scan_kernel");
+  if (few) {
+    gae_scan_kernel<MK, F32MASK><<<grid, dim3(kScanThreads), 0, st>>>(rewards, values, mask, rows, len, g, gl, adv, ret, part, init);
+    SIIRL_LAUNCH_CHECK("gae_scan_kernel");
+  } else {
+    gae_rows_kernel<MK, F32MASK, MODE_SCAN><<<grid, dim3(kWave), 0, st>>>(rewards, values, mask, rows, len, g, gl, adv, ret, part,
+                                                                        init, nullptr);
+    SIIRL_LAUNCH_CHECK("gae_rows_kernel<MODE_SCAN>");
+  }
   return SIIRL_OK;
 }
 

@@ -55,6 +55,13 @@ def test_every_entry_point_cites_the_reference():
         assert "Replaces:" in comment and re.search(r"siirl/[\w/]+\.py:\d+", comment), f"{n} lacks a reference citation"
 
 
+def test_whitening_scratch_is_what_it_was():
+    """Three doubles for each of 8192 partials, whatever the problem: callers may have laid it out once."""
+    h = _lib().lib()
+    assert h.siirl_whiten_workspace_bytes() == 8192 * 3 * 8
+    assert h.siirl_gae_workspace_bytes(1, 8192) == h.siirl_gae_workspace_bytes(1, 4)
+
+
 def test_argument_validation_without_gpu():
     L = _lib()
     h = L.lib()
