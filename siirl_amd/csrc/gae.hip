@@ -176,7 +176,8 @@ __global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __r
 #pragma unroll
             for (int q = 0; q < 4; ++q) dc[q] = dn[q], kc[q] = kn[q];
           }
-          // an overflow stays: a tile that ends finite was finite throughout
+          // An overflow stays: a tile that ends finite was finite throughout.  Only a state that `init` brings can do this
+          // (chunks of rows): from zero, deltas of at most 1e30 take 3e8 tokens to leave the finite numbers.
           if (__builtin_amdgcn_ballot_w64(!(lg - lg == 0.f)) != 0) slow = true, lg = entering;
         }
         if (slow) {

@@ -78,7 +78,7 @@ def test_gae(dev, B, L, kind, mdt, gamma, lam):
     assert (adv.cpu() - adv32).abs().max() < 1e-3
 
 
-@pytest.mark.parametrize("case", ["holes", "empty-rows", "fractional-late", "nan-padding", "inf-reward", "overflow",
+@pytest.mark.parametrize("case", ["holes", "empty-rows", "fractional-late", "nan-padding", "inf-reward", "large",
                                   "huge-value", "growing"])
 @pytest.mark.parametrize("B,L", [(1, 4), (3, 128), (5, 132), (4, 260), (9, 1156)])
 def test_gae_scan_paths(dev, B, L, case):
@@ -100,7 +100,7 @@ def test_gae_scan_paths(dev, B, L, case):
         m[b, at], v[b, at] = 0.0, float("nan")
     elif case == "inf-reward":
         r[b, at] = float("inf")
-    elif case == "overflow":  # A leaves the finite numbers although every delta is below 1e30
+    elif case == "large":  # every delta just below what the two-operation chain takes, A up to 1e33
         r[b], gamma, lam = 9e29, 1.0, 1.0
     elif case == "huge-value":
         v[b, at] = 3e38
@@ -112,6 +112,47 @@ def test_gae_scan_paths(dev, B, L, case):
     if case in ("holes", "empty-rows", "fractional-late"):
         adv64, _ = OC.compute_gae_advantage_return(r.double(), v.double(), m.double(), gamma, lam)
         assert (adv.cpu().double() - adv64).abs().max() <= 1e-4  # fp32 scan, then the division by the deviation
+
+
+@pytest.mark.parametrize("case", ["fractional", "nan-padding", "inf-reward", "minus-inf-reward", "huge-value", "growing"])
+@pytest.mark.parametrize("B,L", [(1, 1024), (3, 4096), (5, 8192)])
+def test_gae_chunked_scan_paths(dev, B, L, case):
+    """The chunked order where the two-operation chain does not hold, from the state that a chunk is entered with on: a
+    non-finite state carried into the chunks to the left, values beyond 1e30, other mask values, |gamma * lam| > 1."""
+    import siirl_amd.core_algos as CA
+
+    g = torch.Generator().manual_seed(B * 10000 + L)
+    r, v = torch.randn(B, L, generator=g), torch.randn(B, L, generator=g)
+    m = (torch.rand(B, L, generator=g) < 0.7).float()
+    m[:, 0], m[:, -1] = 1.0, 1.0
+    gamma, lam = 0.99, 0.95
+    b, at = B // 2, 2 * L // 3
+    if case == "fractional":
+        m[b, at] = 0.5
+    elif case == "nan-padding":
+        m[b, at], v[b, at] = 0.0, float("nan")
+    elif case == "inf-reward":
+        m[b, at], r[b, at] = 1.0, float("inf")
+    elif case == "minus-inf-reward":
+        m[b, at], r[b, at] = 1.0, float("-inf")
+    elif case == "huge-value":
+        m[b, at], v[b, at] = 1.0, 3e38
+    elif case == "growing":  # (a gamma that float32 holds exactly)
+        gamma, lam = 1.0 + 2.0 ** -9, 1.0
+    try:
+        CA.set_gae_scan_order("chunked")
+        _, ret = CA.compute_gae_advantage_return(r.to(dev), v.to(dev), m.to(dev), gamma, lam)
+    finally:
+        CA.set_gae_scan_order("exact")
+    ret = ret.cpu()
+    _, ret32 = OC.gae_unwhitened(r, v, m, gamma, lam)
+    raw64, ret64 = OC.gae_unwhitened(r.double(), v.double(), m.double(), gamma, lam)
+    finite = torch.isfinite(ret32)
+    assert torch.equal(torch.isfinite(ret), finite)
+    scale = raw64.abs().nan_to_num(0.0, 0.0, 0.0).amax(dim=1, keepdim=True) + 1.0
+    # growing: no error is damped, and each of a row's tokens may add its three roundings of 2^-24 of the largest magnitude
+    tol = 3 * L * 2.0 ** -24 if case == "growing" else 1e-5
+    assert bool(((ret.double() - ret64).abs() <= tol * scale)[finite].all())
 
 
 @pytest.mark.parametrize("B,L,mdt", [(2048, 128, torch.int64), (2049, 128, torch.int64), (2049, 132, torch.int64),
