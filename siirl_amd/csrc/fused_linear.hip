@@ -1017,18 +1017,20 @@ constexpr int kBlkFwd = 4, kBlkRecompute = 2, kBlkDHidden = 4, kBlkDWeight = 8;
 // tiles at T=200 a fraction of one (18 runs: 504 workgroups).  The run count is the one with the least time by
 // the kernel's measured 1.2 us per K-step of the two tiles on a CU and about 12 us per tile besides, plus the buffers' write and read at 5 TB/s.
 constexpr int kMaxSplits = 64;
-constexpr double kSplitBytes = 512.0 * 1048576.0;  // bound on the buffers beyond two
+constexpr double kSplitBytes = 512.0 * 1048576.0;  // bound on the buffers of more than two runs
 // Up to 1024 tokens the choice does not look at T (it is the one for a single token tile; at T=1024, H=3584, K=152064
 // 18 runs model as 786 us against 710 us for the best 9), so that a row of d hidden keeps its bits whatever other rows
-// a small batch holds.
+// a small batch holds.  The bound is then that of the 1024.
+constexpr int64_t kSplitSameTokens = 1024;
 inline int pick_splits(int64_t T, int64_t H, int64_t K) {
-  if (T <= 1024) T = BN;
+  const int64_t most = T <= kSplitSameTokens ? kSplitSameTokens : T;
+  if (T <= kSplitSameTokens) T = BN;
   const int64_t tiles = ((T + BN - 1) / BN) * ((H + BM - 1) / BM), KT = K / BK;
   int best = 1;
   double best_us = 0.;
   for (int s = 1; s <= kMaxSplits && s <= KT; ++s) {
     const double bytes = 4.0 * (double)T * (double)H * s;
-    if (s > 2 && bytes > kSplitBytes) break;
+    if (s > 2 && 4.0 * (double)most * (double)H * s > kSplitBytes) break;
     const int64_t per = (KT + s - 1) / s;
     if ((s - 1) * per >= KT) continue;  // the last run would be empty
     const double us = (double)((tiles * s + 511) / 512) * (1.2 * (double)per + 12.0) + 2.0 * bytes / 5e6;

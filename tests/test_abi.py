@@ -62,6 +62,17 @@ def test_whitening_scratch_is_what_it_was():
     assert h.siirl_gae_workspace_bytes(1, 8192) == h.siirl_gae_workspace_bytes(1, 4)
 
 
+@pytest.mark.parametrize("T", [1, 256, 1024, 1025, 4096])
+@pytest.mark.parametrize("H,V", [(64, 152064), (3584, 152064), (13312, 262144), (14848, 262144), (65536, 152064)])
+def test_d_hidden_buffers_are_bounded(T, H, V):
+    """More than two fp32 buffers of d hidden take 512 MiB at most, also where one choice serves all up to 1024 tokens."""
+    h = _lib().lib()
+    with_dh, without = (h.siirl_fused_linear_bwd_workspace_bytes(T, H, V, dh, 0) for dh in (1, 0))
+    one = (T * H * 4 + 255) // 256 * 256
+    assert (with_dh - without) % one == 0 and with_dh - without >= one
+    assert with_dh - without <= max(2 * one, 512 * 2 ** 20)
+
+
 def test_argument_validation_without_gpu():
     L = _lib()
     h = L.lib()
