@@ -54,9 +54,9 @@ def test_fused_matches_oracle(dev, T, H, V, temperature):
 
 
 def test_fused_random_shapes_sweep(dev):
-    """Seeded random token counts, hidden sizes and vocabulary sizes (around the 256-row tile, the 8192-column slab and
-    the 65536-column group boundaries as well as arbitrary ones), temperatures, and which of the two gradients flows,
-    on both backward routes.  ``SIIRL_TEST_SEED=<int>`` in the environment shifts the seeds."""
+    """Seeded random token counts, hidden sizes and vocabulary sizes (around the tile edges and powers of two as well as
+    arbitrary ones; all of one column group), temperatures, and which of the two gradients flows, on both backward
+    routes.  ``SIIRL_TEST_SEED=<int>`` in the environment shifts the seeds."""
     import random
 
     from siirl_amd import fused_linear as FL
@@ -100,30 +100,98 @@ def test_fused_random_shapes_sweep(dev):
         FL.set_saved_logits_limit(0)
 
 
+def _group_columns(T):
+    """Vocabulary columns of one group of the backward: 65536 at 16384 tokens (padded to 64), and as many times more with
+    fewer tokens, up to 64."""
+    return 65536 * max(1, min(64, 16384 // (-(-T // 64) * 64)))
+
+
+def _float64_reference(h, w, y, g_lp, g_h):
+    """log-prob, entropy and both gradients in float64 on the GPU, 2048 tokens at a time."""
+    h64, w64 = h.double(), w.double()
+    lp64, ent64, dh64, dw64 = [], [], [], torch.zeros_like(w64)
+    for lo in range(0, h.shape[0], 2048):
+        rows = slice(lo, lo + 2048)
+        logp = torch.log_softmax(h64[rows] @ w64.t().contiguous(), dim=-1)
+        p = logp.exp()
+        ent64.append(-(p * logp).sum(-1))
+        lp64.append(logp.gather(-1, y[rows, None]).squeeze(-1))
+        d = -g_lp[rows, None].double() * p - g_h[rows, None].double() * p * (logp + ent64[-1][:, None])
+        d[torch.arange(d.shape[0], device=d.device), y[rows]] += g_lp[rows].double()
+        dh64.append(d @ w64)
+        dw64 += d.t().contiguous() @ h64[rows]
+    return torch.cat(lp64), torch.cat(ent64), torch.cat(dh64), dw64
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,groups,more", [(8200, 64, 1, 257), (8200, 128, 1, 1), (8200, 64, 2, 70), (5500, 64, 1, 130),
+                                             (16448, 64, 1, 64)])
+def test_several_column_groups(dev, dtype, T, H, groups, more):
+    """Vocabularies of two and three column groups, the last one shallow and mostly ragged, in every operand dtype: the
+    gradients against float64, and the route that reads parked logits against the one that recomputes them, bit for bit."""
+    import siirl_amd.fused_linear as FL
+    from siirl_amd import _lib
+
+    def scratch(V):
+        return _lib.lib().siirl_fused_linear_bwd_workspace_bytes(T, H, V, 0, 0)
+
+    group = _group_columns(T)
+    assert scratch(group - 256) < scratch(group) == scratch(group + 4096)  # the dlogits of one group and no more
+    V = groups * group + more
+    h, w, y, g_lp, g_h = (t.to(dev) for t in _inputs(T, H, V, seed=T + V))
+    h, w = h.to(dtype), w.to(dtype)
+    out = {}
+    try:
+        for limit in (0, 1 << 40):
+            FL.set_saved_logits_limit(limit)
+            hd, wd = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
+            lp, ent = FL.fused_linear_logprob_entropy(hd, wd, y)
+            torch.autograd.backward([lp, ent], [g_lp, g_h])
+            out[limit] = lp.detach(), ent.detach(), hd.grad, wd.grad
+    finally:
+        FL.set_saved_logits_limit(0)
+    assert all(torch.equal(a, b) for a, b in zip(*out.values()))
+    lp, ent, dh, dw = out[0]
+    lp64, ent64, dh64, dw64 = _float64_reference(h, w, y, g_lp, g_h)
+    assert (lp.double() - lp64).abs().max() < 1e-4 and (ent.double() - ent64).abs().max() < 1e-4
+    _check_grad(dh, dh64, "d_hidden")
+    _check_grad(dw, dw64, "d_weight")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_left_out_with_several_column_groups(dev, rows_left_out, dtype):
+    """More than 8192 live rows, two column groups: what the plain backward gives on the gathered rows, bit for bit."""
+    import siirl_amd.fused_linear as FL
+
+    T, H = 9000, 64
+    live = torch.arange(T, device=dev) % 12 != 5
+    n = int(live.sum())
+    V = _group_columns(n) + 257
+    assert n > 8192 and _group_columns(n) == 65536
+    h, w, y, g_lp, g_h = (t.to(dev) for t in _inputs(T, H, V, seed=T))
+    h, w, g_lp, g_h = h.to(dtype), w.to(dtype), g_lp * live, g_h * live
+    hd, wd = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    torch.autograd.backward(list(FL.fused_linear_logprob_entropy(hd, wd, y)), [g_lp, g_h])
+    FL.set_skip_zero_rows(False)
+    hc, wc = h[live].clone().requires_grad_(True), w.clone().requires_grad_(True)
+    torch.autograd.backward(list(FL.fused_linear_logprob_entropy(hc, wc, y[live])), [g_lp[live], g_h[live]])
+    assert torch.equal(hd.grad[live], hc.grad) and torch.equal(wd.grad, wc.grad)
+    assert not hd.grad[~live].any()
+
+
 @pytest.mark.parametrize("T,H,V", [(8200, 64, 65793), (8192, 128, 70000), (200, 320, 40000), (31, 64, 131073),
                                    (257, 448, 33003)])
 def test_column_groups_and_k_runs(dev, T, H, V):
-    """Vocabularies of more than one column group (8192 tokens and more: 65536 columns; the last group is shallower than
-    the first, down to 5 K-steps), and d hidden summed from many K runs (few token tiles).  Reference: float64 on the GPU."""
+    """d hidden summed from many K runs (few token tiles) and over two column groups (the first case; the others are one).
+    Reference: float64 on the GPU."""
     from siirl_amd.fused_linear import FusedLinearForPPO
 
     h, w, y, g_lp, g_h = (t.to(dev) for t in _inputs(T, H, V, seed=T + V))
     hd, wd = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
     lp, ent = FusedLinearForPPO()(hd, wd, y)
     torch.autograd.backward([lp, ent], [g_lp, g_h])
-    h64, w64 = h.double(), w.double()
-    dh64, dw64 = torch.empty_like(h64), torch.zeros_like(w64)
-    for lo in range(0, T, 2048):
-        rows = slice(lo, min(lo + 2048, T))
-        logp = torch.log_softmax(h64[rows] @ w64.t().contiguous(), dim=-1)
-        p = logp.exp()
-        ent64 = -(p * logp).sum(-1)
-        lp64 = logp.gather(-1, y[rows, None]).squeeze(-1)
-        assert (lp[rows].double() - lp64).abs().max() < 1e-4 and (ent[rows].double() - ent64).abs().max() < 1e-4
-        d = -g_lp[rows, None].double() * p - g_h[rows, None].double() * p * (logp + ent64[:, None])
-        d[torch.arange(d.shape[0], device=dev), y[rows]] += g_lp[rows].double()
-        dh64[rows] = d @ w64
-        dw64 += d.t().contiguous() @ h64[rows]
+    lp64, ent64, dh64, dw64 = _float64_reference(h, w, y, g_lp, g_h)
+    assert (lp.double() - lp64).abs().max() < 1e-4 and (ent.double() - ent64).abs().max() < 1e-4
     _check_grad(hd.grad, dh64, "d_hidden")
     _check_grad(wd.grad, dw64, "d_weight")
 
@@ -526,7 +594,7 @@ def test_fp16_and_fp32_operands(dev, dtype, T, H, V):
 
 def test_fp16_and_fp32_random_shapes_sweep(dev):
     """Seeded random shapes with float16 / float32 operands on both backward routes (recompute and parked logits),
-    around the same tile, slab and group boundaries as the bf16 sweep.  ``SIIRL_TEST_SEED=<int>`` shifts the seeds."""
+    around the same edges as the bf16 sweep (all of one column group).  ``SIIRL_TEST_SEED=<int>`` shifts the seeds."""
     import random
 
     from siirl_amd import fused_linear as FL
