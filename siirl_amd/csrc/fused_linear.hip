@@ -1003,14 +1003,16 @@ int launch_short_k(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_t
   return SIIRL_OK;
 }
 
-// Tiles along M of an XCD's block, per GEMM of the fused path.  Measured at T=16384, H=3584, V=152064 with 256 x 256 tiles
-// (ms per step for blocks of 2 x 16 / 4 x 8 / 8 x 4 / 16 x 2 tiles): forward 13.34 / 13.32 / 13.67 / 15.16; recompute +
-// dlogits 13.97 / 14.17 / 14.30 / 14.90 (1 x 32: slower again); d weight 13.77 / 13.50 / 13.40 / 14.24.  The A operand
+// Tiles along M of an XCD's block, per GEMM of the fused path.  Measured at T=16384, H=3584, V=152064 (ms per step for
+// blocks of 2 x 16 / 4 x 8 / 8 x 4 / 16 x 2 tiles): forward 12.77 / 12.54 / 12.81 / 13.74; recompute + dlogits 13.35 / 12.97 /
+// 13.31 / 13.65; d hidden 15.33 / 13.44 / 14.68 / 15.09; d weight 15.46 / 12.86 / 12.74 / 13.92.  The A operand
 // of the first two is W, streamed from memory once per strip of blk_n token tiles: wider strips read it less often.
-// d hidden with 128 x 256 tiles (us, first group): 7192 / 5574 / 6115 for blocks of 2 x 16 / 4 x 8 / 8 x 4; with one token
-// tile the tiles of a K run share nothing but its dlogits, so they go to one XCD: 649 / 437 / 410 / 304 / 300 us for 2 x 16
-// .. 32 x 1 at T=200.
-constexpr int kBlkFwd = 4, kBlkRecompute = 2, kBlkDHidden = 4, kBlkDWeight = 8;
+// Recompute at fewer tokens, 2 x 16 / 4 x 8 (us, with d weight): H=2048, V=50257 T=3001 1005 / 1026, T=4096 1347 / 1319; H=1024,
+// V=32000 T=2048 227 / 231, T=8192 909 / 870: the wide blocks below 16 token tiles.
+// With one token tile the tiles of a d hidden K run share nothing but its dlogits, so they go to one XCD: 649 / 437 / 410 /
+// 304 / 300 us for 2 x 16 .. 32 x 1 at T=200.
+constexpr int kBlkFwd = 4, kBlkDHidden = 4, kBlkDWeight = 8;
+inline int blk_recompute(int tiles_t) { return tiles_t < 16 ? 2 : 4; }
 
 // Number of K runs of the d-hidden GEMM, each with an fp32 buffer of its own that sum_convert_kernel adds up.  The
 // tiles of [T, H] alone rarely fill the 256 CUs, two each: 1792 tiles at T=16384, H=3584 are 3.5 rounds (two runs: 7), 28
@@ -1326,9 +1328,9 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
                              g_entropy, labels, D + (s0 >> 5) * 1024, ws.kb_d};
         const uint16_t* ws0 = w + (v0 + s0) * Kc;
         if (int rc = f16 ? launch_gemm<DlogitsEpi, A_ROWS, true>(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st,
-                                                                "gemm_nt_kernel<DlogitsEpi, f16>", 1, kBlkRecompute)
+                                                                "gemm_nt_kernel<DlogitsEpi, f16>", 1, blk_recompute(tiles_t))
                          : launch_gemm(ws0, Kc, hp, Kc / 32, Ns, (int)T, (int)Kc, epi, st, "gemm_nt_kernel<DlogitsEpi>", 1,
-                                       kBlkRecompute))
+                                       blk_recompute(tiles_t)))
           return rc;
       }
     } else {
