@@ -564,9 +564,10 @@ size_t siirl_gae_workspace_bytes(int64_t B, int64_t L);
  *   delta = r_t + gamma * V_next - V_t,  A_t = delta + gamma * lam * A_next; a token with mask 0 keeps V_next and
  *   A_next of the token after it (both start at 0).  returns = A + values (before whitening);
  *   advantages = masked_whiten(A, mask).  With SIIRL_GAE_EXACT_ORDER the scan is evaluated in the reference's
- *   float32 operation order and `returns` is bit-identical to the reference's; SIIRL_GAE_CHUNKED shortens the
- *   dependent chain 16-fold for long rows (same arithmetic inside a chunk; the state entering a chunk goes through
- *   the chunks' composed maps, which changes its rounding: results agree to float32 accuracy, not bit for bit).
+ *   float32 operation order and `returns` equals the reference's (only the sign of a zero may differ);
+ *   SIIRL_GAE_CHUNKED shortens the dependent chain 16-fold for long rows (same arithmetic inside a chunk; the state
+ *   entering a chunk goes through the chunks' composed maps, which changes its rounding: results agree to float32
+ *   accuracy).  It pays for few rows only: [64, 8192] 58 us against 93, [1024, 8192] 118 against 105.
  *   stats3 as for siirl_masked_whiten.
  * Replaces: compute_gae_advantage_return siirl/dag_worker/core_algos.py:229-276.
  */

@@ -237,9 +237,9 @@ _gae_order = "exact"
 
 def set_gae_scan_order(order: str) -> None:
     """``"exact"`` (default): each row is scanned in one sequential pass in the reference's float32 operation
-    order, ``returns`` is bit-identical to the reference's.  ``"chunked"``: rows of 1024 tokens or more are cut into
-    up to 16 chunks that are scanned in parallel and stitched through their composed affine maps -- a dependent
-    chain 16 times shorter, results equal to float32 accuracy rather than bit for bit."""
+    order, ``returns`` equals the reference's (only the sign of a zero may differ).  ``"chunked"``: rows of 1024 tokens
+    or more are cut into up to 16 chunks that are scanned in parallel and stitched through their composed affine maps
+    -- a dependent chain 16 times shorter, results equal to float32 accuracy only.  It pays for few long rows."""
     global _gae_order
     if order not in _GAE_ORDERS:
         raise ValueError(f"unknown GAE scan order {order!r}; choose from {sorted(_GAE_ORDERS)}")

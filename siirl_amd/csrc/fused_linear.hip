@@ -19,8 +19,8 @@
 //     and each lane loads its 16-byte operands straight into registers, one K-step ahead.
 //   * all loads of the main loop are inline asm with hand-placed s_waitcnt vmcnt: the compiler's own tracking
 //     would wait for every outstanding DMA before each LDS read.
-// Four epilogues: softmax partials (forward), dlogits in both layouts (backward), fp32 accumulate (d hidden),
-// bf16 store (d weight).  The backward walks the vocabulary in groups of columns: recompute the group's logits into
+// Four epilogues: softmax partials (forward), packed dlogits (backward), fp32 sums (d hidden), a store in the operands'
+// type (d weight).  The backward walks the vocabulary in groups of columns: recompute the group's logits into
 // dlogits[T, group], then dH += dlogits . W_group and dW_group = dlogits^T . hidden as two more runs of the same core.
 // dlogits are written fragment-packed, once, and serve both: as d hidden's B operand (its A is W as it lies in memory,
 // given by K-rows) and as d weight's A operand (its B a packed transposed copy of hidden).  A transposed copy of W, which
@@ -43,8 +43,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Workgroup tile 128 x 256 x 64, 4 waves along N, one per SIMD; two workgroups per CU (the LDS rings), which run through
 // their prologues and epilogues at different times.  Against tiles of 256 x 256 with 8 waves and one workgroup per CU, us:
-// forward T=200 345 -> 297, T=3001 (H=2048, fp16) 1710 -> 1660, T=16384 12990 -> 12500; recompute T=200 334 -> 289, a
-// slab at T=16384 717 -> 684; d weight T=200 542 -> 488, T=16384 the same (H=3584, V=152064 bf16 where not said).
+// forward T=200 345 -> 297, T=3001 (H=2048, fp16) 1710 -> 1660, T=16384 12990 -> 12540; recompute T=200 334 -> 289, 8192
+// columns at T=16384 717 -> 684; d weight T=200 542 -> 488, T=16384 the same (H=3584, V=152064 bf16 where not said).
 constexpr int BM = 128, BN = 256, BK = 64;
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
@@ -556,7 +556,7 @@ struct SoftmaxPartialsEpi {
   }
   __device__ __forceinline__ void operator()(floatx4 (&acc)[MI][NJ], int m0, int n0, int tm, int split, int wn, int lane,
                                              int tid, char* smem) const {
-    // Parking costs about 11 us per 256 KB: the workgroup's own drain, not a burst of the round.
+    // Parking takes the forward at T=16384, H=3584, V=152064 from 12.6 to 13.9 ms for 9.97 GB.
     if (save) {
       f32x4* dst = saved_tile(save, tm, n0 / BN, tiles_n) + tid;
 #pragma unroll
@@ -1047,7 +1047,8 @@ inline int64_t logits_k(int dtype, int64_t H) { return dtype == SIIRL_F32 ? 3 * 
 int check_fused(const void* hidden, const void* weight, int64_t T, int64_t H, int64_t V, float inv_T, int dtype) {
   SIIRL_REQUIRE(dtype == SIIRL_BF16 || dtype == SIIRL_F16 || dtype == SIIRL_F32,
                 "fused lm_head path takes bf16, fp16 or fp32 operands (dtype %d given)", dtype);
-  // 32-bit byte offsets inside a 256-row tile bound the row pitch of every A operand (W: K, D: group + pad)
+  // 32-bit byte offsets inside a tile bound the row pitch of every A operand (W: 128 rows of K or 64 K-rows; D: four
+  // 16-token rows of blocks)
   SIIRL_REQUIRE(T >= 1 && T < (1LL << 22) && V >= 1 && V < (1LL << 30), "T=%lld (< 4194304) V=%lld out of range",
                 (long long)T, (long long)V);
   SIIRL_REQUIRE(H >= BK && H % BK == 0 && logits_k(dtype, H) < (1 << 22),
@@ -1278,8 +1279,9 @@ extern "C" int siirl_fused_linear_logprob_entropy_bwd(const void* hidden, const 
   const uint16_t* h = (const uint16_t*)hidden;
   const uint16_t* w = (const uint16_t*)weight;
   // The logits are recomputed from the operands as given (fp16: the half MFMA; fp32: three bf16 terms per element,
-  // K = 3 H).  The two gradient GEMMs multiply the bf16 dlogits with bf16 copies of hidden and W (for fp16 and fp32
-  // operands: rounded to bf16 while they are transposed and packed) and write their fp32 sums in the operands' dtype.
+  // K = 3 H).  The two gradient GEMMs multiply the bf16 dlogits with hidden and W in bf16 and write their fp32 sums in the
+  // operands' dtype.  hidden is packed transposed (fp16: rounded on the way); W is read by K-rows where it lies (bf16), from
+  // a plain bf16 copy (fp16; 365 us a call at H=3584, V=152064) or from the first term of the staged rows (fp32).
   const int64_t Kc = logits_k(dtype, H);
   const bool f16 = dtype == SIIRL_F16;
   if (dtype == SIIRL_F32) {
