@@ -773,7 +773,7 @@ def bench_critic(args, dev):
                     "GAE + whitening, chunked scan order (not in the step above)": {"ms": gae_chunked_ms},
                     f"multi-agent GAE token walk, {m_req} requests x {m_steps} steps x 3 agents x <= {m_w} tokens "
                     "(not in the step above)": marft},
-        "roofline": {"bound": "hbm", "kernel": "gae_scan_vec_kernel + whiten_apply_kernel", "achieved": gae_bytes / ms[1] / 1e6,
+        "roofline": {"bound": "hbm", "kernel": "gae_scan_kernel + whiten_apply_kernel", "achieved": gae_bytes / ms[1] / 1e6,
                      "peak": 8000.0, "unit": "GB/s", "frac": gae_bytes / ms[1] / 1e6 / 8000.0, "traffic": None,
                      "note": "the scan is a sequential recurrence per row: its duration is the latency of 8192 dependent "
                              "steps, not a bandwidth figure"},
