@@ -75,7 +75,7 @@ typedef enum siirl_kl_mode {
 
 /* ABI version of this header (major * 1000 + minor); siirl_hip_abi_version() returns the one the library was built
  * from.  A host compiled against another version must not call the library. */
-#define SIIRL_HIP_ABI_VERSION 1010
+#define SIIRL_HIP_ABI_VERSION 1011
 int siirl_hip_abi_version(void);
 
 /* Message of the last failing call on this thread ("" if none).  Host pointer, valid until the
@@ -287,6 +287,36 @@ int siirl_actor_loss_bwd(const float* g_loss, const float* old_log_prob, const f
                          float entropy_coeff, int kl_mode, int kl_straight_through, float kl_coef,
                          float policy_drift_coeff, float loss_scale, const float* out16, const float* row_msum,
                          const float* row_s, float* d_log_prob, float* d_entropy, siirl_stream_t stream);
+
+/*
+ * siirl_actor_loss_fwd (token_aux NULL; it goes with the covariance losses, as in siirl_actor_loss_cov_fwd) which also
+ * writes token_grad[B, L] = mask * d(policy term + kl_coef * KL term + drift term) / d log_prob per token, that is
+ * everything of the gradient but the factor that the mask sums, loss_scale and the upstream gradient make.
+ * siirl_token_grad_bwd finishes it: 8 bytes per token in place of reading every operand again.  The policy and the
+ * auxiliary terms must share that factor: refused (SIIRL_ERR_UNSUPPORTED) for geo_mean, whose loss is per sequence, and
+ * for gspo with a KL or drift term under another agg_mode than seq-mean-token-mean.  row_s is needed by gspo only.
+ * Replaces: the forward half of the autograd graph over siirl/dag_worker/core_algos.py:710-792, :795-862, :572-629,
+ *           :865-895, :898-1071 and siirl/engine/actor/dp_actor.py:455-513.
+ */
+int siirl_actor_loss_fwd_grad(const float* old_log_prob, const float* log_prob, const float* advantages,
+                              const void* mask, int mask_dtype, const float* is_weights, const float* entropy,
+                              const float* ref_log_prob, const float* token_aux, int64_t B, int64_t L, int loss_mode,
+                              float clip_low, float clip_high, float clip_c, float log_ratio_clamp, int agg_mode,
+                              float entropy_coeff, int kl_mode, int kl_straight_through, float kl_coef,
+                              float policy_drift_coeff, float loss_scale, float* out16, float* row_msum, float* row_s,
+                              float* token_grad, void* workspace, size_t workspace_bytes, siirl_stream_t stream);
+
+/*
+ * Backward of siirl_actor_loss_fwd_grad for an upstream gradient g_loss[0] (device scalar):
+ * d_log_prob = g_loss * loss_scale * f * token_grad with f the row's factor of policy_agg_mode (gspo: seq-mean-token-mean,
+ * else the agg_mode of the forward), and, when d_entropy is not NULL, d_entropy = -g_loss * loss_scale * entropy_coeff *
+ * d agg_loss(., agg_mode) -- only then is the mask read.  token_grad is left as it is and may not overlap the outputs.
+ * Replaces: the backward of the same functions (siirl/dag_worker/core_algos.py:536-569, :710-1071).
+ */
+int siirl_token_grad_bwd(const float* g_loss, const float* token_grad, const void* mask, int mask_dtype, int64_t B,
+                         int64_t L, int policy_agg_mode, int agg_mode, float entropy_coeff, float loss_scale,
+                         const float* out16, const float* row_msum, float* d_log_prob, float* d_entropy,
+                         siirl_stream_t stream);
 
 /*
  * The two covariance losses (Clip-Cov, KL-Cov) pick a few tokens of the batch by the covariance of advantage and

@@ -113,9 +113,11 @@ __global__ __launch_bounds__(kThreads) void row_finish_kernel(const float* __res
 // ---------------------------------------------------------------------------- segment partials
 
 // KIND >= 0 compiles the token formula of that loss alone (the common ones); KIND < 0 reads a.kind at run time.
-template <int KIND>
+// KEEP: the token's gradient goes to `tg` as far as it is known here, mask * d token / d log-prob of the policy, KL and
+// drift terms together; the factor that the batch's mask decides follows in token_grad_bwd_kernel.
+template <int KIND, bool KEEP>
 __global__ __launch_bounds__(kStream) void loss_partials_kernel(LossArgs a, const float* __restrict__ row_s,
-                                                                 float* __restrict__ partials) {
+                                                                 float* __restrict__ partials, float* __restrict__ tg) {
   const int kind = KIND >= 0 ? KIND : a.kind;
   const int64_t b = blockIdx.x / a.nseg;
   const int seg = blockIdx.x % a.nseg;
@@ -142,6 +144,7 @@ __global__ __launch_bounds__(kStream) void loss_partials_kernel(LossArgs a, cons
     const Quad ent4 = a.ent ? load_quad(a.ent, idx0, vec, nv, 0.f, nt) : const_quad(0.f);
     const Quad ref4 = a.ref ? load_quad(a.ref, idx0, vec, nv, 0.f, nt) : const_quad(0.f);
     const Quad aux4 = ((KIND < 0 || KIND >= KIND_KL_COV) && a.aux) ? load_quad(a.aux, idx0, vec, nv, 0.f, nt) : const_quad(0.f);
+    Quad tg4 = const_quad(0.f);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (e >= nv) break;
@@ -161,9 +164,20 @@ __global__ __launch_bounds__(kStream) void loss_partials_kernel(LossArgs a, cons
       acc[P_RMIN] = fminf(acc[P_RMIN], o.r_raw);
       acc[P_RMAX] = fmaxf(acc[P_RMAX], o.r_raw);
       if (a.ent) acc[P_ENT] += contrib(ent4.v[e], m, a.aux_agg_mode);
-      if (a.ref) acc[P_KL] += contrib(kl_token(lp, ref4.v[e], a.kl_mode, 0).v, m, a.aux_agg_mode);
-      if (a.drift_coef != 0.f) acc[P_AUX0] += contrib(clamp_max(o.r_raw - 1.f, 2.f) * lp, m, a.aux_agg_mode);
+      float d = m * o.dtok;
+      if (a.drift_coef != 0.f) {
+        const float w = clamp_max(o.r_raw - 1.f, 2.f);  // the weight of the drift term is detached
+        acc[P_AUX0] += contrib(w * lp, m, a.aux_agg_mode);
+        d += a.drift_coef * m * w;
+      }
+      if (a.ref) {
+        const KlOut kl = kl_token(lp, ref4.v[e], a.kl_mode, KEEP ? a.kl_st : 0);
+        acc[P_KL] += contrib(kl.v, m, a.aux_agg_mode);
+        d += a.kl_coef * m * kl.g;
+      }
+      tg4.v[e] = d;
     }
+    if (KEEP) store_quad(tg, idx0, vec, nv, tg4, nt);
   }
 
   // one wave-level reduction per partial, one LDS exchange for all of them
@@ -424,6 +438,49 @@ __device__ __forceinline__ AggCoef agg_coef(int agg, float mtotal, float mrow, i
   }
 }
 
+// The backward of a forward that kept the tokens' gradients: d log-prob = g * c * tg, c the aggregation's factor of the
+// row; with an entropy term its gradient besides, which takes the mask alone.  A stream of 4 bytes in and 4 out per
+// token, where loss_bwd_kernel reads every operand again (24 + 4 with four operands and an int64 mask): at [5744, 8192]
+// 63 us (6.0 TB/s) against 227; the forward that keeps them takes 232 us (5.7 TB/s) against 182.
+// kTgQuads quads per thread, all loads issued first.
+constexpr int kTgQuads = kSeg / 4 / kStream;
+template <bool ENT>
+__global__ __launch_bounds__(kStream) void token_grad_bwd_kernel(LossArgs a, const float* __restrict__ g_out,
+                                                                  const float* __restrict__ saved_out,
+                                                                  const float* __restrict__ row_msum,
+                                                                  const float* __restrict__ tg,
+                                                                  float* __restrict__ d_lp, float* __restrict__ d_ent) {
+  const int64_t b = blockIdx.x / a.nseg;
+  const int64_t t0 = (int64_t)(blockIdx.x % a.nseg) * kSeg;
+  const bool vec = a.vec != 0, nt = a.nt != 0;
+  Quad q[kTgQuads], m[kTgQuads];
+#pragma unroll
+  for (int i = 0; i < kTgQuads; ++i) {
+    const int64_t t = t0 + 4 * (threadIdx.x + i * kStream);
+    const int nv = (int)((a.L - t) < 4 ? (a.L - t) : 4);
+    if (nv <= 0) continue;
+    q[i] = load_quad(tg, b * a.L + t, vec, nv, 0.f, nt);
+    if (ENT) m[i] = load_mask_quad(a.mask, a.mask_dtype, b * a.L + t, vec, nv, nt);
+  }
+  const float g = g_out[0] * a.scale;
+  const float mtotal = saved_out[O_MTOTAL], mrow = row_msum[b];
+  const float gc = g * agg_coef(a.agg_mode, mtotal, mrow, a.B, a.L).c;
+  const AggCoef w_ent = agg_coef(a.aux_agg_mode, mtotal, mrow, a.B, a.L);
+#pragma unroll
+  for (int i = 0; i < kTgQuads; ++i) {
+    const int64_t t = t0 + 4 * (threadIdx.x + i * kStream);
+    const int nv = (int)((a.L - t) < 4 ? (a.L - t) : 4);
+    if (nv <= 0) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      q[i].v[e] *= gc;
+      if (ENT) m[i].v[e] = -g * a.ent_coef * w_ent(m[i].v[e]);
+    }
+    store_quad(d_lp, b * a.L + t, vec, nv, q[i]);
+    if (ENT) store_quad(d_ent, b * a.L + t, vec, nv, m[i]);
+  }
+}
+
 template <int KIND>
 __global__ __launch_bounds__(kStream) void loss_bwd_kernel(LossArgs a, const float* __restrict__ g_out,
                                                             const float* __restrict__ saved_out,
@@ -499,6 +556,17 @@ int launch_loss_bwd(const LossArgs& a, const float* g_out, const float* saved_ou
     default: loss_bwd_kernel<-1><<<grid, block, 0, st>>>(a, g_out, saved_out, row_msum, row_s, d_lp, d_ent);
   }
   SIIRL_LAUNCH_CHECK("loss_bwd_kernel");
+  return SIIRL_OK;
+}
+
+int launch_token_grad_bwd(const LossArgs& a, const float* g_out, const float* saved_out, const float* row_msum,
+                          const float* tg, float* d_lp, float* d_ent, hipStream_t st) {
+  const dim3 grid((unsigned)(a.B * a.nseg)), block(kStream);
+  if (d_ent)
+    token_grad_bwd_kernel<true><<<grid, block, 0, st>>>(a, g_out, saved_out, row_msum, tg, d_lp, d_ent);
+  else
+    token_grad_bwd_kernel<false><<<grid, block, 0, st>>>(a, g_out, saved_out, row_msum, tg, d_lp, nullptr);
+  SIIRL_LAUNCH_CHECK("token_grad_bwd_kernel");
   return SIIRL_OK;
 }
 
@@ -849,23 +917,25 @@ int check_agg(int agg) {
 }
 
 
-int launch_loss_partials(const LossArgs& a, const float* row_s, float* partials, hipStream_t st) {
+template <bool KEEP>
+int launch_loss_partials(const LossArgs& a, const float* row_s, float* partials, float* tg, hipStream_t st) {
   const dim3 grid((unsigned)(a.B * a.nseg)), block(kStream);
   switch (a.kind) {
-    case KIND_VANILLA: loss_partials_kernel<KIND_VANILLA><<<grid, block, 0, st>>>(a, row_s, partials); break;
-    case KIND_GSPO: loss_partials_kernel<KIND_GSPO><<<grid, block, 0, st>>>(a, row_s, partials); break;
-    case KIND_AGG: loss_partials_kernel<KIND_AGG><<<grid, block, 0, st>>>(a, row_s, partials); break;
-    case KIND_VALUE: loss_partials_kernel<KIND_VALUE><<<grid, block, 0, st>>>(a, row_s, partials); break;
-    case KIND_KL_COV: loss_partials_kernel<KIND_KL_COV><<<grid, block, 0, st>>>(a, row_s, partials); break;
-    case KIND_CLIP_COV: loss_partials_kernel<KIND_CLIP_COV><<<grid, block, 0, st>>>(a, row_s, partials); break;
-    default: loss_partials_kernel<-1><<<grid, block, 0, st>>>(a, row_s, partials);
+    case KIND_VANILLA: loss_partials_kernel<KIND_VANILLA, KEEP><<<grid, block, 0, st>>>(a, row_s, partials, tg); break;
+    case KIND_GSPO: loss_partials_kernel<KIND_GSPO, KEEP><<<grid, block, 0, st>>>(a, row_s, partials, tg); break;
+    case KIND_AGG: loss_partials_kernel<KIND_AGG, false><<<grid, block, 0, st>>>(a, row_s, partials, nullptr); break;
+    case KIND_VALUE: loss_partials_kernel<KIND_VALUE, false><<<grid, block, 0, st>>>(a, row_s, partials, nullptr); break;
+    case KIND_KL_COV: loss_partials_kernel<KIND_KL_COV, KEEP><<<grid, block, 0, st>>>(a, row_s, partials, tg); break;
+    case KIND_CLIP_COV: loss_partials_kernel<KIND_CLIP_COV, KEEP><<<grid, block, 0, st>>>(a, row_s, partials, tg); break;
+    default: loss_partials_kernel<-1, KEEP><<<grid, block, 0, st>>>(a, row_s, partials, tg);
   }
   SIIRL_LAUNCH_CHECK("loss_partials_kernel");
   return SIIRL_OK;
 }
 
+// `tg`: where the tokens' gradients go, or null
 int run_forward(LossArgs& a, float* out16, float* row_msum, float* row_s, void* ws, size_t ws_bytes,
-                hipStream_t st) {
+                hipStream_t st, float* tg = nullptr) {
   if (a.B == 0) {  // the finish alone: zero sums give the reference's 0 (token-mean, -sum-norm) or NaN (seq-mean-*)
     a.nseg = nseg_of(a.L);
     loss_finish_kernel<<<1, dim3(kThreads), 0, st>>>(a, nullptr, row_s, out16, row_msum);
@@ -877,7 +947,7 @@ int run_forward(LossArgs& a, float* out16, float* row_msum, float* row_s, void* 
     return fail(SIIRL_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu needed for B=%lld L=%lld",
                 ws_bytes, ws_bytes_of(a.B, a.L), (long long)a.B, (long long)a.L);
   SIIRL_REQUIRE(((uintptr_t)ws & 7) == 0, "workspace must be 8-byte aligned");
-  set_vec(a);
+  set_vec(a, tg);
   float* partials = (float*)ws;
   float* pre = partials + (size_t)a.B * a.nseg * kNP;
   dim3 grid((unsigned)(a.B * a.nseg)), block(kThreads);
@@ -888,7 +958,9 @@ int run_forward(LossArgs& a, float* out16, float* row_msum, float* row_s, void* 
                                                                                        a.isw != nullptr, row_s);
     SIIRL_LAUNCH_CHECK("row_finish_kernel");
   }
-  if (int rc = launch_loss_partials(a, row_s, partials, st)) return rc;
+  if (int rc = tg ? launch_loss_partials<true>(a, row_s, partials, tg, st)
+                  : launch_loss_partials<false>(a, row_s, partials, nullptr, st))
+    return rc;
   const size_t used = ((size_t)a.B * a.nseg * (kNP + kNPre) * sizeof(float) + 255) / 256 * 256;
   const float* folded = partials;  // the pre-pass sums are spent by now: their room serves the folding of long rows
   if (int rc = fold_long_rows(folded, partials, pre, a.B, a.nseg, st)) return rc;
@@ -1091,6 +1163,57 @@ extern "C" int siirl_actor_loss_bwd(const float* g_loss, const float* old_log_pr
   return launch_loss_bwd(a, g_loss, out16, row_msum, row_s, d_log_prob, d_entropy, (hipStream_t)stream);
 }
 
+// one factor per row serves every term: see siirl_actor_loss_fwd_grad
+static bool shares_row_factor(const LossArgs& a) {
+  return a.kind != KIND_GEO && (a.agg_mode == a.aux_agg_mode || (a.ref == nullptr && a.drift_coef == 0.f));
+}
+
+extern "C" int siirl_actor_loss_fwd_grad(const float* old_log_prob, const float* log_prob, const float* advantages,
+                                         const void* mask, int mask_dtype, const float* is_weights,
+                                         const float* entropy, const float* ref_log_prob, const float* token_aux,
+                                         int64_t B, int64_t L, int loss_mode, float clip_low, float clip_high,
+                                         float clip_c, float log_ratio_clamp, int agg_mode, float entropy_coeff,
+                                         int kl_mode, int kl_straight_through, float kl_coef, float policy_drift_coeff,
+                                         float loss_scale, float* out16, float* row_msum, float* row_s,
+                                         float* token_grad, void* workspace, size_t workspace_bytes,
+                                         siirl_stream_t stream) {
+  LossArgs a{};
+  const bool cov = loss_mode == SIIRL_LOSS_KL_COV || loss_mode == SIIRL_LOSS_CLIP_COV;
+  SIIRL_REQUIRE(B == 0 || cov == (token_aux != nullptr), "token_aux goes with the kl_cov and clip_cov losses");
+  if (int rc = fill_actor_args(a, old_log_prob, log_prob, advantages, mask, mask_dtype, is_weights, entropy,
+                               ref_log_prob, B, L, loss_mode, clip_low, clip_high, clip_c, log_ratio_clamp, agg_mode,
+                               entropy_coeff, kl_mode, kl_straight_through, kl_coef, policy_drift_coeff, loss_scale,
+                               token_aux, cov))
+    return rc;
+  SIIRL_REQUIRE(out16 && (B == 0 || (row_msum && token_grad)), "NULL output");
+  SIIRL_REQUIRE(B == 0 || loss_mode != SIIRL_LOSS_GSPO || row_s, "row_s is required for the gspo loss");
+  if (!shares_row_factor(a))
+    return fail(SIIRL_ERR_UNSUPPORTED, "loss mode %d with agg_mode %d: the terms of the loss share no row factor",
+                loss_mode, agg_mode);
+  return run_forward(a, out16, row_msum, row_s, workspace, workspace_bytes, (hipStream_t)stream, token_grad);
+}
+
+extern "C" int siirl_token_grad_bwd(const float* g_loss, const float* token_grad, const void* mask, int mask_dtype,
+                                    int64_t B, int64_t L, int policy_agg_mode, int agg_mode, float entropy_coeff,
+                                    float loss_scale, const float* out16, const float* row_msum, float* d_log_prob,
+                                    float* d_entropy, siirl_stream_t stream) {
+  if (int rc = check_dims(B, L)) return rc;
+  if (int rc = check_agg(policy_agg_mode)) return rc;
+  if (int rc = check_agg(agg_mode)) return rc;
+  if (B == 0) return SIIRL_OK;
+  SIIRL_REQUIRE(g_loss && token_grad && out16 && row_msum && d_log_prob, "NULL operand");
+  SIIRL_REQUIRE(d_entropy == nullptr || mask != nullptr, "the gradient of the entropy term needs the mask");
+  LossArgs a{};
+  a.lp = token_grad; a.agg_mode = policy_agg_mode; a.aux_agg_mode = agg_mode;
+  a.ent_coef = entropy_coeff; a.scale = loss_scale; a.B = B; a.L = L; a.nseg = nseg_of(L);
+  if (d_entropy) {
+    if (int rc = check_mask_dtype(mask_dtype)) return rc;
+    a.mask = mask; a.mask_dtype = mask_dtype;
+  }
+  set_vec(a, d_log_prob, d_entropy);
+  return launch_token_grad_bwd(a, g_loss, out16, row_msum, token_grad, d_log_prob, d_entropy, (hipStream_t)stream);
+}
+
 extern "C" size_t siirl_cov_workspace_bytes(void) { return (size_t)kCovGrid * kCovSums * sizeof(double); }
 
 extern "C" int siirl_cov_scores(const float* old_log_prob, const float* log_prob, const float* advantages,
@@ -1265,7 +1388,7 @@ extern "C" int siirl_masked_reduce(const float* values, const void* mask, int ma
   hipStream_t st = (hipStream_t)stream;
   float* partials = (float*)workspace;
   set_vec(a);
-  if (int rc = launch_loss_partials(a, nullptr, partials, st)) return rc;
+  if (int rc = launch_loss_partials<false>(a, nullptr, partials, nullptr, st)) return rc;
   const size_t used = ((size_t)B * a.nseg * (kNP + kNPre) * sizeof(float) + 255) / 256 * 256;
   const float* folded = partials;
   if (int rc = fold_long_rows(folded, partials, partials + (size_t)B * a.nseg * kNP, B, a.nseg, st)) return rc;

@@ -123,13 +123,13 @@ __device__ __forceinline__ Quad load_mask_quad(const void* p, int dt, int64_t id
   }
   return q;
 }
-__device__ __forceinline__ void store_quad(float* __restrict__ p, int64_t idx, bool vec, int nv, const Quad& q) {
+__device__ __forceinline__ void store_quad(float* __restrict__ p, int64_t idx, bool vec, int nv, const Quad& q,
+                                           bool nt = SIIRL_LOSS_NT_STORE != 0) {
   if (vec) {
-#if SIIRL_LOSS_NT_STORE
-    __builtin_nontemporal_store(u32x4{f2u(q.v[0]), f2u(q.v[1]), f2u(q.v[2]), f2u(q.v[3])}, reinterpret_cast<u32x4*>(p + idx));
-#else
-    *reinterpret_cast<float4*>(p + idx) = make_float4(q.v[0], q.v[1], q.v[2], q.v[3]);
-#endif
+    if (SIIRL_LOSS_NT_STORE && nt)
+      __builtin_nontemporal_store(u32x4{f2u(q.v[0]), f2u(q.v[1]), f2u(q.v[2]), f2u(q.v[3])}, reinterpret_cast<u32x4*>(p + idx));
+    else
+      *reinterpret_cast<float4*>(p + idx) = make_float4(q.v[0], q.v[1], q.v[2], q.v[3]);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)

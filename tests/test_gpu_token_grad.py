@@ -1,0 +1,106 @@
+"""GPU parity of the loss forward that keeps the tokens' gradients (``siirl_actor_loss_fwd_grad``,
+``siirl_token_grad_bwd``) against the backward that reads the operands again, for every loss, aggregation and term, at the
+edges of quads and of segments of 2048 tokens, and through autograd.
+
+Tolerance: both multiply the same per-token factors, in another order (g * c * (m * d) against g * ((m * c) * d)), so a
+gradient differs by a few roundings (2^-24 each) of its largest term: 1e-6 of the row's largest gradient bounds it."""
+
+import ctypes
+import itertools
+
+import pytest
+import torch
+
+import siirl_amd.core_algos as CA
+from siirl_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+TERMS = {"plain": (False, False, 0.0), "all": (True, True, 0.05)}
+SHAPES = [(1, 1), (3, 5), (2, 2044), (5, 2048), (2, 2049), (3, 4100), (130, 513)]
+NONE = ctypes.c_void_p(0)
+
+
+def _mask(B, L, i, g, dev):
+    mask = torch.rand(B, L, generator=g) < 0.7
+    mask[:, 0] = True
+    return mask.to([torch.bool, torch.int64, torch.float32, torch.bfloat16][i % 4]).to(dev)
+
+
+def _buffers(B, L, dev, mask):
+    f = lambda *s: torch.full(s, float("nan"), device=dev)  # noqa: E731  every word must be written
+    nws = _lib.lib().siirl_loss_workspace_bytes(B, L)
+    m = (_lib.ptr(mask), _lib.dtype_code(mask.dtype))
+    return f(16), f(B), f(B), f(B, L), torch.empty(nws, dtype=torch.uint8, device=dev), nws, m
+
+
+@pytest.mark.parametrize("mode,agg,terms", list(itertools.product(["vanilla", "gspo", "cpgd", "gpg", "geo_mean"], range(4),
+                                                                   TERMS)))
+def test_kept_token_gradients(dev, mode, agg, terms):
+    ent, ref, drift = TERMS[terms]
+    P, h, st = _lib.ptr, _lib.lib(), _lib.current_stream(dev)
+    for i, (B, L) in enumerate(SHAPES):
+        g = torch.Generator().manual_seed(1000 * agg + i)
+        f = lambda: torch.randn(B, L, generator=g).to(dev)  # noqa: E731
+        lp, old = 0.3 * f() - 1.0, 0.3 * f() - 1.0
+        adv, isw = f(), torch.rand(B, L, generator=g).to(dev) + 0.5
+        e, r = (f().abs() if ent else None), (lp + 0.1 * f() if ref else None)
+        mask = _mask(B, L, i, g, dev)
+        args = (CA._LOSS_CODES[mode], 0.2, 0.28, 3.0, 20.0, agg, 0.01 if ent else 0.0, 3, False, 0.1 if ref else 0.0, drift, 0.7)
+        out16, msum, rs, tg, ws, nws, m = _buffers(B, L, dev, mask)
+        rc = h.siirl_actor_loss_fwd_grad(P(old), P(lp), P(adv), *m, P(isw), P(e), P(r), NONE, B, L, *args, P(out16), P(msum),
+                                         P(rs), P(tg), P(ws), nws, st)
+        if mode == "geo_mean" or (mode == "gspo" and terms == "all" and agg != 2):
+            assert rc == -2 and b"row factor" in h.siirl_hip_last_error()
+            continue
+        assert rc == 0
+        o_out16, o_msum, o_rs = torch.ops.siirl_hip.policy_loss_fwd(old, lp, adv, mask, isw, e, r, *args)
+        assert torch.equal(out16, o_out16) and torch.equal(msum, o_msum)
+        up = torch.tensor([1.7], device=dev)
+        want, want_e = torch.ops.siirl_hip.policy_loss_bwd(up, old, lp, adv, mask, isw, e, r, *args, o_out16, o_msum, o_rs)
+        got, got_e = torch.full_like(lp, float("nan")), torch.full_like(lp, float("nan"))
+        kept = tg.clone()
+        rc = h.siirl_token_grad_bwd(P(up), P(tg), *(m if ent else (NONE, 0)), B, L, 2 if mode == "gspo" else agg, agg, args[6],
+                                    args[-1], P(out16), P(msum), P(got), P(got_e) if ent else NONE, st)
+        assert rc == 0 and torch.equal(tg, kept)
+        assert ((got - want).abs() <= 1e-6 * want.abs().amax(1, keepdim=True)).all(), (B, L)
+        if ent:
+            assert torch.equal(got_e, want_e)
+
+
+def test_autograd_takes_the_kept_gradients(dev):
+    """Above the rule's line: two backwards of one graph, the entropy's gradient, changed operands."""
+    B, L = 1025, 2052
+    f = lambda: torch.randn(B, L, device=dev)  # noqa: E731
+    torch.manual_seed(3)
+    lp, old, adv, ref, ent = 0.3 * f(), 0.3 * f(), f(), 0.3 * f(), f().abs()
+    mask = (torch.rand(B, L, device=dev) < 0.7).long()
+    args = (0, 0.2, 0.28, 3.0, 20.0, 0, 0.01, 3, False, 0.1, 0.0, 0.7)
+    leaf, eleaf = lp.clone().requires_grad_(True), ent.clone().requires_grad_(True)
+    outs = torch.ops.siirl_hip.actor_loss(leaf, eleaf, old, adv, mask, None, ref, *args, False, None)
+    up = torch.tensor(1.7, device=dev)
+    got, got_e = torch.autograd.grad(outs[0], [leaf, eleaf], up, retain_graph=True)
+    (again,) = torch.autograd.grad(outs[0], leaf, 2 * up)
+    fwd = torch.ops.siirl_hip.policy_loss_fwd(old, lp, adv, mask, None, ent, ref, *args)
+    want, want_e = torch.ops.siirl_hip.policy_loss_bwd(up.reshape(1), old, lp, adv, mask, None, ent, ref, *args, *fwd)
+    bound = 1e-6 * want.abs().amax(1, keepdim=True)
+    assert not torch.equal(got, want)  # (the other order of the products: it is the kept gradients that were scaled)
+    assert ((got - want).abs() <= bound).all() and ((again - 2 * want).abs() <= 2 * bound).all()
+    assert torch.equal(got_e, want_e)
+    outs = torch.ops.siirl_hip.actor_loss(leaf, None, old, adv, mask, None, ref, *args, False, None)
+    old += 1.0  # a saved operand that changes before the backward is refused, though the backward would not read it
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(outs[0], leaf)
+
+
+def test_no_gradient_is_kept_for_nothing(dev):
+    """Without differentiation the forward allocates no [B, L] buffer."""
+    lp, old, adv = (torch.randn(1025, 2052, device=dev) for _ in range(3))
+    mask = torch.ones_like(lp, dtype=torch.bool)
+    args = (0, 0.2, 0.2, 3.0, 20.0, 0, 0.0, 0, False, 0.0, 0.0, 1.0, False, None)
+    torch.ops.siirl_hip.actor_loss(lp, None, old, adv, mask, None, None, *args)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    torch.ops.siirl_hip.actor_loss(lp, None, old, adv, mask, None, None, *args)
+    assert torch.cuda.max_memory_allocated() - before < lp.numel()
