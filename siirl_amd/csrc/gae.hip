@@ -106,11 +106,18 @@ __device__ __forceinline__ void load_mask_pieces(const void* mask, int64_t idx, 
 // the right with m = 1 (the row's entering state if there is none), so that only a product and a sum per token remain
 // on the chain:  A <- d + k * A  with d = delta, k = gamma * lam where m = 1 and d = 0, k = 1 where m = 0.  (Zeros may
 // differ in their sign.)  A workgroup owns four rows in tiles of 128 columns, right to left.  Its first wave walks the
-// chain, a row per lane; two more waves fetch the tiles four ahead (16-byte loads), prepare d and k a tile ahead and
-// store the tile behind with its whitening statistics.  Four rows per workgroup: 256 workgroups at B = 1024.
-// B = 1024, L = 8192, int64 mask: 91 us (2.6 TB/s), gae_rows_kernel 508 us (149 cycles a token).
+// chain; two more waves fetch the tiles four ahead (16-byte loads), prepare d and k a tile ahead and store the tile behind
+// with its whitening statistics.  Four rows per workgroup: 256 workgroups at B = 1024.
+// In the chain's wave every LDS instruction is time that the chain does not move: the product and the sum of a token take
+// 8.6 cycles, a 16-byte read of four tokens 8, a 16-byte write of four 28.  So all 64 lanes walk, 16 of them each row
+// alike, without a branch; each keeps the state that enters one quad out of 16 (a select), writes it once per 64 tokens,
+// and the wave that stores the tile walks its quads once more from there.  The reads are 32 tokens ahead.  (Writing every
+// A from four lanes took 20 cycles a token against 16 now; k in a register where a tile's rows are all ones or all zeros
+// gained nothing, nor did reading d and k through DPP, whose wait states cost more than the LDS.)
+// B = 1024, L = 8192, int64 mask: 65 us (3.1 TB/s), before 91 us, gae_rows_kernel 508 us (149 cycles a token).
 // A tile with another mask value, or with a delta that is not finite and moderate, or that takes A out of the finite
 // numbers, is walked by the recurrence as it stands, and so is the rest of those rows (`slow`).
+constexpr int kCkPitch = 48;  // the 64 lanes of the chain's wave write to as many banks
 constexpr int kScanRows = 4, kScanHelpers = kScanRows * kCols / 4, kScanThreads = kWave + kScanHelpers, kAhead = 4;
 static_assert(kScanHelpers % kWave == 0 && kCols / 4 == 32, "a helper wave holds two rows, a quad per lane");
 
@@ -124,6 +131,8 @@ __global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __r
   // two buffers of each: tile t + 1 is prepared and tile t - 1 stored while tile t is walked
   __shared__ __align__(16) float s_d[2][kScanRows * kPitch], s_k[2][kScanRows * kPitch], s_a[2][kScanRows * kPitch];
   __shared__ __align__(16) float s_r[2][kScanRows * kPitch], s_v[2][kScanRows * kPitch], s_m[2][kScanRows * kPitch];
+  __shared__ float s_c[2][kScanRows * kCkPitch];                // A entering each quad
+  __shared__ int s_walked[2];                                   // the tile's A is in s_a: it was walked as it stands
   __shared__ float s_nv[2][kScanRows];                          // V' entering the tile
   __shared__ int s_slow[2][kScanHelpers / kWave];               // the tile needs the recurrence as it stands
   __shared__ double s_st[kScanHelpers / kWave][kNStat];
@@ -135,46 +144,47 @@ __global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __r
   if (__builtin_amdgcn_readfirstlane(tid / kWave) == 0) {
     // ---- the chain
     float nv = 0.f, lg = 0.f;
-    if (init != nullptr && lane < nrows) lg = init[2 * (row0 + lane) + 1];
     bool slow = !(fabsf(gamma_lam) <= 1.f);
     bool first_slow = true;
-    const int row = lane < kScanRows ? lane : 0;  // (the other lanes walk row 0 again and store nothing)
+    const int row = lane % kScanRows, mine = lane / kScanRows;  // every row is walked by 16 lanes, alike
+    if (init != nullptr && row < nrows) lg = init[2 * (row0 + row) + 1];
     for (int i = 0; i < (NT + 1) / kAhead * kAhead + kAhead; ++i) {  // (as many barriers as the helpers meet)
       const int t = i - 1;
       if (t >= 0 && t < NT) {
         const int b = t & 1;
         const float entering = lg;
-        slow |= __builtin_amdgcn_readfirstlane(s_slow[b][0] | s_slow[b][1]) != 0;
-        if (!slow) {
-          const float* d = s_d[b] + row * kPitch;
-          const float* k = s_k[b] + row * kPitch;
-          float* a = s_a[b] + row * kPitch;
-          // the LDS reads of the next 16 tokens are issued before the current 16 are walked
-          float4 dc[4], kc[4], dn[4], kn[4];
+        const float *d = s_d[b] + row * kPitch, *k = s_k[b] + row * kPitch;
+        // 32 tokens are read while the 32 before them are walked (left to itself the compiler reads them just before)
+        float4 dc[8], kc[8], dn[8], kn[8];
+        auto fetch = [&](float4 (&dd)[8], float4 (&kk)[8], int c0) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            dc[q] = *reinterpret_cast<const float4*>(d + kCols - 16 + 4 * q);
-            kc[q] = *reinterpret_cast<const float4*>(k + kCols - 16 + 4 * q);
+          for (int q = 7; q >= 0; --q) {
+            dd[q] = *reinterpret_cast<const float4*>(d + c0 + 4 * q);
+            kk[q] = *reinterpret_cast<const float4*>(k + c0 + 4 * q);
           }
+        };
+        const int odd = s_slow[b][0] | s_slow[b][1];
+        fetch(dc, kc, kCols - 32);
+        __builtin_amdgcn_sched_barrier(0);
+        slow |= __builtin_amdgcn_readfirstlane(odd) != 0;
+        if (!slow) {
+          float enters = 0.f;
 #pragma unroll
-          for (int cc = kCols - 16; cc >= 0; cc -= 16) {
-            const int nx = cc >= 16 ? cc - 16 : 0;
+          for (int c0 = kCols - 32; c0 >= 0; c0 -= 32) {
+            if (c0 > 0) fetch(dn, kn, c0 - 32);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              dn[q] = *reinterpret_cast<const float4*>(d + nx + 4 * q);
-              kn[q] = *reinterpret_cast<const float4*>(k + nx + 4 * q);
+            for (int q = 7; q >= 0; --q) {
+              enters = mine == (c0 / 4 + q) % 16 ? lg : enters;
+              lg = dc[q].w + kc[q].w * lg;
+              lg = dc[q].z + kc[q].z * lg;
+              lg = dc[q].y + kc[q].y * lg;
+              lg = dc[q].x + kc[q].x * lg;
             }
+            if (c0 % 64 == 0) s_c[b][row * kCkPitch + c0 / 4 + mine] = enters;
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int q = 3; q >= 0; --q) {
-              float4 o;
-              lg = dc[q].w + kc[q].w * lg; o.w = lg;
-              lg = dc[q].z + kc[q].z * lg; o.z = lg;
-              lg = dc[q].y + kc[q].y * lg; o.y = lg;
-              lg = dc[q].x + kc[q].x * lg; o.x = lg;
-              if (lane < kScanRows) *reinterpret_cast<float4*>(a + cc + 4 * q) = o;
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) dc[q] = dn[q], kc[q] = kn[q];
+            for (int q = 0; q < 8; ++q) dc[q] = dn[q], kc[q] = kn[q];
           }
           // An overflow stays: a tile that ends finite was finite throughout.  Only a state that `init` brings can do this
           // (chunks of rows): from zero, deltas of at most 1e30 take 3e8 tokens to leave the finite numbers.
@@ -198,6 +208,7 @@ __global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __r
               *reinterpret_cast<float4*>(s_a[b] + lane * kPitch + cc) = o;
             }
         }
+        if (lane == 0) s_walked[b] = slow;
       }
       __syncthreads();
     }
@@ -235,7 +246,14 @@ __global__ __launch_bounds__(kScanThreads) void gae_scan_kernel(const float* __r
         // them): with a fixed number of loads between a load and its use the wait for it leaves the later ones in flight.
         {  // store tile t - 1
           const int64_t col = (int64_t)(NT - t) * kCols + 4 * ch;
-          const float4 a = *reinterpret_cast<const float4*>(s_a[(t - 1) & 1] + o);
+          const int b = (t - 1) & 1;
+          const float4 d = *reinterpret_cast<const float4*>(s_d[b] + o), k = *reinterpret_cast<const float4*>(s_k[b] + o);
+          float4 a;
+          a.w = d.w + k.w * s_c[b][rr * kCkPitch + ch];
+          a.z = d.z + k.z * a.w;
+          a.y = d.y + k.y * a.z;
+          a.x = d.x + k.x * a.y;
+          if (__builtin_amdgcn_readfirstlane(s_walked[b])) a = *reinterpret_cast<const float4*>(s_a[b] + o);
           if (row_in && t >= 1 && t <= NT && col < L) {
             *reinterpret_cast<float4*>(adv + rbase + col) = a;
             *reinterpret_cast<float4*>(ret + rbase + col) = make_float4(a.x + v2.x, a.y + v2.y, a.z + v2.z, a.w + v2.w);
@@ -627,11 +645,11 @@ extern "C" size_t siirl_gae_workspace_bytes(int64_t B, int64_t L) {
 // with masks of up to four bytes: registers), and a workgroup pays four intervals however short its rows are;
 // gae_rows_kernel holds 64 rows a CU and streams.  So the first for up to three rounds of long rows (two, with the narrower
 // masks), the second beyond, and for rows of one tile from the end of the first round on.  GAE with whitening, first /
-// second (us), int64 mask: [1024, 128] 14.8 / 17.2, [2048, 128] 15.4 / 17.4, [3072, 128] 18.6 / 17.7, [4096, 32] 19.3 / 14.7,
-// [6144, 256] 30.2 / 31.9, [6144, 8192] 384 / 589, [8192, 256] 38.5 / 33.7, [8192, 1024] 90.3 / 90.5, [8192, 8192] 506 / 616,
-// [12000, 256] 53.5 / 36.1, [131072, 32] 382 / 77; in chunks of rows [1024, 8192] 161 / 118, [5488, 8192] 753 / 488.
-// float32 mask: [3072, 128] 16.2 / 17.1, [4096, 64] 16.4 / 14.7, [8192, 256] 31.0 / 32.2, [8192, 4096] 222 / 291, [12000, 256]
-// 40.7 / 32.4.  (Masks of other values than 0 and 1 would rather have the second from 3000 rows on, [4096, 8192] 554 / 494.)
+// second (us), int64 mask: [1024, 128] 12.6 / 17.1, [2048, 128] 14.2 / 17.4, [3072, 128] 18.3 / 18.3, [4096, 32] 18.3 / 15.0,
+// [6144, 256] 27.6 / 32.5, [6144, 8192] 306 / 594, [8192, 256] 34.4 / 33.5, [8192, 1024] 76 / 90, [8192, 8192] 398 / 621,
+// [12000, 256] 46.6 / 34.5, [12000, 1024] 107 / 98, [131072, 32] 299 / 74; in chunks of rows [1024, 8192] 142 / 113, [5488, 8192]
+// 692 / 488.  float32 mask: [3072, 128] 15.7 / 17.2, [4096, 128] 16.5 / 18.1, [4096, 64] 16.2 / 15.0, [8192, 256] 27.8 / 32.7,
+// [8192, 4096] 206 / 296, [12000, 256] 35.9 / 33.0.  (Masks of other values than 0 and 1 would rather have the second from 3000 rows on, [4096, 8192] 554 / 494.)
 static bool few_rows(int64_t rows, int64_t len, bool mask64) {
   if (len <= kCols) return rows <= (mask64 ? 2048 : 3072);
   return rows <= (mask64 && len < 1024 ? 6144 : 8192);
