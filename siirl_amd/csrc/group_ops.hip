@@ -24,7 +24,11 @@ namespace siirl {
 namespace {
 
 constexpr int kThreads = 256;   // streaming kernels (row sums, broadcast)
-constexpr int kGroupThreads = 64;  // all-pairs kernels: one wave per workgroup, so B = 8192 already fills 128 CUs
+// Run-walking kernels.  They are all latency: of the ordering check, B loads per workgroup, so fewer and larger workgroups
+// (eight loads a thread, in flight at once, at B = 8192); of the ends of a run, which ballots find inside a wave; and of the
+// members, which are read from an LDS copy of the workgroup's entries.  B = 8192, n = 16: keep mask 6.6 us, advantages
+// 6.0 us; one-wave workgroups that walked global memory member by member took 17.6 and 12.
+constexpr int kGroupThreads = 1024;
 
 // ---------------------------------------------------------------------------- row sums
 
@@ -48,22 +52,36 @@ __global__ __launch_bounds__(kThreads) void row_sum_kernel(const float* __restri
   if (threadIdx.x == 0) out[b] = (float)s;
 }
 
-// true iff uid[0] <= uid[1] <= ... ; evaluated by the whole workgroup (one wave), result uniform
+// true iff uid[0] <= uid[1] <= ... ; evaluated by the whole workgroup, result uniform
 __device__ __forceinline__ bool uid_non_decreasing(const int64_t* __restrict__ uid, int64_t B) {
   int bad = 0;  // no short circuit: the loads of successive iterations stay independent
 #pragma unroll 8
   for (int64_t j = threadIdx.x; j + 1 < B; j += kGroupThreads) bad |= (uid[j] > uid[j + 1]) ? 1 : 0;
-  return __all(bad == 0);
+  return __syncthreads_or(bad) == 0;
 }
-// the run [lo, hi) of positions around i that share uid[i] (uid non-decreasing)
+// the run [lo, hi) of positions around i that share uid[i] (uid non-decreasing); called by whole waves
 __device__ __forceinline__ void run_of(const int64_t* __restrict__ uid, int64_t B, int64_t i, int64_t& lo, int64_t& hi) {
-  const int64_t my = uid[i];
-  lo = i;
-  while (lo > 0 && uid[lo - 1] == my) --lo;
-  hi = i + 1;
-  while (hi < B && uid[hi] == my) ++hi;
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool in = i < B;
+  const int64_t my = in ? uid[i] : 0;
+  const uint64_t starts = __builtin_amdgcn_ballot_w64(in && (i == 0 || uid[i - 1] != my));
+  const uint64_t ends = __builtin_amdgcn_ballot_w64(in && (i == B - 1 || uid[i + 1] != my));
+  lo = hi = i;
+  if (!in) return;
+  const uint64_t before = starts & (~0ull >> (kWave - 1 - lane)), after = ends >> lane;
+  if (before) {
+    lo = i - lane + (kWave - 1 - __builtin_clzll(before));
+  } else {
+    lo = i - lane;
+    while (lo > 0 && uid[lo - 1] == my) --lo;
+  }
+  if (after) {
+    hi = i + __builtin_ctzll(after) + 1;
+  } else {
+    hi = i - lane + kWave;  // (no end in the wave: the run goes past it)
+    while (hi < B && uid[hi] == my) ++hi;
+  }
 }
-
 
 // ---------------------------------------------------------------------------- GRPO advantage
 
@@ -83,27 +101,38 @@ __device__ __forceinline__ float grpo_value(double s, double mean, double sd, fl
 __global__ __launch_bounds__(kGroupThreads) void grpo_group_kernel(const float* __restrict__ scores,
                                                               const int64_t* __restrict__ uid, int64_t B, float eps,
                                                               int norm_by_std, float* __restrict__ a_out) {
-  const int64_t i = (int64_t)blockIdx.x * kGroupThreads + threadIdx.x;
-  const bool runs = uid_non_decreasing(uid, B);
-  if (i >= B) return;
+  __shared__ float s_own[kGroupThreads];
+  const int64_t first = (int64_t)blockIdx.x * kGroupThreads, i = first + threadIdx.x;
+  const float mine = i < B ? scores[i] : 0.f;
+  s_own[threadIdx.x] = mine;
+  const bool runs = uid_non_decreasing(uid, B);  // (and s_own is published)
   if (!runs) {
-    a_out[i] = u2f(kPendingBits);
+    if (i < B) a_out[i] = u2f(kPendingBits);
     return;
   }
   int64_t lo, hi;
   run_of(uid, B, i, lo, hi);
+  if (i >= B) return;
   const int n = (int)(hi - lo);
-  double sum = 0.0;
-  for (int64_t j = lo; j < hi; ++j) sum += (double)scores[j];
-  const double mean = n > 1 ? sum / (double)n : 0.0;
-  double ss = 0.0;
-  if (n > 1)
-    for (int64_t j = lo; j < hi; ++j) {
-      const double d = (double)scores[j] - mean;
-      ss += d * d;
-    }
+  double mean = 0.0, ss = 0.0;
+  auto stats = [&](auto* v) {
+    double sum = 0.0;
+#pragma unroll 8
+    for (int j = 0; j < n; ++j) sum += (double)v[j];
+    mean = n > 1 ? sum / (double)n : 0.0;
+    if (n > 1)
+#pragma unroll 8
+      for (int j = 0; j < n; ++j) {
+        const double d = (double)v[j] - mean;
+        ss += d * d;
+      }
+  };
+  if (lo >= first && hi <= first + kGroupThreads)
+    stats(s_own + (int)(lo - first));
+  else
+    stats(scores + lo);
   const double sd = n > 1 ? sqrt(ss / (double)(n - 1)) : 1.0;
-  a_out[i] = grpo_value((double)scores[i], mean, sd, eps, norm_by_std);
+  a_out[i] = grpo_value((double)mine, mean, sd, eps, norm_by_std);
 }
 
 // Stages uid[base, base + kWaveTile) into LDS (all threads of the workgroup), then calls f(j) on the calling wave for
@@ -214,6 +243,25 @@ struct NpBlock {
   __device__ T finish() const { return (nb > 0 && n == nb) ? fold() : res; }
 };
 
+// numpy's pairwise_sum over v[0 .. n), n <= 128, of the values or of (v - mean)^2
+template <typename T, bool SQDEV, typename P>
+__device__ __forceinline__ T np_sum(P v, int n, T mean) {
+  auto term = [&](int k) {
+    const T x = v[k];
+    if (!SQDEV) return x;
+    const T d = x - mean;
+    return d * d;
+  };
+  T r[8] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
+  const int nb = n < 8 ? 0 : n - n % 8;
+  for (int k = 0; k < nb; k += 8)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] += term(k + e);
+  T res = nb > 0 ? ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7])) : T(0);
+  for (int k = nb; k < n; ++k) res += term(k);
+  return res;
+}
+
 // Pull-style iterator over the members of uid `my`, in batch order, from global memory.
 template <typename T>
 struct MemberCursor {
@@ -283,32 +331,30 @@ template <typename T>
 __global__ __launch_bounds__(kGroupThreads) void keep_mask_kernel(const T* __restrict__ val, const int64_t* __restrict__ uid,
                                                              int64_t B, uint8_t* __restrict__ keep,
                                                              int32_t* __restrict__ group_size) {
-  const int64_t i = (int64_t)blockIdx.x * kGroupThreads + threadIdx.x;
-  const bool runs = uid_non_decreasing(uid, B);
-  if (i >= B) return;
+  __shared__ T s_own[kGroupThreads];
+  const int64_t first = (int64_t)blockIdx.x * kGroupThreads, i = first + threadIdx.x;
+  if (i < B) s_own[threadIdx.x] = val[i];
+  const bool runs = uid_non_decreasing(uid, B);  // (and s_own is published)
   if (!runs) {
-    keep[i] = kPendingKeep;
+    if (i < B) keep[i] = kPendingKeep;
     return;
   }
-  const int64_t my = uid[i];
   int64_t lo, hi;
   run_of(uid, B, i, lo, hi);
+  if (i >= B) return;
   const int n = (int)(hi - lo);
   T mean, ssq;
   if (n <= 128) {
-    NpBlock<T> blk;
-    blk.begin(n);
-    if (n > 1)
-      for (int64_t j = lo; j < hi; ++j) blk.push(val[j]);
-    mean = blk.finish() / (T)n;
-    blk.begin(n);
-    if (n > 1)
-      for (int64_t j = lo; j < hi; ++j) {
-        const T d = val[j] - mean;
-        blk.push(d * d);
-      }
-    ssq = blk.finish();
+    auto stats = [&](auto* v) {
+      mean = np_sum<T, false>(v, n, T(0)) / (T)n;
+      ssq = np_sum<T, true>(v, n, mean);
+    };
+    if (lo >= first && hi <= first + kGroupThreads)
+      stats(s_own + (int)(lo - first));
+    else
+      stats(val + lo);
   } else {
+    const int64_t my = uid[i];
     MemberCursor<T> c1{uid, val, B, lo, my};
     mean = np_pairwise<T, false>(c1, n, T(0)) / (T)n;
     MemberCursor<T> c2{uid, val, B, lo, my};

@@ -250,3 +250,25 @@ def test_dynamic_sampling_end_to_end(dev):
     allsame = dict(batch, token_level_rewards=torch.ones(P * n, L, device=dev))
     res = DF.dynamic_sampling(cfg, allsame)
     assert res.metrics["dapo_sampling/filtered_indices"] == [] and res.batch == {}
+
+
+@pytest.mark.parametrize("sizes", [[1], [1024], [1025], [1] * 1030, [63, 2, 64, 65, 7, 8, 9, 1, 16, 129, 128, 127, 1100, 3, 600],
+                                   [1000, 30, 5, 1, 2000], [16] * 70 + [17]])
+def test_runs_across_waves_and_workgroups(dev, sizes):
+    """Sorted uids whose runs begin and end anywhere in a wave of 64 and a workgroup of 1024 trajectories."""
+    import siirl_amd.core_algos as CA
+    from siirl_amd.dapo_filter import group_keep_mask
+
+    g = torch.Generator().manual_seed(len(sizes))
+    uid = np.repeat(np.arange(len(sizes)) * 3 - 7, sizes)
+    B = len(uid)
+    for values in (torch.randint(0, 3, (B,), generator=g).float() * 0.1, torch.full((B,), 0.1), torch.randn(B, generator=g)):
+        for vals in (values.numpy(), values.double().numpy()):
+            keep, gsz = group_keep_mask(vals, uid, return_group_size=True)
+            assert np.array_equal(keep.cpu().numpy(), OD.keep_mask(vals, uid))
+            assert np.array_equal(gsz.cpu().numpy(), np.repeat(sizes, sizes))
+        mask = torch.ones(B, 1)
+        adv, _ = CA.compute_grpo_outcome_advantage(values[:, None].to(dev), mask.to(dev), uid)
+        want, _ = OC.compute_grpo_outcome_advantage(values[:, None].double(), mask, uid)
+        # (all-equal values: the deviation is the rounding of the mean, and 0 / (0 + eps) either way)
+        assert _rel_close(adv.cpu(), want, rtol=1e-5, atol=2e-6)[0]
