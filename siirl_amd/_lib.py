@@ -148,6 +148,19 @@ def dtype_code(torch_dtype) -> int:
     return table[torch_dtype]
 
 
+def to_device(arr, dev):
+    """A host array as a tensor on ``dev``, by way of pinned memory: the copy is queued like a kernel, where one from
+    pageable memory waits until the stream has done all that was queued before it.  (The pinned block is torch's and is
+    not used again before the copy has run.)  Under stream capture, which a pageable copy refuses, it stays refused: a
+    graph would read the block again at every replay."""
+    import torch
+
+    t = torch.from_numpy(arr)
+    if t.numel() == 0 or torch.device(dev).type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return t.to(dev)
+    return t.pin_memory().to(dev, non_blocking=True)
+
+
 def ptr(t):
     """Device pointer of a tensor (or NULL for None)."""
     return None if t is None else C.c_void_p(t.data_ptr())

@@ -225,7 +225,7 @@ def _uid_tensor(index, n, dev) -> torch.Tensor:
             seq = list(index) if isinstance(index, (list, tuple)) else list(arr.reshape(-1))
             codes: dict = {}
             arr = np.fromiter((codes.setdefault(int(v), len(codes)) for v in seq), dtype=np.int64, count=len(seq))
-        out = torch.from_numpy(np.ascontiguousarray(arr)).to(dev)
+        out = _lib.to_device(np.ascontiguousarray(arr), dev)
     if out.numel() != n:
         raise ValueError(f"index has {out.numel()} entries for a batch of {n}")
     return out.contiguous()

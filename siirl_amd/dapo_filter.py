@@ -51,9 +51,9 @@ def _metric_tensor(values, dev) -> torch.Tensor:
     arr = np.asarray(values)
     arr = arr.reshape(-1)
     if arr.dtype == np.float32:
-        return torch.from_numpy(np.ascontiguousarray(arr)).to(dev)
+        return _lib.to_device(np.ascontiguousarray(arr), dev)
     if arr.dtype.kind in "fiub" and arr.dtype != np.float16:
-        return torch.from_numpy(np.ascontiguousarray(arr.astype(np.float64))).to(dev)
+        return _lib.to_device(np.ascontiguousarray(arr.astype(np.float64)), dev)
     raise TypeError(f"metric dtype {arr.dtype} is not supported (float32, float64, integers, bool)")
 
 
@@ -66,12 +66,12 @@ def _uid_tensor(uids, dev) -> torch.Tensor:
         return uids.detach().reshape(-1).to(device=dev, dtype=torch.int64).contiguous()
     arr = np.asarray(uids)
     if arr.dtype.kind in "iu" and (arr.dtype.kind == "i" or arr.size == 0 or int(arr.max()) < 2 ** 63):
-        return torch.from_numpy(np.ascontiguousarray(arr.reshape(-1).astype(np.int64))).to(dev)
+        return _lib.to_device(np.ascontiguousarray(arr.reshape(-1).astype(np.int64)), dev)
     seq = list(uids) if isinstance(uids, (list, tuple)) else list(arr.reshape(-1))
     codes: dict = {}
     out = np.fromiter((codes.setdefault(int(v) if hasattr(v, "item") else v, len(codes)) for v in seq),
                       dtype=np.int64, count=len(seq))
-    return torch.from_numpy(out).to(dev)
+    return _lib.to_device(out, dev)
 
 
 def group_keep_mask(metric_values, uids, device=None, return_group_size: bool = False):
@@ -128,7 +128,7 @@ def filter_tensordict(batch, indices: List[int]):
         data = getattr(value, "data", value) if type(value).__name__ == "NonTensorData" else value
         if isinstance(value, torch.Tensor):
             if value.device not in idx_on:
-                idx_on[value.device] = torch.from_numpy(idx_np).to(value.device)
+                idx_on[value.device] = _lib.to_device(idx_np, value.device) if value.is_cuda else torch.from_numpy(idx_np)
             out[key] = _select_rows(value, idx_on[value.device])
         elif isinstance(data, np.ndarray) and len(data) == bsz:
             out[key] = data[idx_np]
@@ -222,11 +222,11 @@ def dynamic_sampling(config, batch, **kwargs) -> NodeOutput:
     codes = torch.add(keep, gsz, alpha=2).cpu().numpy()
     mask = (codes & 1).astype(bool)
     kept_rows = np.flatnonzero(mask)
+    filtered = filter_tensordict(batch, kept_rows)  # the GPU has its next work before the host counts groups
     kept = kept_rows.tolist()
     inv = 1.0 / (codes >> 1)  # each group of n members contributes n * (1/n) = 1
     total_groups = int(np.rint(inv.sum()))
     kept_groups = int(np.rint(inv[mask].sum()))
-    filtered = filter_tensordict(batch, kept_rows)
     final = len(kept)
     metrics = {
         "dapo_sampling/kept_trajectories_ratio": final / initial if initial > 0 else 1.0,
