@@ -3,7 +3,8 @@
 edges of quads and of segments of 2048 tokens, and through autograd.
 
 Tolerance: both multiply the same per-token factors, in another order (g * c * (m * d) against g * ((m * c) * d)), so a
-gradient differs by a few roundings (2^-24 each) of its largest term: 1e-6 of the row's largest gradient bounds it."""
+gradient differs by a few roundings (2^-24 each) of its largest term: 1e-6 of the row's largest gradient bounds it.
+The result block of the two forwards: sums in double, rounded once to float32, so one unit in the last place."""
 
 import ctypes
 import itertools
@@ -17,7 +18,7 @@ from siirl_amd import _lib
 pytestmark = pytest.mark.gpu
 
 TERMS = {"plain": (False, False, 0.0), "all": (True, True, 0.05)}
-SHAPES = [(1, 1), (3, 5), (2, 2044), (5, 2048), (2, 2049), (3, 4100), (130, 513)]
+SHAPES = [(1, 1), (3, 5), (2, 2044), (5, 2048), (2, 2049), (3, 4100), (8, 2048), (1, 16381), (9, 700), (130, 513), (1025, 6)]
 NONE = ctypes.c_void_p(0)
 
 
@@ -55,7 +56,8 @@ def test_kept_token_gradients(dev, mode, agg, terms):
             continue
         assert rc == 0
         o_out16, o_msum, o_rs = torch.ops.siirl_hip.policy_loss_fwd(old, lp, adv, mask, isw, e, r, *args)
-        assert torch.equal(out16, o_out16) and torch.equal(msum, o_msum)
+        # few segments take one launch, with a kept gradient always several: the sums are in double, in another order
+        assert ((out16 - o_out16).abs() <= 1.2e-7 * o_out16.abs()).all() and torch.equal(msum, o_msum), (B, L)
         up = torch.tensor([1.7], device=dev)
         want, want_e = torch.ops.siirl_hip.policy_loss_bwd(up, old, lp, adv, mask, isw, e, r, *args, o_out16, o_msum, o_rs)
         got, got_e = torch.full_like(lp, float("nan")), torch.full_like(lp, float("nan"))
