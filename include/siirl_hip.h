@@ -597,7 +597,7 @@ size_t siirl_gae_workspace_bytes(int64_t B, int64_t L);
  *   float32 operation order and `returns` equals the reference's (only the sign of a zero may differ);
  *   SIIRL_GAE_CHUNKED shortens the dependent chain 16-fold for long rows (same arithmetic inside a chunk; the state
  *   entering a chunk goes through the chunks' composed maps, which changes its rounding: results agree to float32
- *   accuracy).  It pays for few rows only: [64, 8192] 58 us against 93, [1024, 8192] 118 against 105.
+ *   accuracy).  It pays for few rows only: [64, 8192] 56 us against 66, [1024, 8192] 113 against 79.
  *   stats3 as for siirl_masked_whiten.
  * Replaces: compute_gae_advantage_return siirl/dag_worker/core_algos.py:229-276.
  */
