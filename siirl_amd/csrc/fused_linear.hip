@@ -136,7 +136,14 @@ __device__ __forceinline__ int col_of_lane(int wn, int j, int lane) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 // F16: the 16-bit operands are IEEE half instead of bf16 (the same data movement, the other MFMA)
-template <class Epi, int AL = A_ROWS, bool F16 = false>
+// A_ONCE: one token tile, so that W is read once, and W larger than the memory-side cache: its loads are non-temporal, or
+// what they bring in would push out what every workgroup reads, the B operand, and itself before anyone asks for it again.
+// Forward / recompute / d hidden (us): T=200, H=3584, V=152064 297 / 281 / 280 -> 256 / 278 / 292 (the ordinary loads find the
+// end of W that the product before left in the cache: alone they take 317), T=256, H=2048, V=151936 fp16 200 / 226 / 170 ->
+// 155 / 175 / 172, T=50, H=2048, V=100000 175 / 125 / 94 -> 114 / 123 / 112.  A smaller W stays in the cache from one product
+// to the next: T=64, H=2048, V=50257 79 / 45 / 47 -> 60 / 64 / 55.  With more token tiles W comes from the L2 to all but the
+// first of them: T=400 437 / 454 / 618 -> 479 / 514 / 702.
+template <class Epi, int AL = A_ROWS, bool F16 = false, bool A_ONCE = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_nt_kernel(GemmArgs g, Epi epi) {
   static_assert(!(F16 && Epi::kRowsPerLane), "the gradient GEMMs multiply bf16");
   extern __shared__ __align__(16) char smem[];
@@ -225,7 +232,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
 #pragma unroll
     for (int i = i0; i < i1; ++i) {
       const uint32_t dst = lds0 + stage * kStageBytes + (wu * kDmaPerWave + i) * 1024;
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(offA[i]), "s"(base) : "m0", "memory");
+      if constexpr (A_ONCE)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(dst), "v"(offA[i]), "s"(base) : "m0", "memory");
+      else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(offA[i]), "s"(base) : "m0", "memory");
     }
   };
   auto bload = [&](u32x4 (&b)[NJ][KS], int kt, int j) {
@@ -975,13 +985,20 @@ inline int fit_blk_m(int blk_m, int64_t tiles_m, int64_t tiles_n) {
 template <class Epi, int AL = A_ROWS, bool F16 = false>
 int launch_gemm(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_total, int M, int N, int K, const Epi& epi,
                 hipStream_t st, const char* what, int splits = 1, int blk_m = 8, const uint16_t* A_tail = nullptr) {
-  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<Epi, AL, F16>), kSmemBytes)) return rc;
   GemmArgs g{A, lda, Bp, kb_total, M, N, K, (M + BM - 1) / BM, (N + BN - 1) / BN, splits, blk_m, 0,
              A_tail, A_tail ? K / BK - 1 : K / BK};
   g.blk_m = fit_blk_m(blk_m, g.tiles_m, (int64_t)g.tiles_n * splits);
   if (AL == A_PACKED && lda * 32 < (int64_t)g.tiles_m * BM) return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: row pitch %lld is shorter than %d tiles", what, (long long)lda, g.tiles_m);
   const int64_t grid = raster_grid(g);
-  gemm_nt_kernel<Epi, AL, F16><<<dim3((unsigned)grid), dim3(kThreads), kSmemBytes, st>>>(g, epi);
+  auto launch = [&](auto once) -> int {
+    auto* kernel = &gemm_nt_kernel<Epi, AL, F16, decltype(once)::value>;
+    if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmemBytes)) return rc;
+    kernel<<<dim3((unsigned)grid), dim3(kThreads), kSmemBytes, st>>>(g, epi);
+    return SIIRL_OK;
+  };
+  constexpr bool kReadsW = AL != A_PACKED;  // (the packed A of d weight is small and read by every column tile)
+  const bool once = kReadsW && g.tiles_n == 1 && streams_past_cache(2.0 * (double)M * (double)K);
+  if (int rc = once ? launch(std::bool_constant<kReadsW>{}) : launch(std::false_type{})) return rc;
   SIIRL_LAUNCH_CHECK(what);
   return SIIRL_OK;
 }

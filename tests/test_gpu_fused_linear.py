@@ -196,6 +196,28 @@ def test_column_groups_and_k_runs(dev, T, H, V):
     _check_grad(wd.grad, dw64, "d_weight")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,V", [(1, 64, 2457700), (256, 1088, 144600), (129, 1088, 144601), (257, 1088, 144601)])
+def test_one_token_tile_of_a_weight_beyond_the_cache(dev, dtype, T, H, V):
+    """Weights just above 300 MiB, which one token tile (up to 256 tokens) reads once, with rows and K-steps left over.
+    Reference: float64 on the GPU; the bars are those of the other sizes."""
+    import siirl_amd.fused_linear as FL
+
+    g = torch.Generator(device=dev).manual_seed(T + H)
+    h = torch.randn(T, H, device=dev, generator=g).to(dtype)
+    w = torch.empty(V, H, device=dev, dtype=dtype).normal_(0.0, 2.0 / H ** 0.5, generator=g)
+    y = torch.randint(0, V, (T,), device=dev, generator=g)
+    g_lp, g_h = (torch.randn(T, device=dev, generator=g) * 1e-2 for _ in range(2))
+    assert w.numel() * 2 > 300 * 2 ** 20
+    hd, wd = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    lp, ent = FL.fused_linear_logprob_entropy(hd, wd, y)
+    torch.autograd.backward([lp, ent], [g_lp, g_h])
+    lp64, ent64, dh64, dw64 = _float64_reference(h, w, y, g_lp, g_h)
+    assert (lp.double() - lp64).abs().max() < 1e-4 and (ent.double() - ent64).abs().max() < 1e-4
+    _check_grad(hd.grad, dh64, "d_hidden")
+    _check_grad(wd.grad, dw64, "d_weight")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("T", [1, 64, 65, 129, 192, 193, 256, 257])
 @pytest.mark.parametrize("H,V", [(64, 129), (320, 1000), (576, 70000)])
