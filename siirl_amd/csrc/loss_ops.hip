@@ -50,9 +50,11 @@ enum O { O_LOSS = 0, O_PG, O_CLIPFRAC, O_PPOKL, O_CLIPLOWER, O_ENTLOSS, O_KLLOSS
 
 using namespace tok;
 
-// Reductions over a whole wave by DPP (pairs, quads, halves and rows of 16 lanes) and the four rows by lane reads: no LDS
-// traffic, where a __shfl_xor is an LDS instruction per 32 bits and step -- 108 of them for the totals of the finish, which
-// 16 waves of one workgroup queue for.  Every lane gets the result; all 64 lanes must be active.
+// Reductions over a whole wave, the tree of wave_sum (lanes 32 apart, 16, 8, 4, 2, 1) with its last four steps by DPP:
+// a __shfl_xor is an LDS instruction per 32 bits and step -- 108 of them for the totals of the finish, which 16 waves of one
+// workgroup queue for.  (A rotation of a row of 16 lanes by 8, then by 4, is the exchange it stands for once the row repeats
+// itself after 16, then 8 lanes.)  The order is part of the results: a mean that cancels shows in it.  Every lane gets the
+// result; all 64 lanes must be active.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x) {
   return u2f((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f2u(x), CTRL, 0xf, 0xf, true));
@@ -64,20 +66,14 @@ __device__ __forceinline__ double dpp(double x) {
   const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
-__device__ __forceinline__ float lane_value(float x, int lane) { return u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(x), lane)); }
-__device__ __forceinline__ double lane_value(double x, int lane) {
-  const uint64_t u = __builtin_bit_cast(uint64_t, x);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 template <typename T, typename Op>
 __device__ __forceinline__ T wave_fold(T v, Op op) {
-  v = op(v, dpp<0xb1>(v));   // quad_perm: lane ^ 1
+  v = op(v, __shfl_xor(v, 32, kWave));
+  v = op(v, __shfl_xor(v, 16, kWave));
+  v = op(v, dpp<0x128>(v));  // row_ror:8
+  v = op(v, dpp<0x124>(v));  // row_ror:4
   v = op(v, dpp<0x4e>(v));   // quad_perm: lane ^ 2
-  v = op(v, dpp<0x141>(v));  // row_half_mirror
-  v = op(v, dpp<0x140>(v));  // row_mirror
-  return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48)));
+  return op(v, dpp<0xb1>(v));  // quad_perm: lane ^ 1
 }
 struct Add {
   template <typename T>
@@ -461,7 +457,7 @@ __device__ __forceinline__ void write_result(const LossArgs& a, const Totals& t,
 
 // small batches: one workgroup folds every row and writes the result block.  It is all latency, of a row's segment records
 // one after the other: up to 1024 threads, several a row where there are fewer rows, the records of four segments in
-// flight.  [1024, 8192] 10.7 us, with 256 threads of one row each and a reduction per total 12; [32, 32768] 6.3 and 9.5.
+// flight.  [1024, 8192] 10.5 us, with 256 threads of one row each and a reduction per total 12; [32, 32768] 6.8 and 9.5.
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void loss_finish_kernel(LossArgs a, const float* __restrict__ partials,
                                                               const float* __restrict__ row_s, int lanes,
@@ -486,7 +482,7 @@ int launch_loss_finish(const LossArgs& a, const float* partials, const float* ro
 
 // the whole forward of at most kSmallSegments segments in one workgroup, 128 threads a segment: the same sums in the same
 // order as the two to three launches it stands for.  A launch costs the host about 3 us, which is what a micro-batch waits
-// for: [8, 256] forward + backward 75.5 -> 71.7 us, the forward kernels 13.3 -> 7.6.
+// for: [8, 256] forward + backward 75.5 -> 71.7 us, the forward kernels 13.3 -> 7.5.
 constexpr int kSmallSegments = 8, kSmallThreads = kSmallSegments * kStream;
 template <int KIND>
 __global__ __launch_bounds__(kSmallThreads) void loss_small_kernel(LossArgs a, float* __restrict__ row_s,
