@@ -136,15 +136,15 @@ __device__ __forceinline__ int col_of_lane(int wn, int j, int lane) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 // F16: the 16-bit operands are IEEE half instead of bf16 (the same data movement, the other MFMA)
-// A_ONCE: one token tile, so that W is read once, and W larger than the memory-side cache: its loads are non-temporal, or
+// A_ONCE (gemm_once_kernel): one token tile, so that W is read once, and W larger than the memory-side cache: its loads are non-temporal, or
 // what they bring in would push out what every workgroup reads, the B operand, and itself before anyone asks for it again.
 // Forward / recompute / d hidden (us): T=200, H=3584, V=152064 297 / 281 / 280 -> 256 / 278 / 292 (the ordinary loads find the
 // end of W that the product before left in the cache: alone they take 317), T=256, H=2048, V=151936 fp16 200 / 226 / 170 ->
 // 155 / 175 / 172, T=50, H=2048, V=100000 175 / 125 / 94 -> 114 / 123 / 112.  A smaller W stays in the cache from one product
 // to the next: T=64, H=2048, V=50257 79 / 45 / 47 -> 60 / 64 / 55.  With more token tiles W comes from the L2 to all but the
 // first of them: T=400 437 / 454 / 618 -> 479 / 514 / 702.
-template <class Epi, int AL = A_ROWS, bool F16 = false, bool A_ONCE = false>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_nt_kernel(GemmArgs g, Epi epi) {
+template <class Epi, int AL, bool F16, bool A_ONCE>
+__device__ __forceinline__ void gemm_nt_tile(GemmArgs g, Epi epi) {
   static_assert(!(F16 && Epi::kRowsPerLane), "the gradient GEMMs multiply bf16");
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
@@ -397,6 +397,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWaves
   int em0 = m0, en0 = n0, el = lane;
   asm volatile("" : "+s"(em0), "+s"(en0), "+v"(el));  // (no address of the epilogue is computed before the main loop)
   epi(acc, em0, en0, tc.tm, split, wn, el, tid, smem);
+}
+
+template <class Epi, int AL = A_ROWS, bool F16 = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_nt_kernel(GemmArgs g, Epi epi) {
+  gemm_nt_tile<Epi, AL, F16, false>(g, epi);
+}
+
+template <class Epi, int AL = A_ROWS, bool F16 = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd, kWavesPerSimd))) void gemm_once_kernel(GemmArgs g, Epi epi) {
+  gemm_nt_tile<Epi, AL, F16, true>(g, epi);
 }
 #pragma clang diagnostic pop
 
@@ -990,15 +1000,19 @@ int launch_gemm(const uint16_t* A, int64_t lda, const u32x4* Bp, int64_t kb_tota
   g.blk_m = fit_blk_m(blk_m, g.tiles_m, (int64_t)g.tiles_n * splits);
   if (AL == A_PACKED && lda * 32 < (int64_t)g.tiles_m * BM) return fail(SIIRL_ERR_INVALID_ARGUMENT, "%s: row pitch %lld is shorter than %d tiles", what, (long long)lda, g.tiles_m);
   const int64_t grid = raster_grid(g);
-  auto launch = [&](auto once) -> int {
-    auto* kernel = &gemm_nt_kernel<Epi, AL, F16, decltype(once)::value>;
+  auto launch = [&](void (*kernel)(GemmArgs, Epi)) -> int {
     if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kSmemBytes)) return rc;
     kernel<<<dim3((unsigned)grid), dim3(kThreads), kSmemBytes, st>>>(g, epi);
     return SIIRL_OK;
   };
-  constexpr bool kReadsW = AL != A_PACKED;  // (the packed A of d weight is small and read by every column tile)
-  const bool once = kReadsW && g.tiles_n == 1 && streams_past_cache(2.0 * (double)M * (double)K);
-  if (int rc = once ? launch(std::bool_constant<kReadsW>{}) : launch(std::false_type{})) return rc;
+  if constexpr (AL != A_PACKED) {  // (the packed A of d weight is small and read by every column tile)
+    if (g.tiles_n == 1 && streams_past_cache(2.0 * (double)M * (double)K)) {
+      if (int rc = launch(&gemm_once_kernel<Epi, AL, F16>)) return rc;
+      SIIRL_LAUNCH_CHECK(what);
+      return SIIRL_OK;
+    }
+  }
+  if (int rc = launch(&gemm_nt_kernel<Epi, AL, F16>)) return rc;
   SIIRL_LAUNCH_CHECK(what);
   return SIIRL_OK;
 }
