@@ -39,9 +39,6 @@ SEED = 20250602
 # counter reads for a plain 2 GiB device copy (FETCH_SIZE reads half the bytes fetched: factor 2.0;
 # WRITE_SIZE factor 1.0).  Figures and commands: profiles/lpe_config2_hbm_traffic.md
 MEASURED_TRAFFIC_BYTES = int((4872246.35 * 2.0 + 9733599.87) * 1024)
-# The same for loss_partials_kernel + loss_bwd_kernel at config 3 with 5488 kept trajectories
-# (profiles/loss_path_config3_hbm_traffic.md)
-MEASURED_TRAFFIC_BYTES_CONFIG3 = int(((526927.5 + 527223.3) * 2.0 + 1372.0 + 176093.0) * 1024)
 
 
 def cpu_model() -> str:
@@ -170,7 +167,8 @@ def bench_config3(args, dev, quick=False):
     grp_ms = sum(e[0].elapsed_time(e[1]) for e in evs) / steps
     loss_ms = sum(e[1].elapsed_time(e[2]) for e in evs) / steps
     tokens = Bk * L
-    loss_bytes = tokens * (2 * (4 * 4 + 8) + 4)  # forward and backward each read 4 fp32 operands + int64 mask; d_lp written
+    # forward: 4 fp32 operands and the int64 mask read, the tokens' gradients written; backward: those read, d_lp written
+    loss_bytes = tokens * ((4 * 4 + 8) + 4 + 4 + 4)
 
     # the path's smaller building blocks on the same [kept, L] tensors, each timed alone (not part of the step)
     import siirl_amd.torch_functional as SF
@@ -211,7 +209,7 @@ def bench_config3(args, dev, quick=False):
         cov_scores, cov_stats = torch.ops.siirl_hip.cov_scores(None, lpd, adv_b, mk, CA.LOSS_KL_COV, 0.0, 0.0)
         k_cov = max(1, int(int(float(cov_stats[0]) + float(cov_stats[4])) * 0.0002))
         blocks = {
-            "kl_cov policy loss forward + backward: scores, top-k pick, loss, gradient (108 B/token)": (kl_cov_fb, 108),
+            "kl_cov policy loss forward + backward: scores, top-k pick, loss, gradient (92 B/token)": (kl_cov_fb, 92),
             f"siirl_topk_mark: the {k_cov} largest of the covariance scores marked (20 B/token: four reads, one write)":
                 (lambda: torch.ops.siirl_hip.topk_mark(cov_scores, k_cov, 1.0), 20),
             "masked_mean(values, mask) -> scalar (12 B/token)": (lambda: SF.masked_mean(lpd, mk), 12),
@@ -236,11 +234,10 @@ def bench_config3(args, dev, quick=False):
         "config": {"workload": f"config3: {P} prompts x {n} responses, L = {L}; {Bk} trajectories kept by the filter",
                    "trajectories": B, "kept": Bk, "response_length": L, "seed": SEED},
         "kernels": {"keep mask + GRPO advantage": {"ms": grp_ms},
-                    "actor loss forward + backward (loss_partials/finish/bwd kernels)": {"ms": loss_ms, "GB/s": gbs}},
+                    "actor loss forward + backward (loss_partials/finish/token_grad_bwd kernels)": {"ms": loss_ms, "GB/s": gbs}},
         "building_blocks": block_ms,
-        "roofline": {"bound": "hbm", "kernel": "loss_partials_kernel + loss_bwd_kernel", "achieved": gbs, "peak": 8000.0,
-                     "unit": "GB/s", "frac": gbs / 8000.0,
-                     "traffic": MEASURED_TRAFFIC_BYTES_CONFIG3 if Bk == 5488 else None},
+        "roofline": {"bound": "hbm", "kernel": "loss_partials_kernel + token_grad_bwd_kernel", "achieved": gbs, "peak": 8000.0,
+                     "unit": "GB/s", "frac": gbs / 8000.0, "traffic": None},
         "cpu_baseline": None,
     }
     if not args.no_cpu_baseline:  # the oracle's eager ops on the host cores, a 512-trajectory sample of the same step

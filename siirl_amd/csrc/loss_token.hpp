@@ -16,7 +16,8 @@
 // per launch): what the forward has read is then still cached when the backward reads it again -- forward + backward
 // at [1024, 8192] (192 MiB per pass) 99.8 -> 94 us, at [512, 8192] 55.3 -> 51 us; at [2048, 8192] (384 MiB) the
 // non-temporal loads are the faster ones again (166 against 183 us).  Stores are non-temporal at every size: ordinary
-// ones gain nothing there (51.8 against 51.1 us, 94.9 against 94.4 us) and their write-back delays the next kernel.
+// ones gain nothing there (51.8 against 51.1 us, 94.9 against 94.4 us) and their write-back delays the next kernel.  (The
+// token gradients that a forward keeps are stored as the pass reads: the backward wants them back.)
 #ifndef SIIRL_LOSS_NT_STORE
 #define SIIRL_LOSS_NT_STORE 1
 #endif
