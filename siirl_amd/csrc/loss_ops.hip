@@ -91,14 +91,15 @@ struct Max {
 // per segment: GSPO { sum_t (lp - old) * m, sum_t m };  GEO { sum_t x * m, sum_t m, sum_t A * m,
 // sum_t log(isw + 1e-10) * m }, x the token's clipped log-ratio
 // Four tokens an access, as in the other passes: [512, 32768] int64 mask, gspo, 59.5 -> 41.5 us (6.5 TB/s).
-constexpr int kNPre = 4;
-__device__ __forceinline__ void prepass_segment(const LossArgs& a, int64_t b, int seg, int tid, int nthreads,
-                                                float (&sum)[kNPre]) {
+// A segment is summed by kThreads threads wherever it is summed: a row's sums, and with them its ratio, its loss and its
+// gradient, do not depend on how many rows the call has.
+constexpr int kNPre = 4, kPreWaves = kThreads / kWave;
+__device__ __forceinline__ void prepass_segment(const LossArgs& a, int64_t b, int seg, int tid, float (&sum)[kNPre]) {
   const int64_t t0 = (int64_t)seg * kSeg;
   const bool vec = a.vec != 0, nt = a.nt != 0, geo = a.kind != KIND_GSPO;
 #pragma unroll
   for (int k = 0; k < kNPre; ++k) sum[k] = 0.f;
-  for (int gq = tid; gq < kSeg / 4; gq += nthreads) {
+  for (int gq = tid; gq < kSeg / 4; gq += kThreads) {
     const int64_t t = t0 + 4 * gq;
     if (t >= a.L) break;
     const int nv = (int)((a.L - t) < 4 ? (a.L - t) : 4);
@@ -122,24 +123,26 @@ __device__ __forceinline__ void prepass_segment(const LossArgs& a, int64_t b, in
       }
     }
   }
-#pragma unroll
-  for (int k = 0; k < kNPre; ++k) sum[k] = wave_fold(sum[k], Add{});
+}
+// sum k of a segment from its waves' sums
+__device__ __forceinline__ float join_prepass(const float (*waves)[kNPre], int k) {
+  float v = 0.f;
+  for (int w = 0; w < kPreWaves; ++w) v += waves[w][k];
+  return v;
 }
 __global__ __launch_bounds__(kThreads) void row_prepass_kernel(LossArgs a, float* __restrict__ pre) {
   const int64_t b = blockIdx.x / a.nseg;
   const int seg = blockIdx.x % a.nseg;
   float sum[kNPre];
-  prepass_segment(a, b, seg, threadIdx.x, kThreads, sum);
-  __shared__ float sh[kThreads / kWave][kNPre];
-  if ((threadIdx.x & (kWave - 1)) == 0)
+  prepass_segment(a, b, seg, threadIdx.x, sum);
+  __shared__ float sh[kPreWaves][kNPre];
 #pragma unroll
-    for (int k = 0; k < kNPre; ++k) sh[threadIdx.x / kWave][k] = sum[k];
-  __syncthreads();
-  if (threadIdx.x < kNPre) {
-    float v = 0.f;
-    for (int w = 0; w < kThreads / kWave; ++w) v += sh[w][threadIdx.x];
-    pre[(b * a.nseg + seg) * kNPre + threadIdx.x] = v;
+  for (int k = 0; k < kNPre; ++k) {
+    const float v = wave_fold(sum[k], Add{});
+    if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave][k] = v;
   }
+  __syncthreads();
+  if (threadIdx.x < kNPre) pre[(b * a.nseg + seg) * kNPre + threadIdx.x] = join_prepass(sh, threadIdx.x);
 }
 
 // GSPO: the sequence's mean log-ratio, sum d*m / max(sum m, 1), from the pre-pass sums of its segments; every wave that
@@ -480,32 +483,36 @@ int launch_loss_finish(const LossArgs& a, const float* partials, const float* ro
   return SIIRL_OK;
 }
 
-// the whole forward of at most kSmallSegments segments in one workgroup, 128 threads a segment: the same sums in the same
-// order as the two to three launches it stands for.  A launch costs the host about 3 us, which is what a micro-batch waits
+// the whole forward of at most kSmallSegments segments in one workgroup, 128 threads a segment.  A segment's sums and a
+// row's ratio are those of the two to three launches it stands for, bit for bit; segments and rows are added in double, in
+// an order of its own.  A launch costs the host about 3 us, which is what a micro-batch waits
 // for: [8, 256] forward + backward 75.5 -> 71.7 us, the forward kernels 13.3 -> 7.5.
 constexpr int kSmallSegments = 8, kSmallThreads = kSmallSegments * kStream;
 template <int KIND>
 __global__ __launch_bounds__(kSmallThreads) void loss_small_kernel(LossArgs a, float* __restrict__ row_s,
                                                                    float* __restrict__ out, float* __restrict__ row_msum) {
   __shared__ float sh[kSmallThreads / kWave][kNP], part[kSmallSegments * kNP], pre[kSmallSegments * kNPre];
-  constexpr int kWaves = kStream / kWave;  // per segment
+  __shared__ float shp[kSmallSegments][kPreWaves][kNPre];
+  constexpr int kWaves = kStream / kWave, kPreShare = kThreads / kStream;  // per segment
+  static_assert(kThreads % kStream == 0, "a thread takes whole shares of the pre-pass");
   const int g = threadIdx.x / kStream, tid = threadIdx.x % kStream, lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
   const bool active = g < (int)a.B * a.nseg;
   const int64_t b = g / a.nseg;
   const int seg = g % a.nseg;
   float seq_s = 0.f;
   if (KIND == KIND_GSPO) {
-    float sum[kNPre] = {0.f, 0.f, 0.f, 0.f};
-    if (active) prepass_segment(a, b, seg, tid, kStream, sum);
-    if (lane == 0)
+    float sum[kPreShare][kNPre];  // each thread does the work of kPreShare of row_prepass_kernel's
 #pragma unroll
-      for (int k = 0; k < kNPre; ++k) sh[wid][k] = sum[k];
+    for (int h = 0; h < kPreShare; ++h) prepass_segment(a, b, seg, tid + h * kStream, sum[h]);
+#pragma unroll
+    for (int h = 0; h < kPreShare; ++h)
+#pragma unroll
+      for (int k = 0; k < kNPre; ++k) {
+        const float v = wave_fold(sum[h][k], Add{});
+        if (lane == 0) shp[g][h * kWaves + wid % kWaves][k] = v;
+      }
     __syncthreads();
-    if (tid < kNPre) {
-      float v = 0.f;
-      for (int w = 0; w < kWaves; ++w) v += sh[g * kWaves + w][tid];
-      pre[g * kNPre + tid] = v;
-    }
+    if (tid < kNPre) pre[g * kNPre + tid] = join_prepass(shp[g], tid);
     __syncthreads();
     if (active) {
       seq_s = gspo_row(pre, b, a.nseg);

@@ -503,3 +503,29 @@ def test_very_long_rows(dev, B, L):
     torch.cuda.synchronize()
     per_call = (time.perf_counter() - t0) / 3
     assert per_call < 1.5e-3, per_call  # 0.2 GB of operands at most: well under a millisecond of streaming
+
+
+@pytest.mark.parametrize("B,L", [(1, 1), (8, 5), (8, 255), (8, 256), (8, 700), (8, 1024), (8, 1025), (8, 2044), (8, 2048), (2, 2049),
+                                 (2, 8192), (1, 16384), (1, 16381)])
+@pytest.mark.parametrize("mdt", [torch.int64, torch.float32])
+def test_gspo_rows_do_not_depend_on_the_batch(dev, B, L, mdt):
+    """A row's ratio, mask sum and gradient are the same bits in a call of a few segments (one launch) and among more rows.
+    The gradient's factor 1 / rows differs by a power of two, which is exact."""
+    import siirl_amd.core_algos as CA
+
+    n = 16 * B
+    lp, old, _, adv, mask, _ = (t.to(dev) for t in _batch(n, L, seed=B + L, dtype_mask=mdt))
+    if mdt == torch.float32:  # any weights, in one row the smallest ones
+        mask = mask * torch.rand(n, L, generator=torch.Generator().manual_seed(L)).to(dev) + 0.125
+        mask[0] *= 2.0 ** -20
+    args = (CA.LOSS_GSPO, 3e-4, 4e-4, 3.0, 20.0, 2, 0.0, 0, False, 0.0, 0.0, 1.0)
+    up = torch.ones(1, device=dev)
+
+    def rows(k):
+        ops = [t[:k].contiguous() for t in (old, lp, adv, mask)]
+        out16, msum, row_s = torch.ops.siirl_hip.policy_loss_fwd(*ops, None, None, None, *args)
+        d, _ = torch.ops.siirl_hip.policy_loss_bwd(up, *ops, None, None, None, *args, out16, msum, row_s)
+        return msum[:B], row_s[:B], d[:B] * (k // B)
+
+    for few, many in zip(rows(B), rows(n)):
+        assert torch.equal(few, many), (few.double() - many.double()).abs().max()
