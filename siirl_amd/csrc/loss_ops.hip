@@ -145,8 +145,12 @@ __global__ __launch_bounds__(kThreads) void row_prepass_kernel(LossArgs a, float
   if (threadIdx.x < kNPre) pre[(b * a.nseg + seg) * kNPre + threadIdx.x] = join_prepass(sh, threadIdx.x);
 }
 
-// GSPO: the sequence's mean log-ratio, sum d*m / max(sum m, 1), from the pre-pass sums of its segments; every wave that
-// needs it folds them for itself (a launch less than a kernel that does it for all rows)
+// GSPO: the sequence's mean log-ratio, sum d*m / max(sum m, 1), from the pre-pass sums of its segments, by a whole wave.
+// Every wave that needs it folds them for itself (a launch less than a kernel that does it for all rows) up to kFoldOwn
+// segments a row; beyond, where that reads nseg records nseg times, gspo_rows_kernel does it once per row.  Forward, own /
+// once (us), bool mask: [4, 524288] 21.3 / 23.3, [1, 2097152] 27.9 / 29.4, [32, 1048576] 148 / 141, [16, 4194304] 342 / 260,
+// [2, 16777216] 286 / 172; one thread per row for all of them took 106, 137, 247, 606 and 1023.
+constexpr int kFoldOwn = 256;
 __device__ __forceinline__ float gspo_row(const float* pre, int64_t b, int nseg) {
   double sd = 0.0, sm = 0.0;
   for (int s = threadIdx.x & (kWave - 1); s < nseg; s += kWave) {
@@ -156,6 +160,10 @@ __device__ __forceinline__ float gspo_row(const float* pre, int64_t b, int nseg)
   sd = wave_fold(sd, Add{});
   sm = wave_fold(sm, Add{});
   return (float)sd / fmaxf((float)sm, 1.f);  // .clamp(min=1)
+}
+__global__ __launch_bounds__(kWave) void gspo_rows_kernel(const float* __restrict__ pre, int nseg, float* __restrict__ row_s) {
+  const float s = gspo_row(pre, blockIdx.x, nseg);
+  if (threadIdx.x == 0) row_s[blockIdx.x] = s;
 }
 
 // GEO: folds the pre-pass segments of each row into the sequence's loss -adv_b * exp(sum x*m / (n + 1e-8))
@@ -258,8 +266,12 @@ __global__ __launch_bounds__(kStream) void loss_partials_kernel(LossArgs a, cons
   const int seg = blockIdx.x % a.nseg;
   float seq_s = 0.f;
   if (kind == KIND_GSPO) {
-    seq_s = gspo_row(pre, b, a.nseg);
-    if (seg == 0 && threadIdx.x == 0) row_s[b] = seq_s;  // for the backward
+    if (a.nseg > kFoldOwn) {
+      seq_s = row_s[b];
+    } else {
+      seq_s = gspo_row(pre, b, a.nseg);
+      if (seg == 0 && threadIdx.x == 0) row_s[b] = seq_s;  // for the backward
+    }
   }
   float acc[kNP];
   segment_sums<KIND, KEEP>(a, b, seg, threadIdx.x, seq_s, tg, acc);
@@ -1125,6 +1137,9 @@ int run_forward(LossArgs& a, float* out16, float* row_msum, float* row_s, void* 
       geo_rows_kernel<<<dim3((unsigned)((a.B + kThreads - 1) / kThreads)), block, 0, st>>>(pre, a.nseg, a.B,
                                                                                          a.isw != nullptr, row_s);
       SIIRL_LAUNCH_CHECK("geo_rows_kernel");
+    } else if (a.nseg > kFoldOwn) {
+      gspo_rows_kernel<<<dim3((unsigned)a.B), dim3(kWave), 0, st>>>(pre, a.nseg, row_s);
+      SIIRL_LAUNCH_CHECK("gspo_rows_kernel");
     }
   }
   if (int rc = tg ? launch_loss_partials<true>(a, pre, row_s, partials, tg, st)

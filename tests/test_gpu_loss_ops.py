@@ -529,3 +529,44 @@ def test_gspo_rows_do_not_depend_on_the_batch(dev, B, L, mdt):
 
     for few, many in zip(rows(B), rows(n)):
         assert torch.equal(few, many), (few.double() - many.double()).abs().max()
+
+
+@pytest.mark.parametrize("B,L", [(3, 2048 * 256), (3, 2048 * 256 + 1), (2, 2048 * 300 + 5), (1, 2048 * 5000)])
+def test_gspo_long_rows(dev, B, L):
+    """Around and above the number of segments from which a row's pre-pass sums are folded by a launch of their own.  The
+    ratio is a mean of float32 sums of at most 2048 products each (8 by 8 in a thread, then a tree): 32 * 2^-24 of the mean
+    magnitude bounds it."""
+    import siirl_amd.core_algos as CA
+
+    g = torch.Generator(device=dev).manual_seed(L)
+    lp, adv = (torch.randn(B, L, device=dev, generator=g) for _ in range(2))
+    old = lp + 0.02 * torch.randn(B, L, device=dev, generator=g)
+    mask = torch.rand(B, L, device=dev, generator=g) < 0.7
+    args = (CA.LOSS_GSPO, 3e-4, 4e-4, 3.0, 20.0, 2, 0.0, 0, False, 0.0, 0.0, 1.0)
+    _, msum, row_s = torch.ops.siirl_hip.policy_loss_fwd(old, lp, adv, mask, None, None, None, *args)
+    d = (lp - old).double() * mask
+    assert torch.equal(msum, mask.sum(1).float())
+    assert ((row_s - d.sum(1) / mask.sum(1)).abs() <= 32 * 2.0 ** -24 * d.abs().sum(1) / mask.sum(1)).all()
+
+
+def test_gspo_time_is_linear_in_the_row(dev):
+    """One row of 2^26 tokens and 1024 rows of 65536: the same bytes.  (Its 32768 segments fold their row's sums once; when
+    every workgroup folded them again the row took 4.2 times as long as the rows, with one fold 1.25 times.)"""
+    import siirl_amd.core_algos as CA
+
+    args = (CA.LOSS_GSPO, 3e-4, 4e-4, 3.0, 20.0, 2, 0.0, 0, False, 0.0, 0.0, 1.0)
+    lp, old, adv = (torch.full((2 ** 26,), 0.1 * k, device=dev) for k in range(3))
+    mask = torch.ones(2 ** 26, dtype=torch.bool, device=dev)
+    best = []
+    for B in (1024, 1):
+        ops = [t.view(B, -1) for t in (old, lp, adv, mask)]
+        ms = []
+        for _ in range(8):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            torch.ops.siirl_hip.policy_loss_fwd(*ops, None, None, None, *args)
+            end.record()
+            end.synchronize()
+            ms.append(start.elapsed_time(end))
+        best.append(min(ms))
+    assert best[1] < 2.5 * best[0], best
