@@ -497,8 +497,11 @@ int launch_loss_finish(const LossArgs& a, const float* partials, const float* ro
 
 // the whole forward of at most kSmallSegments segments in one workgroup, 128 threads a segment.  A segment's sums and a
 // row's ratio are those of the two to three launches it stands for, bit for bit; segments and rows are added in double, in
-// an order of its own.  A launch costs the host about 3 us, which is what a micro-batch waits
-// for: [8, 256] forward + backward 75.5 -> 71.7 us, the forward kernels 13.3 -> 7.5.
+// an order of its own.  A launch costs the host about 3 us, which is what a micro-batch waits for.  Up to 8 segments because
+// 1024 threads are a workgroup's most.  Forward + backward pass / forward kernels alone, several launches -> one (us):
+// vanilla [8, 256] 76.7 -> 71.6 / 7.7 -> 7.4, [8, 1024] 75.7 -> 71.9 / 9.9 -> 10.6, [4, 2048] 75.7 -> 72.1 / 13.8 -> 12.6, [8, 2048]
+// 75.9 -> 72.2 / 14.1 -> 16.8; gspo [8, 256] 76.2 -> 73.7 / 10.0 -> 7.9, [8, 2048] 79.6 -> 73.5 / 14.4 -> 14.7.  (One CU moves what
+// eight did, so from 8192 tokens on a caller whose GPU is never idle, a captured graph say, would rather have the launches.)
 constexpr int kSmallSegments = 8, kSmallThreads = kSmallSegments * kStream;
 template <int KIND>
 __global__ __launch_bounds__(kSmallThreads) void loss_small_kernel(LossArgs a, float* __restrict__ row_s,
@@ -508,8 +511,7 @@ __global__ __launch_bounds__(kSmallThreads) void loss_small_kernel(LossArgs a, f
   constexpr int kWaves = kStream / kWave, kPreShare = kThreads / kStream;  // per segment
   static_assert(kThreads % kStream == 0, "a thread takes whole shares of the pre-pass");
   const int g = threadIdx.x / kStream, tid = threadIdx.x % kStream, lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-  const bool active = g < (int)a.B * a.nseg;
-  const int64_t b = g / a.nseg;
+  const int64_t b = g / a.nseg;  // (the block has exactly the threads of the call's segments)
   const int seg = g % a.nseg;
   float seq_s = 0.f;
   if (KIND == KIND_GSPO) {
@@ -526,20 +528,16 @@ __global__ __launch_bounds__(kSmallThreads) void loss_small_kernel(LossArgs a, f
     __syncthreads();
     if (tid < kNPre) pre[g * kNPre + tid] = join_prepass(shp[g], tid);
     __syncthreads();
-    if (active) {
-      seq_s = gspo_row(pre, b, a.nseg);
-      if (seg == 0 && tid == 0) row_s[b] = seq_s;
-    }
+    seq_s = gspo_row(pre, b, a.nseg);
+    if (seg == 0 && tid == 0) row_s[b] = seq_s;
   }
-  if (active) {
-    float acc[kNP];
-    segment_sums<KIND, false>(a, b, seg, tid, seq_s, nullptr, acc);
-    if (lane == 0)
+  float acc[kNP];
+  segment_sums<KIND, false>(a, b, seg, tid, seq_s, nullptr, acc);
+  if (lane == 0)
 #pragma unroll
-      for (int k = 0; k < kNP; ++k) sh[wid][k] = acc[k];
-  }
+    for (int k = 0; k < kNP; ++k) sh[wid][k] = acc[k];
   __syncthreads();
-  if (active && tid < kNP) {
+  if (tid < kNP) {
     float v = sh[g * kWaves][tid];
     for (int w = 1; w < kWaves; ++w) v = join_partials(tid, v, sh[g * kWaves + w][tid]);
     part[g * kNP + tid] = v;
