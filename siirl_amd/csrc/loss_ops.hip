@@ -124,7 +124,15 @@ __device__ __forceinline__ void prepass_segment(const LossArgs& a, int64_t b, in
     }
   }
 }
-// sum k of a segment from its waves' sums
+// the sums of a wave into its record
+__device__ __forceinline__ void store_prepass(float (&sum)[kNPre], float* wave) {
+#pragma unroll
+  for (int k = 0; k < kNPre; ++k) sum[k] = wave_fold(sum[k], Add{});
+  if ((threadIdx.x & (kWave - 1)) == 0)
+#pragma unroll
+    for (int k = 0; k < kNPre; ++k) wave[k] = sum[k];
+}
+// sum k of a segment from its waves' records
 __device__ __forceinline__ float join_prepass(const float (*waves)[kNPre], int k) {
   float v = 0.f;
   for (int w = 0; w < kPreWaves; ++w) v += waves[w][k];
@@ -136,11 +144,7 @@ __global__ __launch_bounds__(kThreads) void row_prepass_kernel(LossArgs a, float
   float sum[kNPre];
   prepass_segment(a, b, seg, threadIdx.x, sum);
   __shared__ float sh[kPreWaves][kNPre];
-#pragma unroll
-  for (int k = 0; k < kNPre; ++k) {
-    const float v = wave_fold(sum[k], Add{});
-    if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave][k] = v;
-  }
+  store_prepass(sum, sh[threadIdx.x / kWave]);
   __syncthreads();
   if (threadIdx.x < kNPre) pre[(b * a.nseg + seg) * kNPre + threadIdx.x] = join_prepass(sh, threadIdx.x);
 }
@@ -500,7 +504,7 @@ int launch_loss_finish(const LossArgs& a, const float* partials, const float* ro
 // an order of its own.  A launch costs the host about 3 us, which is what a micro-batch waits for.  Up to 8 segments because
 // 1024 threads are a workgroup's most.  Forward + backward pass / forward kernels alone, several launches -> one (us):
 // vanilla [8, 256] 76.7 -> 71.6 / 7.7 -> 7.4, [8, 1024] 75.7 -> 71.9 / 9.9 -> 10.6, [4, 2048] 75.7 -> 72.1 / 13.8 -> 12.6, [8, 2048]
-// 75.9 -> 72.2 / 14.1 -> 16.8; gspo [8, 256] 76.2 -> 73.7 / 10.0 -> 7.9, [8, 2048] 79.6 -> 73.5 / 14.4 -> 14.7.  (One CU moves what
+// 75.9 -> 72.2 / 14.1 -> 16.8; gspo [8, 256] 76.2 -> 73.7 / 10.2 -> 8.2, [8, 2048] 79.6 -> 73.5 / 14.5 -> 15.0.  (One CU moves what
 // eight did, so from 8192 tokens on a caller whose GPU is never idle, a captured graph say, would rather have the launches.)
 constexpr int kSmallSegments = 8, kSmallThreads = kSmallSegments * kStream;
 template <int KIND>
@@ -519,12 +523,7 @@ __global__ __launch_bounds__(kSmallThreads) void loss_small_kernel(LossArgs a, f
 #pragma unroll
     for (int h = 0; h < kPreShare; ++h) prepass_segment(a, b, seg, tid + h * kStream, sum[h]);
 #pragma unroll
-    for (int h = 0; h < kPreShare; ++h)
-#pragma unroll
-      for (int k = 0; k < kNPre; ++k) {
-        const float v = wave_fold(sum[h][k], Add{});
-        if (lane == 0) shp[g][h * kWaves + wid % kWaves][k] = v;
-      }
+    for (int h = 0; h < kPreShare; ++h) store_prepass(sum[h], shp[g][h * kWaves + wid % kWaves]);
     __syncthreads();
     if (tid < kNPre) pre[g * kNPre + tid] = join_prepass(shp[g], tid);
     __syncthreads();
