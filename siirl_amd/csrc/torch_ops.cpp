@@ -838,7 +838,11 @@ constexpr int kActorOuts = 13;  // SIIRL_OUT_LOSS .. SIIRL_OUT_DRIFT_LOSS
 
 // Above this many tokens a differentiated loss forward leaves the tokens' gradients for the backward to scale.  Below it the
 // host is what a pass waits for, and the buffer is one more allocation: forward + backward at [32, 32768], gspo, 82.8 us
-// without and 84.2 us with it (kernels 32 and 36 us); [5744, 8192], four operands and an int64 mask, 410 and 301 us.
+// without and 84.2 us with it (kernels 32 and 36 us).  Above it, kernels without / with (us), operands from memory: vanilla
+// with KL, int64 mask, 2 M tokens 39.7 / 32.5, 4 M 53.4 / 43.5, 8 M 96.4 / 73.7, 12 M 137 / 104, 46 M 412 / 313; gspo, int64,
+// 2 M 38.1 / 33.6, 12 M 138 / 118; vanilla, bool mask, rows of 1024, 2 M 25.9 / 23.8, 12 M 79.5 / 68.9.  A forward that no
+// backward follows pays for it (182 -> 232 us at 47 M tokens, 4 bytes a token until the node dies): such calls belong under
+// no_grad, where nothing is kept.
 constexpr int64_t kKeepGradTokens = 1 << 21;
 
 // Whether it can: every term of the loss that depends on log_prob is aggregated in one mode (gspo brings its own;
@@ -855,15 +859,15 @@ std::tuple<Tensor, Tensor> token_grad_bwd(const Tensor& g, const Tensor& token_g
   require_f32c(token_grad, "token_grad");  // what a saved-tensor hook hands back is checked like any operand
   TORCH_CHECK_VALUE(token_grad.dim() == 2, "token_grad must be [B, L]");
   const int64_t B = token_grad.size(0), L = token_grad.size(1);
-  require_mask(mask, token_grad);
+  if (want_ent) require_mask(mask, token_grad);  // (only the entropy's gradient reads it)
   require_f32_n(g, 1, token_grad, "g_loss");
   require_f32_n(out16, 16, token_grad, "out16");
   require_f32_n(row_msum, B, token_grad, "row_msum");
   Tensor d_lp = empty_f32({B, L}, token_grad), d_ent;
   if (want_ent) d_ent = empty_f32({B, L}, token_grad);
   DeviceGuard guard(token_grad.device());
-  check_rc(siirl_token_grad_bwd(ptr<float>(g), ptr<float>(token_grad), want_ent ? ptr(mask) : nullptr, mask_code(mask), B,
-                                L, (int)policy_agg, (int)agg, (float)entropy_coeff, (float)scale, ptr<float>(out16),
+  check_rc(siirl_token_grad_bwd(ptr<float>(g), ptr<float>(token_grad), want_ent ? ptr(mask) : nullptr,
+                                want_ent ? mask_code(mask) : 0, B, L, (int)policy_agg, (int)agg, (float)entropy_coeff, (float)scale, ptr<float>(out16),
                                 ptr<float>(row_msum), ptr<float>(d_lp), ptr<float>(d_ent), stream_of(token_grad)),
            "siirl_token_grad_bwd");
   return {d_lp, d_ent};
@@ -918,8 +922,15 @@ struct ActorLossFn : public torch::autograd::Function<ActorLossFn> {
     if (keep_grad && B * L > kKeepGradTokens && keeps_token_grad(c, has(ref))) token_grad = empty_f32({B, L}, lp);
     policy_loss_fwd_launch(old, lp, adv, m, isw, ent, ref, aux, c, ptr<float>(out16), ptr<float>(row_msum),
                            ptr<float>(row_s), ptr<float>(buf) + head, nws, ptr<float>(token_grad));
-    ctx->save_for_backward({lp, old, adv, m, out16, row_msum, row_s, isw ? *isw : Tensor(), ent ? *ent : Tensor(),
-                            ref ? *ref : Tensor(), aux ? *aux : Tensor(), token_grad});
+    // The backward of a kept gradient reads no operand but the mask of an entropy term.  The caller's own tensors are saved
+    // all the same, so that one that is changed in place before the backward is refused; copies made here are not.
+    auto kept = [&](const Tensor& t, const Tensor& given) {
+      return !token_grad.defined() || t.is_alias_of(given) ? t : Tensor();
+    };
+    auto kept_opt = [&](const optional<Tensor>& t, const optional<Tensor>& given) { return t ? kept(*t, *given) : Tensor(); };
+    ctx->save_for_backward({kept(lp, log_prob), kept(old, old_log_prob), kept(adv, advantages),
+                            ent ? m : kept(m, response_mask), out16, row_msum, row_s, kept_opt(isw, is_weights),
+                            kept_opt(ent, entropy), kept_opt(ref, ref_log_prob), kept_opt(aux, token_aux), token_grad});
     ctx->saved_data["i"] = std::vector<int64_t>{loss_mode, agg_mode, kl_mode, (int64_t)kl_st, (int64_t)policy_only,
                                                 (int64_t)log_prob.scalar_type(),
                                                 has(entropy) ? (int64_t)entropy->scalar_type() : -1};
@@ -954,15 +965,16 @@ struct ActorLossFn : public torch::autograd::Function<ActorLossFn> {
     if (s[9].defined()) ref = s[9];
     if (s[10].defined()) aux = s[10];
     const int64_t policy_agg = c.loss_mode == SIIRL_LOSS_GSPO ? SIIRL_AGG_SEQ_MEAN_TOKEN_MEAN : c.agg_mode;
+    const bool want_ent = iv[6] >= 0;
     auto [d_lp, d_ent] =
-        s[11].defined() ? token_grad_bwd(scalar_grad(g_in), s[11], s[3], has(ent), policy_agg, c.agg_mode,
+        s[11].defined() ? token_grad_bwd(scalar_grad(g_in), s[11], s[3], want_ent, policy_agg, c.agg_mode,
                                          c.entropy_coeff, c.scale, s[4], s[5])
                         : policy_loss_bwd_impl(scalar_grad(g_in), s[1], s[0], s[2], s[3], isw, ent, ref, aux, c, s[4],
                                                s[5], s[6]);
     d_lp = d_lp.reshape(ctx->saved_data["lp_shape"].toIntVector());
     if ((at::ScalarType)iv[5] != at::kFloat) d_lp = d_lp.to((at::ScalarType)iv[5]);
     none[0] = d_lp;
-    if (ent) {
+    if (want_ent) {
       d_ent = d_ent.reshape(ctx->saved_data["ent_shape"].toIntVector());
       if ((at::ScalarType)iv[6] != at::kFloat) d_ent = d_ent.to((at::ScalarType)iv[6]);
       none[1] = d_ent;

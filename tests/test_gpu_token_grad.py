@@ -106,3 +106,29 @@ def test_no_gradient_is_kept_for_nothing(dev):
     before = torch.cuda.memory_allocated()
     torch.ops.siirl_hip.actor_loss(lp, None, old, adv, mask, None, None, *args)
     assert torch.cuda.max_memory_allocated() - before < lp.numel()
+
+
+def test_a_kept_gradient_keeps_no_copy_of_an_operand(dev):
+    """Half-precision and strided operands are converted for the forward; with the tokens' gradients kept, the backward reads
+    none of them, and the node holds the gradient and the result block (under a quarter of it here) alone."""
+    B, L = 1025, 2052
+    torch.manual_seed(5)
+    lp, old, ref, ent = (torch.randn(B, L, device=dev, dtype=torch.bfloat16) for _ in range(4))
+    adv, mask = torch.randn(L, B, device=dev).t(), (torch.rand(L, B, device=dev) < 0.7).double().t()
+    args = (0, 0.2, 0.28, 3.0, 20.0, 0)
+    tail = (3, False, 0.1, 0.0, 0.7, False, None)
+    lp, ent = lp.requires_grad_(True), ent.requires_grad_(True)
+    for with_ent in (False, True):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        outs = torch.ops.siirl_hip.actor_loss(lp, ent if with_ent else None, old, adv, mask, None, ref, *args, 0.01, *tail)
+        held = torch.cuda.memory_allocated() - before
+        assert held < (2.25 if with_ent else 1.25) * 4 * B * L, held  # an entropy's gradient reads the (converted) mask
+        got = torch.autograd.grad(outs[0], [lp, ent] if with_ent else [lp])
+        leaf, eleaf = lp.detach().float().requires_grad_(True), ent.detach().float().requires_grad_(True)
+        outs = torch.ops.siirl_hip.actor_loss(leaf, eleaf if with_ent else None, old.float(), adv.contiguous(),
+                                              mask.float().contiguous(), None, ref.float(), *args, 0.01, *tail)
+        want = torch.autograd.grad(outs[0], [leaf, eleaf] if with_ent else [leaf])
+        for a, b in zip(got, want):
+            assert torch.equal(a, b.to(torch.bfloat16))
+        del outs, got, want
