@@ -152,11 +152,16 @@ def to_device(arr, dev):
     """A host array as a tensor on ``dev``, by way of pinned memory: the copy is queued like a kernel, where one from
     pageable memory waits until the stream has done all that was queued before it.  (The pinned block is torch's and is
     not used again before the copy has run.)  Under stream capture, which a pageable copy refuses, it stays refused: a
-    graph would read the block again at every replay."""
+    graph would read the block again at every replay.  The stream that is asked, and the device that the block is made
+    for, are those of ``dev``, whichever device is current."""
     import torch
 
+    dev = torch.device(dev)
+    if dev.type == "cuda" and dev.index not in (None, torch.cuda.current_device()):
+        with torch.cuda.device(dev):
+            return to_device(arr, dev)
     t = torch.from_numpy(arr)
-    if t.numel() == 0 or torch.device(dev).type != "cuda" or torch.cuda.is_current_stream_capturing():
+    if t.numel() == 0 or dev.type != "cuda" or torch.cuda.is_current_stream_capturing():
         return t.to(dev)
     return t.pin_memory().to(dev, non_blocking=True)
 

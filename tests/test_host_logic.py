@@ -217,3 +217,45 @@ def test_marft_requests_must_not_overlap():
         _check_marft_chains([(4, 4), (0, 6)], 10)
     with pytest.raises(IndexError):
         _check_marft_chains([(0, 4), (4, 7)], 10)
+
+
+def test_host_arrays_go_by_the_device_they_are_sent_to(monkeypatch):
+    """With another device current, the capture state that is asked for and the pinned block are the target's."""
+    from siirl_amd import _lib
+
+    current, seen = [0], []
+
+    class Device:
+        def __init__(self, dev):
+            self.index = dev.index
+
+        def __enter__(self):
+            self.before, current[0] = current[0], self.index
+
+        def __exit__(self, *exc):
+            current[0] = self.before
+
+    class Host:
+        def numel(self):
+            return 1
+
+        def pin_memory(self):
+            seen.append(("pinned", current[0]))
+            return self
+
+        def to(self, dev, non_blocking=False):
+            seen.append(("queued" if non_blocking else "waited for", current[0]))
+            return self
+
+    capturing = set()
+    monkeypatch.setattr(torch, "from_numpy", lambda arr: Host())
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[0] in capturing)
+    _lib.to_device(None, torch.device("cuda:1"))
+    _lib.to_device(None, "cuda")
+    assert seen == [("pinned", 1), ("queued", 1), ("pinned", 0), ("queued", 0)] and current == [0]
+    seen.clear()
+    capturing.add(1)
+    _lib.to_device(None, torch.device("cuda", 1))  # a pageable copy, which a capture refuses
+    assert seen == [("waited for", 1)]
