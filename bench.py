@@ -39,6 +39,9 @@ SEED = 20250602
 # counter reads for a plain 2 GiB device copy (FETCH_SIZE reads half the bytes fetched: factor 2.0;
 # WRITE_SIZE factor 1.0).  Figures and commands: profiles/lpe_config2_hbm_traffic.md
 MEASURED_TRAFFIC_BYTES = int((4872246.35 * 2.0 + 9733599.87) * 1024)
+# The same for loss_partials_kernel + token_grad_bwd_kernel at config 3 with 5488 kept trajectories
+# (profiles/loss_path_config3_hbm_traffic.md)
+MEASURED_TRAFFIC_BYTES_CONFIG3 = int(((527683.8 + 87838.8) * 2.0 + 176988.0 + 175689.7) * 1024)
 
 
 def cpu_model() -> str:
@@ -237,7 +240,8 @@ def bench_config3(args, dev, quick=False):
                     "actor loss forward + backward (loss_partials/finish/token_grad_bwd kernels)": {"ms": loss_ms, "GB/s": gbs}},
         "building_blocks": block_ms,
         "roofline": {"bound": "hbm", "kernel": "loss_partials_kernel + token_grad_bwd_kernel", "achieved": gbs, "peak": 8000.0,
-                     "unit": "GB/s", "frac": gbs / 8000.0, "traffic": None},
+                     "unit": "GB/s", "frac": gbs / 8000.0,
+                     "traffic": MEASURED_TRAFFIC_BYTES_CONFIG3 if Bk == 5488 else None},
         "cpu_baseline": None,
     }
     if not args.no_cpu_baseline:  # the oracle's eager ops on the host cores, a 512-trajectory sample of the same step
@@ -1044,6 +1048,31 @@ def bench_host(args, dev):
     per_call["actor_loss (fused)"]["fwd_bwd_us"] = round(fwd_bwd(
         lambda: CA.actor_loss(old, lp_leaf, adv, mask, cfg, ref_log_prob=ref).loss, lp_leaf), 1)
 
+    # the halves of a loss call with torch.autograd.grad, and what torch's engine takes for a graph without work of its own
+    def halves(n=300):
+        t = [0.0, 0.0]
+        for k in range(-30, n):
+            if k == 0:
+                torch.cuda.synchronize()
+                t = [0.0, 0.0]
+            t0 = time.perf_counter()
+            loss = CA.actor_loss(old, lp_leaf, adv, mask, cfg, ref_log_prob=ref).loss
+            t1 = time.perf_counter()
+            torch.autograd.grad(loss, lp_leaf)
+            t2 = time.perf_counter()
+            t[0] += t1 - t0
+            t[1] += t2 - t1
+        torch.cuda.synchronize()
+        return [round(x / n * 1e6, 1) for x in t]
+
+    one = torch.ones((), device=dev, requires_grad=True)
+    ones = torch.ones((), device=dev)
+    view = one.view_as(one)
+    fwd_us, grad_us = halves()
+    split = {"actor_loss forward_us": fwd_us, "autograd.grad of it_us": grad_us,
+             "autograd.grad through one view_us": round(host_us(lambda: torch.autograd.grad(view, one, retain_graph=True)), 1),
+             "the same, gradient given_us": round(host_us(lambda: torch.autograd.grad(view, one, ones, retain_graph=True)), 1)}
+
     def micro_batch():  # dp_actor.py:403-501 with the drop-in functions: the reference's own ten calls
         lp = SF.logprobs_from_logits(logits, labels, inplace_backward=False)
         ent = SF.entropy_from_logits(logits)
@@ -1067,7 +1096,7 @@ def bench_host(args, dev):
     out = {"metric": "host microseconds per call of the drop-in functions (GPU work negligible)", "unit": "us",
            "n_gpus": 1, "data": "synthetic", "config": {"workload": f"host: [B, L] = [{B}, {L}] fp32 operands, logits "
                                                                     f"[{B}, {L}, {V}] fp32, int64 mask"},
-           "per_call": per_call,
+           "per_call": per_call, "actor_loss_halves": split,
            "micro_batch_drop_in_us": round(host_us(micro_batch, 200), 1),
            "micro_batch_actor_loss_us": round(host_us(micro_batch_fused, 200), 1),
            "cpu": cpu_model()}
