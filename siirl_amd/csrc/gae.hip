@@ -649,7 +649,10 @@ extern "C" size_t siirl_gae_workspace_bytes(int64_t B, int64_t L) {
 // [6144, 256] 27.6 / 32.5, [6144, 8192] 306 / 594, [8192, 256] 34.4 / 33.5, [8192, 1024] 76 / 90, [8192, 8192] 398 / 621,
 // [12000, 256] 46.6 / 34.5, [12000, 1024] 107 / 98, [131072, 32] 299 / 74; in chunks of rows [1024, 8192] 142 / 113, [5488, 8192]
 // 692 / 488.  float32 mask: [3072, 128] 15.7 / 17.2, [4096, 128] 16.5 / 18.1, [4096, 64] 16.2 / 15.0, [8192, 256] 27.8 / 32.7,
-// [8192, 4096] 206 / 296, [12000, 256] 35.9 / 33.0.  (Masks of other values than 0 and 1 would rather have the second from 3000 rows on, [4096, 8192] 554 / 494.)
+// [8192, 4096] 206 / 296, [12000, 256] 35.9 / 33.0.  The lines were drawn when the first took 91 us at [1024, 8192], where it
+// takes 65 now, and have stayed: the second is still taken where the first would win, just above them for long rows (1.1 to
+// 1.6 times at 8192 rows of 1024 and more) and at [4096, 128] with a float32 mask.  (Masks of other values than 0 and 1 would
+// rather have the second from 3000 rows on, [4096, 8192] 554 / 494.)
 static bool few_rows(int64_t rows, int64_t len, bool mask64) {
   if (len <= kCols) return rows <= (mask64 ? 2048 : 3072);
   return rows <= (mask64 && len < 1024 ? 6144 : 8192);

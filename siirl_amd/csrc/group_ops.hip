@@ -26,8 +26,8 @@ namespace {
 constexpr int kThreads = 256;   // streaming kernels (row sums, broadcast)
 // Run-walking kernels.  They are all latency: of the ordering check, B loads per workgroup, so fewer and larger workgroups
 // (eight loads a thread, in flight at once, at B = 8192); of the ends of a run, which ballots find inside a wave; and of the
-// members, which are read from an LDS copy of the workgroup's entries.  B = 8192, n = 16: keep mask 6.6 us, advantages
-// 6.0 us; one-wave workgroups that walked global memory member by member took 17.6 and 12.
+// members, which are read from an LDS copy of the workgroup's entries.  B = 8192, n = 16: keep mask 5.5 to
+// 8.7 us, advantages 6.0 to 7.0 us, box to box; one-wave workgroups that walked global memory member by member took 17.6 and 12.
 constexpr int kGroupThreads = 1024;
 
 // ---------------------------------------------------------------------------- row sums

@@ -376,7 +376,8 @@ struct Totals {
 };
 
 // folds the segments of row b into the totals and writes the row's mask sum; `lanes` (a power of two) consecutive lanes
-// share a row, and the first of them keeps what does not add up lane by lane
+// share a row, and the first of them keeps what does not add up lane by lane.  (The mask sum, which the row's gradient is
+// scaled by, does not depend on `lanes`: float32 sums add up in double without a rounding unless they are 2^25 apart.)
 __device__ __forceinline__ void fold_row(const LossArgs& a, const float* __restrict__ partials,
                                          const float* __restrict__ row_s, float* __restrict__ row_msum, int64_t b,
                                          int lanes, Totals& t) {

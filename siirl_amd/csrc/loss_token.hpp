@@ -16,8 +16,11 @@
 // per launch): what the forward has read is then still cached when the backward reads it again -- forward + backward
 // at [1024, 8192] (192 MiB per pass) 99.8 -> 94 us, at [512, 8192] 55.3 -> 51 us; at [2048, 8192] (384 MiB) the
 // non-temporal loads are the faster ones again (166 against 183 us).  Stores are non-temporal at every size: ordinary
-// ones gain nothing there (51.8 against 51.1 us, 94.9 against 94.4 us) and their write-back delays the next kernel.  (The
-// token gradients that a forward keeps are stored as the pass reads: the backward wants them back.)
+// ones gain nothing there (51.8 against 51.1 us, 94.9 against 94.4 us) and their write-back delays the next kernel.
+// All of these figures are of a backward that reads the operands again.  Where the forward keeps the tokens' gradients
+// instead, its operands are read once and the gradients are what the backward wants back: they are stored with the hint
+// that the operands are read with, and the backward picks its own by their size.  Measured as a whole only, forward +
+// backward, four operands and an int64 mask: [1024, 8192] 96 -> 74 us, [2048, 8192] 166 -> 128, [5744, 8192] 410 -> 301.
 #ifndef SIIRL_LOSS_NT_STORE
 #define SIIRL_LOSS_NT_STORE 1
 #endif
